@@ -6,6 +6,7 @@
 #include "km_common.h"
 
 #include <map>
+#include <set>
 #include <tuple>
 
 // Coarse level of one p' system: B x B aggregates of the interior, i-major.
@@ -34,6 +35,8 @@ struct km_coarse {
     uint64_t used = 0;        // coarse_tick of the last solve that used this level
     // tile shape of the fused smoothing launches per (NX, NY, sizeof T)
     std::map<std::tuple<int, int, int>, int> tiles;
+    // systems whose tile km_twolevel_set_tile chose: they solve by launches
+    std::set<std::tuple<int, int, int>> pinned;
 };
 
 namespace kmcoarse {
@@ -108,6 +111,11 @@ template <typename T>
 int fused_inner(km_ctx* ctx, int NX, int NY, const T* coefT, const T* rhs, T* xd, T* ws, double eps, int max_iter,
                 bool use_graph, KState* out, const std::function<int()>* tail = nullptr, bool sym = false,
                 const double* coef64 = nullptr);
+
+// Whether fused_inner<T> solves level C's system in one launch
+// (km_persist.hip); the launch's tile shape in *shape.
+template <typename T>
+bool one_launch(km_ctx* ctx, const km_coarse* C, int* shape);
 
 // Group solves: up to kGroupSystems independent symmetric FP64 systems of
 // fused_inner (from x = 0), each on its own coarse level C[k] (set up by the

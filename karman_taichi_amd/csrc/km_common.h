@@ -123,6 +123,7 @@ struct GraphKey {
 struct km_net;   // learned preconditioner buffers (km_unet.hip)
 struct km_batch; // batched cases (km_batch.hip)
 struct km_coarse; // coarse level of the two-level preconditioner (km_coarse.hip)
+struct km_persist; // exchange buffers of the one-launch solves (km_persist.hip)
 struct km_mg;     // multigrid hierarchy of the V-cycle preconditioner (km_mg.hip)
 
 struct km_ctx {
@@ -156,6 +157,7 @@ struct km_ctx {
     uint64_t coarse_tick = 0;
     void* blas = nullptr;          // rocBLAS handle (the coarse levels' Newton-Schulz GEMM)
     void* scratch = nullptr;       // device address of this device's no-allocation scratch array
+    km_persist* persist = nullptr; // exchange buffers of the one-launch solves
     km_mg* mg = nullptr;           // V-cycle hierarchy (KM_FLAG_MG)
 };
 

@@ -3,6 +3,7 @@
 #include "km_unet.h"
 #include "km_coarse.h"
 #include "km_mg.h"
+#include "km_persist.h"
 
 #include <cstdlib>
 #include <cstring>
@@ -153,6 +154,7 @@ int km_destroy(km_ctx* ctx) {
     km_net_free(ctx);
     km_batch_free(ctx);
     km_coarse_free(ctx);
+    km_persist_free(ctx);
     km_mg_free(ctx);
     KmHostLock lk(km_host_mutex());
     if (ctx->ws) (void)hipFree(ctx->ws);

@@ -1059,10 +1059,14 @@ int fbicg_group(km_ctx* ctx, int n, const int* NX, const int* NY, const double* 
     char* V = static_cast<char*>(km_ws_vectors(ctx));
     // every level set up (in system order, as separate solves would) and its tile chosen
     std::vector<km_coarse*> C(n);
-    std::vector<int> tile(n);
+    std::vector<int> tile(n, 0);
+    std::vector<char> alone(n, 0);   // solved in one launch of its own, as its own solve would be
     for (int k = 0; k < n; ++k) {
         if (int rc = kmcoarse::setup(ctx, NX[k], NY[k], coef[k], ctx->stream, true)) return rc;
         C[k] = ctx->coarse;
+        int shape = 0;
+        alone[k] = kmcoarse::one_launch<double>(ctx, C[k], &shape);
+        if (alone[k]) continue;
         double* scratch = reinterpret_cast<double*>(V + up(cells[k]));
         if (int rc = kmcoarse::group_tile(ctx, C[k], coef[k], b[k], scratch, &tile[k])) return rc;
     }
@@ -1072,8 +1076,25 @@ int fbicg_group(km_ctx* ctx, int n, const int* NX, const int* NY, const double* 
         if (taken[a]) continue;
         int g[kmcoarse::kGroupSystems];
         int m = 0;
+        if (alone[a]) {
+            taken[a] = 1;
+            ctx->coarse = C[a];
+            double* r = reinterpret_cast<double*>(V);
+            double* w = reinterpret_cast<double*>(V + up(cells[a]));
+            const std::function<int()> tail = [&]() {
+                return km_residual_async(ctx, NX[a], NY[a], coef[a], b[a], x[a], r);
+            };
+            KState st;
+            if (int rc = kmcoarse::fused_inner<double>(ctx, NX[a], NY[a], coef[a], b[a], x[a], w, kInnerMargin * eps,
+                                                       mi[a], use_graph, &st, &tail, true, coef[a]))
+                return rc;
+            if (int rc = fbicg_solve<double>(ctx, NX[a], NY[a], coef[a], b[a], x[a], eps, mi[a], flags, nullptr,
+                                             info ? &info[a] : nullptr, &st, km_mapped_res(ctx, 0)))
+                return rc;
+            continue;
+        }
         for (int c = a; c < n && m < kmcoarse::kGroupSystems; ++c)
-            if (!taken[c] && tile[c] == tile[a]) {
+            if (!taken[c] && !alone[c] && tile[c] == tile[a]) {
                 taken[c] = 1;
                 g[m++] = c;
             }

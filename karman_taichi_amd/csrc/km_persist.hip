@@ -1,0 +1,1099 @@
+// A whole preconditioned flexible BiCGSTAB solve in one launch: the two-level
+// solve of a p' system and the smoothed solves of the momentum systems, for
+// systems of up to a few thousand cells per compute unit.
+//
+// What bounds it.  The launch-per-stage iteration of km_twolevel.hip costs the
+// latency of four launches (three for the momentum systems), 45-50 us per
+// iteration at 1282 x 258 cells, however few bytes it moves.  Here one
+// workgroup per tile stays on its compute unit for the whole solve: the five
+// coefficients, r, p and v of the tile and its halo and x, r~ of the tile live
+// in registers, z in LDS, and only what other workgroups need goes through
+// memory: the tile's edge cells of v and t, the restriction pieces of P^T v and
+// P^T t, the partial sums and, on the larger coarse levels, the coarse values.
+// What is left is the exchange: two rounds per iteration (four with shared
+// coarse values), each a store, a flag and a load through the memory side.
+//
+// The recurrences, the preconditioner and the stopping test are those of
+// km_twolevel.hip; every workgroup sums the same partial sums in the same order,
+// so all take the same decisions.  A workgroup holds r, p and v on its halo
+// too and advances them by the same expressions as their owner.
+//
+// Exchange.  Values other workgroups read are stored and loaded as relaxed
+// agent-scope atomics (they bypass the caches that are not coherent between
+// the eight dies).  A round: every wave waits until its stores are complete
+// (vmcnt 0), the workgroup meets, one thread stores the round's number into
+// the workgroup's flag, then every workgroup reads all flags until they have
+// it.  Round numbers only grow, over all launches of a context, so a flag is
+// never cleared.  A flag has a 64-byte line of its own: 1.65 us a round for 256
+// workgroups, against 4.5 us with the flags in neighbouring words and 3.9 us
+// for a central counter.  The few shared coarse values carry the round's number
+// in each 64-bit word instead (half a double beside a 32-bit tag): their
+// readers need no round, 1.5 us instead of 3.2.  The same for the partial sums
+// and the halo took longer (5-11 us a round: more words to ask for again and
+// again, and registers spilled).
+//
+// All workgroups must be resident at once: the host admits at most one per
+// compute unit and orders these launches of a process one after another
+// (Gate).  A wait is bounded in time; on the limit (another process holding
+// compute units, say) every workgroup leaves, and the host solves by launches.
+#include "km_persist.h"
+#include "km_coarse.h"
+
+#include <algorithm>
+#include <mutex>
+#include <type_traits>
+
+// Per-context exchange buffers (allocated at the first such solve).
+struct km_persist {
+    char* arena = nullptr;
+    unsigned* flags = nullptr;   // [2 systems][kMaxWg] lines of kFlagStride words
+    unsigned* abort = nullptr;   // set by a wait that ran into its limit
+    uint64_t* Y = nullptr;       // [2][kMaxM][2] shared coarse values Y(p), Y(s) with their round
+    double* part = nullptr;      // [2 systems][2 half-iterations][kMaxWg][4] partial sums
+    double* rc = nullptr;        // [2][kMaxSlots][kMaxM] restriction pieces of P^T v, P^T t
+    unsigned round = 0;          // the last round's number
+    bool clean = false;          // flags and Y hold numbers up to ``round`` only
+    int off = 0;                 // launches that ran into the limit: the path closes after two
+};
+
+namespace {
+
+constexpr int kMaxWg = 256;
+constexpr int kFlagStride = 16;
+constexpr int kMaxSlots = 16;
+constexpr int kMaxM = 2048;
+constexpr int kMaxF = 64;                // aggregates under one tile's z frame
+constexpr size_t kLdsBytes = 160 * 1024;
+constexpr int kEpt = 4;                  // restricted values per thread: m <= kEpt NT
+constexpr int kStallWindow = 300;        // as km_twolevel.hip
+constexpr long long kWaitTicks = 200000000LL;   // 2 s of the 100 MHz clock
+constexpr int kUnsupported = 100;        // status words of a launch that gave up
+constexpr int kAborted = 101;
+
+// Tile shapes (interior rows x columns of a workgroup) and threads, smallest
+// first: a solve takes the first shape whose tiles number at most one per
+// compute unit.  Threads: as many as the register frame (tile plus halo 4) has
+// pairs of cells, or half or a third of them.
+constexpr int kNumShapes = 6;
+constexpr int kTI[kNumShapes] = {16, 16, 32, 40, 48, 48};
+constexpr int kTJ[kNumShapes] = {16, 32, 32, 32, 32, 48};
+constexpr int kNT[kNumShapes] = {320, 512, 512, 512, 512, 512};
+
+template <typename T>
+struct PSys {
+    int NX, NY, tiles_j, G;
+    const void* c;        // five coefficient planes
+    const T* b;
+    T* x;
+    T* v;                 // edge cells of v and t for the neighbours
+    T* t;
+    unsigned* flags;
+    unsigned* abort;
+    unsigned round;       // the last round before this launch
+    double* pa;           // partial sums of the two half-iterations
+    double* pb;
+    double eps;
+    int max_iter;
+    T om;
+    int* hw;              // the host's words
+    // coarse level
+    int B, mJ, m, SJ;
+    int R;                // > 0: each workgroup computes R coarse values and shares them; 0: all it needs
+    int cached;           // rows of A_c^-1 kept in LDS
+    const uint8_t* mask;
+    const double* inv;
+    double* rcv;
+    double* rct;
+    uint64_t* Yp;         // shared coarse values (R > 0)
+    uint64_t* Ys;
+};
+
+__device__ __forceinline__ bool fin(double v) { return v == v && v - v == 0.0; }
+
+// 1 / d refined as in km_twolevel.hip
+__device__ __forceinline__ double recip(double d) {
+    double x = __builtin_amdgcn_rcp(d);
+    x = __builtin_fma(x, __builtin_fma(-d, x, 1.0), x);
+    x = __builtin_fma(x, __builtin_fma(-d, x, 1.0), x);
+    return x;
+}
+__device__ __forceinline__ float recip(float d) { return 1.0f / d; }
+
+template <typename V>
+__device__ __forceinline__ void put(V* p, V v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename V>
+__device__ __forceinline__ V get(const V* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// base[k], base the same in all lanes: a 32-bit offset per lane
+template <typename V>
+__device__ __forceinline__ V get_at(const V* base, int k) {
+    return get(reinterpret_cast<const V*>(reinterpret_cast<const char*>(base) + (uint32_t)k * (uint32_t)sizeof(V)));
+}
+
+// One round: false when the wait ran into its limit here or elsewhere.
+template <int NT>
+__device__ __forceinline__ bool meet(unsigned* flags, int L, int G, unsigned round, unsigned* abort, int* bad) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) put(flags + L * kFlagStride, round);
+    if ((int)threadIdx.x < G) {
+        const unsigned* f = flags + threadIdx.x * kFlagStride;
+        if (get(f) < round) {
+            const long long t0 = wall_clock64();
+            int spin = 0;
+            while (get(f) < round) {
+                if ((++spin & 63) == 0 && (wall_clock64() - t0 > kWaitTicks || get(abort)) && get(f) < round) {
+                    put(abort, 1u);
+                    *bad = 1;
+                    break;
+                }
+            }
+        }
+    }
+    __syncthreads();
+    return *bad == 0;
+}
+
+// Totals over the workgroups' partial sums P[G][4], in a fixed order: thread t
+// holds workgroup t's values.
+template <int NV, int NT>
+__device__ __forceinline__ void totals(const double (&mine)[NV], int G, double (&out)[NV], double* red) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int nw = (G + 63) >> 6;
+    if (w < nw) {
+#pragma unroll
+        for (int q = 0; q < NV; ++q) {
+            const double a = wave_sum(mine[q]);
+            if (lane == 0) red[w * NV + q] = a;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < NV; ++q) {
+        double a = red[q];
+        for (int k = 1; k < nw; ++k) a += red[k * NV + q];
+        out[q] = a;
+    }
+}
+
+// The workgroup's sums of NV values, published as its partial sums.
+template <int NV, int NT>
+__device__ __forceinline__ void publish(const double (&v)[NV], double* P, double* red) {
+    constexpr int NW = NT / 64;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+    for (int q = 0; q < NV; ++q) {
+        const double a = wave_sum(v[q]);
+        if (lane == 0) red[w * NV + q] = a;
+    }
+    __syncthreads();
+    if (threadIdx.x < NV) {
+        double a = red[threadIdx.x];
+        for (int k = 1; k < NW; ++k) a += red[k * NV + threadIdx.x];
+        put(P + threadIdx.x, a);
+    }
+}
+
+// Part of an aggregate in a tile: first cell in yb, width, cells, the steps of
+// 64 cells in rows and columns, 65536 / width rounded up, its slot's value.
+struct Piece {
+    int at, wdt, cnt, dr, dc, inv, dst;
+};
+
+// A row of the cached A_c^-1, by its offset in the dynamic LDS (a plain
+// pointer would turn its loads into flat ones).
+struct LdsRow {
+    int at;
+    __device__ __forceinline__ double operator[](int k) const {
+        extern __shared__ double dyn[];
+        return dyn[at + k];
+    }
+};
+
+// SW red-black sweeps (halo NS = 2 SW); COARSE: the two-level preconditioner.
+// CT: coefficient and arithmetic type (FP64 for the two-level solve of FP32
+// vectors, see k_tl_tile's C64).
+template <typename T, typename CT, int TI, int TJ, int NT, int SW, bool COARSE>
+__device__ __forceinline__ void solve_body(const PSys<T>& s, int L) {
+#pragma clang fp contract(fast)
+    constexpr int NS = 2 * SW;
+    constexpr int WZ = TJ + 2 * (NS + 1), HZ = TI + 2 * (NS + 1);
+    constexpr int WR = TJ + 2 * NS, HR = TI + 2 * NS;
+    constexpr int NPI = TI * TJ / 2, NP = HR * WR / 2;
+    constexpr int QI = (NPI + NT - 1) / NT, Q = (NP + NT - 1) / NT;
+    constexpr int BAND = NS * (WR / 2);
+    constexpr int QZ = (HZ * WZ + NT - 1) / NT;
+    constexpr int NW = NT / 64;
+    static_assert(TJ % 2 == 0 && TI >= NS && TJ >= NS && NT % 64 == 0 && NT >= kMaxWg, "tile");
+    extern __shared__ double dyn[];            // COARSE: m restricted values, then the cached rows of A_c^-1
+    __shared__ T za[HZ * WZ];
+    __shared__ double yb[COARSE ? TI * TJ : 1];
+    // Y(r), Y(p), Y(v), Y(s) of the coarse rows computed here; yl: shared
+    // values of the aggregates under the z frame
+    __shared__ double yr[COARSE ? kMaxF : 1], yp[COARSE ? kMaxF : 1], yv[COARSE ? kMaxF : 1], ysv[COARSE ? kMaxF : 1];
+    __shared__ double yl[COARSE ? kMaxF : 1];
+    __shared__ Piece piece[COARSE ? kMaxF : 1];
+    __shared__ double red[4 * (NW > 4 ? NW : 4)];
+    __shared__ double red2[4 * 4];
+    // x, r~ and p^ of the own cells: each thread reads back what it wrote
+    __shared__ T xs[2 * QI * NT], rts[2 * QI * NT], hps[2 * QI * NT];
+    __shared__ int bad;
+
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int NX = s.NX, NY = s.NY, nx = NX - 2, ny = NY - 2, G = s.G;
+    const int64_t n = (int64_t)NX * NY;
+    const CT* __restrict__ c = static_cast<const CT*>(s.c);
+    const CT om = (CT)s.om;
+    const int ta = L / s.tiles_j, tb = L - ta * s.tiles_j;
+    const int ti0 = 1 + ta * TI, tj0 = 1 + tb * TJ;
+    unsigned round = s.round;
+    if (t == 0) bad = 0;
+
+    // boundary cells of the system next to this tile: x = 0, and their rows
+    // must be empty (checked: otherwise the launch gives up)
+    double odd = 0.0;
+    {
+        const int j0 = tb == 0 ? 0 : tj0, j1 = tj0 + TJ > ny ? NY : tj0 + TJ;
+        const int i0 = ta == 0 ? 0 : ti0, i1 = ti0 + TI > nx ? NX : ti0 + TI;
+        auto check = [&](int i, int j) {
+            const int64_t k = (int64_t)i * NY + j;
+            bool any = s.b[k] != T(0);
+            for (int e = 0; e < 5; ++e) any = any || c[e * n + k] != CT(0);
+            if (any) odd += 1.0;
+            s.x[k] = T(0);
+        };
+        if (ta == 0)
+            for (int j = j0 + t; j < j1; j += NT) check(0, j);
+        if (ti0 + TI > nx)
+            for (int j = j0 + t; j < j1; j += NT) check(NX - 1, j);
+        if (tb == 0)
+            for (int i = i0 + t; i < i1; i += NT) check(i, 0);
+        if (tj0 + TJ > ny)
+            for (int i = i0 + t; i < i1; i += NT) check(i, NY - 1);
+    }
+
+    // the frame: pair slots as k_tl_tile's, the tile's own block first
+    CT cr[Q][2][5], wd[Q][2];
+    T r[Q][2], p[Q][2], v[Q][2];
+    int kq[Q][2];
+    short dq[Q][2], pz[Q][2];   // distance outside the tile (99: not in the system), z index
+    uint32_t own = 0, edge = 0, fm = 0;   // bit 2 q + c: own cell; read by a neighbour; free cell
+    const int par0 = (ti0 + tj0) & 1;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        const int P = t + q * NT;
+        int a, b0;
+        if (P < NPI) {
+            a = NS + P / (TJ / 2);
+            b0 = NS + 2 * (P - (P / (TJ / 2)) * (TJ / 2));
+        } else {
+            const int u0 = P - NPI;
+            if (u0 < BAND) {
+                a = u0 / (WR / 2);
+                b0 = 2 * (u0 - a * (WR / 2));
+            } else if (u0 < 2 * BAND) {
+                const int u = u0 - BAND;
+                a = NS + TI + u / (WR / 2);
+                b0 = 2 * (u - (u / (WR / 2)) * (WR / 2));
+            } else {
+                const int u = u0 - 2 * BAND, e = u - (u / NS) * NS;
+                a = NS + u / NS;
+                b0 = e < NS / 2 ? 2 * e : TJ + NS + 2 * (e - NS / 2);
+            }
+        }
+        const int par = (par0 + a) & 1;
+#pragma unroll
+        for (int cc = 0; cc < 2; ++cc) {
+            const int b = b0 + (par ^ cc);
+            const int i = ti0 - NS + a, j = tj0 - NS + b;
+            const bool in = P < NP && i >= 1 && i <= nx && j >= 1 && j <= ny;
+            const int k = in ? i * NY + j : 0;
+            kq[q][cc] = k;
+            pz[q][cc] = (short)(P < NP ? (a + 1) * WZ + b + 1 : 0);
+            const int di = NS - a > a - (TI + NS - 1) ? NS - a : a - (TI + NS - 1);
+            const int dj = NS - b > b - (TJ + NS - 1) ? NS - b : b - (TJ + NS - 1);
+            const int d = di > dj ? di : dj;
+            dq[q][cc] = (short)(in ? d : 99);
+            const uint32_t bit = 1u << (2 * q + cc);
+            if (q < QI && in && P < NPI) {
+                own |= bit;
+                if (a < 2 * NS || a >= TI || b < 2 * NS || b >= TJ) edge |= bit;
+            }
+#pragma unroll
+            for (int e = 0; e < 5; ++e) cr[q][cc][e] = c[e * n + k];
+            r[q][cc] = s.b[k];
+        }
+    }
+    double rr = 0.0;
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+#pragma unroll
+        for (int cc = 0; cc < 2; ++cc) {
+            const bool in = dq[q][cc] != 99;
+            if (!in) r[q][cc] = T(0);
+            wd[q][cc] = cr[q][cc][0] != CT(0) ? om * recip(cr[q][cc][0]) : CT(0);
+            p[q][cc] = r[q][cc];
+            v[q][cc] = T(0);
+            if (q < QI) {
+                const bool o = (own >> (2 * q + cc)) & 1u;
+                const T b = o ? r[q][cc] : T(0);
+                xs[(2 * q + cc) * NT + t] = T(0);
+                rts[(2 * q + cc) * NT + t] = b;
+                rr += (double)b * (double)b;
+                if (COARSE && o && s.mask[kq[q][cc]]) fm |= 1u << (2 * q + cc);
+            }
+        }
+    // z frame: which cells take a coarse value, and from which aggregate
+    uint32_t zm = 0;
+    short zi[COARSE ? QZ : 1];
+    int I0 = 0, J0 = 0, nI = 0, nJ = 0;
+    uint32_t slots[COARSE ? kEpt : 1];
+    if (COARSE) {
+        const int ilo = ti0 - NS - 1 < 1 ? 1 : ti0 - NS - 1, ihi = ti0 + TI + NS > nx ? nx : ti0 + TI + NS;
+        const int jlo = tj0 - NS - 1 < 1 ? 1 : tj0 - NS - 1, jhi = tj0 + TJ + NS > ny ? ny : tj0 + TJ + NS;
+        I0 = (ilo - 1) / s.B;
+        J0 = (jlo - 1) / s.B;
+        nI = (ihi - 1) / s.B - I0 + 1;
+        nJ = (jhi - 1) / s.B - J0 + 1;
+#pragma unroll
+        for (int q = 0; q < QZ; ++q) {
+            const int idx = t + q * NT;
+            const int a = idx / WZ, b = idx - (idx / WZ) * WZ;
+            const int i = ti0 - NS - 1 + a, j = tj0 - NS - 1 + b;
+            const bool in = idx < HZ * WZ && i >= 1 && i <= nx && j >= 1 && j <= ny;
+            zi[q] = in ? (short)(((i - 1) / s.B - I0) * nJ + (j - 1) / s.B - J0) : (short)0;
+            if (in && s.mask[(int64_t)i * NY + j]) zm |= 1u << q;
+        }
+        // the slots of each restricted value this thread sums that a tile writes
+#pragma unroll
+        for (int e = 0; e < kEpt; ++e) {
+            const int k = t + e * NT;
+            uint32_t u = 0;
+            if (k < s.m) {
+                const int I = k / s.mJ, J = k - I * s.mJ;
+                const int ie = ((I + 1) * s.B < nx ? (I + 1) * s.B : nx) - 1;
+                const int je = ((J + 1) * s.B < ny ? (J + 1) * s.B : ny) - 1;
+                const int ni = ie / TI - (I * s.B) / TI + 1, nj = je / TJ - (J * s.B) / TJ + 1;
+                for (int a = 0; a < ni; ++a)
+                    for (int b = 0; b < nj; ++b) u |= 1u << (a * s.SJ + b);
+            }
+            slots[e] = u;
+        }
+    }
+    // coarse rows computed here: local row f is coarse unknown unknown(f)
+    const bool shared = COARSE && s.R > 0;
+    const int row0 = L * s.R;
+    const int nF = !COARSE ? 0 : shared ? (row0 + s.R <= s.m ? s.R : (row0 < s.m ? s.m - row0 : 0)) : nI * nJ;
+    auto unknown = [&](int f) { return shared ? row0 + f : (I0 + f / nJ) * s.mJ + J0 + f % nJ; };
+    const int nc = COARSE ? (s.cached < nF ? s.cached : nF) : 0;
+    if (COARSE) {
+        for (int f = w; f < nc; f += NW) {
+            const double* __restrict__ a = s.inv + (int64_t)unknown(f) * s.m;
+            for (int k = lane; k < s.m; k += 64) dyn[(int64_t)(f + 1) * s.m + k] = a[k];
+        }
+    }
+
+    // P^T of the values in yb, one wave per piece (the part of an aggregate in
+    // this tile), published in the tile's slots
+    const int np = !COARSE ? 0 : [&]() {
+        const int r0 = ti0 - 1, c0 = tj0 - 1;
+        const int r1 = r0 + TI < nx ? r0 + TI : nx, c1 = c0 + TJ < ny ? c0 + TJ : ny;
+        const int B = s.B, A0 = r0 / B, C0 = c0 / B;
+        const int mJt = (c1 - 1) / B - C0 + 1, cnt = ((r1 - 1) / B - A0 + 1) * mJt;
+        for (int u = t; u < cnt; u += NT) {
+            const int I = A0 + u / mJt, J = C0 + u % mJt;
+            const int ra = I * B > r0 ? I * B : r0, rb = (I + 1) * B < r1 ? (I + 1) * B : r1;
+            const int ca = J * B > c0 ? J * B : c0, cb = (J + 1) * B < c1 ? (J + 1) * B : c1;
+            const int wdt = cb - ca;
+            Piece q;
+            q.at = (ra - r0) * TJ + (ca - c0);
+            q.wdt = wdt;
+            q.cnt = (rb - ra) * wdt;
+            q.dr = 64 / wdt;
+            q.dc = 64 % wdt;
+            q.inv = 65536 / wdt + 1;
+            q.dst = ((ta - (I * B) / TI) * s.SJ + (tb - (J * B) / TJ)) * s.m + I * s.mJ + J;
+            piece[COARSE ? u : 0] = q;
+        }
+        return cnt;
+    }();
+    auto restrict_yb = [&](double* rcs) {
+        __syncthreads();
+        for (int u = w; u < np; u += NW) {
+            const Piece q = piece[COARSE ? u : 0];
+            const int er = (lane * q.inv) >> 16;          // lane / wdt
+            int ec = lane - er * q.wdt, at = q.at + er * TJ + ec;
+            double acc = 0.0;
+            for (int e = lane; e < q.cnt; e += 64) {
+                acc += yb[at];
+                ec += q.dc;
+                at += q.dr * TJ + q.dc;
+                if (ec >= q.wdt) {
+                    ec -= q.wdt;
+                    at += TJ - q.wdt;
+                }
+            }
+            acc = wave_sum(acc);
+            if (lane == 0) put(rcs + q.dst, acc);
+        }
+    };
+    // A_c^-1 times the gathered restricted values: g(f, value) by lane 0.
+    // Where the rows of all aggregates under the
+    // frame fit the LDS, every workgroup computes the values it needs (an
+    // aggregate's value has the same bits wherever it is computed: no further
+    // round of exchange; 320 x 64 cells 13.3 us per iteration against 19 with
+    // two more rounds).  Where they do not, reading them from the L2 twice an
+    // iteration costs more than to share them (1280 x 256: 4 us and as much again
+    // waiting for the workgroups with more rows, against 3 us), so each
+    // workgroup computes R rows and shares them (R > 0).
+    // rows [f1, f2), row f at at(f)[k], NR rows per wave and U loads of each at a time
+    auto some_rows = [&](auto NRc, auto Uc, int f1, int f2, auto at, auto g) {
+        constexpr int NR = decltype(NRc)::value, U = decltype(Uc)::value;
+        for (int f0 = f1 + w; f0 < f2; f0 += NR * NW) {
+            decltype(at(0)) a[NR];
+            double acc[NR];
+#pragma unroll
+            for (int u = 0; u < NR; ++u) {
+                a[u] = at(f0 + u * NW < f2 ? f0 + u * NW : f0);
+                acc[u] = 0.0;
+            }
+            int k = lane;
+            for (; k + 64 * (U - 1) < s.m; k += 64 * U) {
+                double av[NR][U];
+#pragma unroll
+                for (int u = 0; u < NR; ++u)
+#pragma unroll
+                    for (int e = 0; e < U; ++e) av[u][e] = a[u][k + 64 * e];
+#pragma unroll
+                for (int e = 0; e < U; ++e) {
+                    const double d = dyn[k + 64 * e];
+#pragma unroll
+                    for (int u = 0; u < NR; ++u) acc[u] += av[u][e] * d;
+                }
+            }
+            for (; k < s.m; k += 64) {
+                const double d = dyn[k];
+#pragma unroll
+                for (int u = 0; u < NR; ++u) acc[u] += a[u][k] * d;
+            }
+#pragma unroll
+            for (int u = 0; u < NR; ++u) {
+                const double y = wave_sum(acc[u]);
+                if (lane == 0 && f0 + u * NW < f2) g(f0 + u * NW, y);
+            }
+        }
+    };
+    auto rows = [&](auto g) {
+        using std::integral_constant;
+        const auto mem = [&](int f) -> const double* { return s.inv + (int64_t)unknown(f) * s.m; };
+        const auto lds = [&](int f) { return LdsRow{(f + 1) * s.m}; };
+        if (nc < nF) some_rows(integral_constant<int, 1>(), integral_constant<int, 8>(), nc, nF, mem, g);
+        if (nc <= NW) some_rows(integral_constant<int, 1>(), integral_constant<int, 8>(), 0, nc, lds, g);
+        else some_rows(integral_constant<int, 3>(), integral_constant<int, 4>(), 0, nc, lds, g);
+    };
+    // the restricted vector from its pieces, added in slot order; the loads of
+    // a thread's first two pieces per value are in flight together
+    auto gather = [&](const double* rcs) {
+        double g0[kEpt], g1[kEpt];
+#pragma unroll
+        for (int e = 0; e < kEpt; ++e) {
+            const uint32_t u = slots[e], u1 = u & (u - 1);
+            const int k = t + e * NT;
+            g0[e] = u ? get_at(rcs, (__ffs(u) - 1) * s.m + k) : 0.0;
+            g1[e] = u1 ? get_at(rcs, (__ffs(u1) - 1) * s.m + k) : 0.0;
+        }
+#pragma unroll
+        for (int e = 0; e < kEpt; ++e) {
+            const int k = t + e * NT;
+            const uint32_t u1 = slots[e] & (slots[e] - 1);
+            double acc = g0[e] + g1[e];
+            for (uint32_t u = u1 & (u1 - 1); u; u &= u - 1) acc += get_at(rcs, (__ffs(u) - 1) * s.m + k);
+            if (k < s.m) dyn[k] = acc;
+        }
+    };
+    // the frame's coarse values from the workgroups that computed them
+    auto share = [&](const double* y, uint64_t* Y, unsigned tag) {
+        const uint64_t hi = (uint64_t)tag << 32;
+        for (int f = t; f < nF; f += NT) {
+            uint64_t* q = Y + 2 * (row0 + f);
+            put(q, hi | (uint32_t)__double2loint(y[f]));
+            put(q + 1, hi | (uint32_t)__double2hiint(y[f]));
+        }
+        if (t < nI * nJ) {
+            const uint64_t* q = Y + 2 * ((I0 + t / nJ) * s.mJ + J0 + t % nJ);
+            uint64_t a = get(q), b = get(q + 1);
+            if ((unsigned)(a >> 32) != tag || (unsigned)(b >> 32) != tag) {
+                const long long t0 = wall_clock64();
+                for (int spin = 1;; ++spin) {
+                    a = get(q);
+                    b = get(q + 1);
+                    if ((unsigned)(a >> 32) == tag && (unsigned)(b >> 32) == tag) break;
+                    if ((spin & 63) == 0 && (wall_clock64() - t0 > kWaitTicks || get(s.abort))) {
+                        put(s.abort, 1u);
+                        bad = 1;
+                        break;
+                    }
+                }
+            }
+            yl[COARSE ? t : 0] = __hiloint2double((int)(uint32_t)b, (int)(uint32_t)a);
+        }
+        __syncthreads();
+    };
+    // z = z1 from the frame's coarse values y, or 0
+    auto start_z = [&](const double* y) {
+#pragma unroll
+        for (int q = 0; q < QZ; ++q) {
+            const int idx = t + q * NT;
+            if (idx < HZ * WZ) za[idx] = COARSE && ((zm >> q) & 1u) ? (T)y[zi[COARSE ? q : 0]] : T(0);
+        }
+        __syncthreads();
+    };
+    auto sweep = [&](const T (&src)[Q][2]) {
+#pragma unroll
+        for (int hs = 0; hs < NS; ++hs) {
+            const int h = NS - hs, cc = hs & 1;
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                if (dq[q][cc] > h) continue;
+                const int z0 = pz[q][cc];
+                const CT zc = za[z0];
+                CT az = cr[q][cc][0] * zc;
+                az = az + cr[q][cc][1] * (CT)za[z0 - WZ];
+                az = az + cr[q][cc][2] * (CT)za[z0 + WZ];
+                az = az + cr[q][cc][3] * (CT)za[z0 + 1];
+                az = az + cr[q][cc][4] * (CT)za[z0 - 1];
+                za[z0] = (T)(zc + wd[q][cc] * ((CT)src[q][cc] - az));
+            }
+            __syncthreads();
+        }
+    };
+    // y = A z of an own cell
+    auto matvec = [&](int q, int cc) {
+        const int z0 = pz[q][cc];
+        CT y = cr[q][cc][0] * (CT)za[z0];
+        y = y + cr[q][cc][1] * (CT)za[z0 - WZ];
+        y = y + cr[q][cc][2] * (CT)za[z0 + WZ];
+        y = y + cr[q][cc][3] * (CT)za[z0 + 1];
+        y = y + cr[q][cc][4] * (CT)za[z0 - 1];
+        return y;
+    };
+    auto into_yb = [&](int q, int cc, double y) {
+        const int P = t + q * NT, lr = P / (TJ / 2);
+        const int lc = pz[q][cc] - (lr + NS + 1) * WZ - (NS + 1);
+        yb[lr * TJ + lc] = ((fm >> (2 * q + cc)) & 1u) ? y : 0.0;
+    };
+
+    double rho = 0.0, alpha = 0.0, omega = 1.0, r0 = 0.0, best = 1e300;
+    int it = 0, best_it = 0, status = -1;
+    __syncthreads();
+    if (COARSE) {
+        // Y(r) = Y(p) = A_c^-1 P^T rhs
+#pragma unroll
+        for (int q = 0; q < QI; ++q)
+#pragma unroll
+            for (int cc = 0; cc < 2; ++cc)
+                if (t + q * NT < NPI) into_yb(q, cc, (double)rts[(2 * q + cc) * NT + t]);
+        // (through the second buffer, whose next words follow another round)
+        restrict_yb(s.rct);
+        if (!meet<NT>(s.flags, L, G, ++round, s.abort, &bad)) status = kAborted;
+        gather(s.rct);
+        __syncthreads();
+        rows([&](int k, double y) {
+            yr[k] = y;
+            yp[k] = y;
+        });
+        __syncthreads();
+    }
+    while (status < 0) {
+        // ---- p^ = M(p), v = A p^; <r~,v>, <r,r>
+        if (shared) share(yp, s.Yp, round + 1);
+        start_z(shared ? yl : yp);
+        sweep(p);
+        {
+            double sum[3] = {0.0, rr, it == 0 ? odd : 0.0};
+#pragma unroll
+            for (int q = 0; q < QI; ++q)
+#pragma unroll
+                for (int cc = 0; cc < 2; ++cc) {
+                    const uint32_t bit = 1u << (2 * q + cc);
+                    CT y = CT(0);
+                    if (own & bit) {
+                        y = matvec(q, cc);
+                        v[q][cc] = (T)y;
+                        hps[(2 * q + cc) * NT + t] = za[pz[q][cc]];
+                        if (edge & bit) put(s.v + kq[q][cc], (T)y);
+                        sum[0] += (double)rts[(2 * q + cc) * NT + t] * (double)y;
+                    }
+                    if (COARSE && t + q * NT < NPI) into_yb(q, cc, (double)y);
+                }
+            if (COARSE) restrict_yb(s.rcv);
+            publish<3, NT>(sum, s.pa + 4 * L, red);
+        }
+        if (!meet<NT>(s.flags, L, G, ++round, s.abort, &bad)) { status = kAborted; break; }
+        double tot[3];
+        {
+            double mine[3] = {0.0, 0.0, 0.0};
+            if (t < G)
+#pragma unroll
+                for (int q = 0; q < 3; ++q) mine[q] = get_at(s.pa, 4 * t + q);
+#pragma unroll
+            for (int q = 0; q < Q; ++q)
+#pragma unroll
+                for (int cc = 0; cc < 2; ++cc)
+                    if (dq[q][cc] > 0 && dq[q][cc] <= NS) v[q][cc] = get_at(s.v, kq[q][cc]);
+            if (COARSE) gather(s.rcv);
+            totals<3, NT>(mine, G, tot, red2);   // its barrier covers dyn
+        }
+        // the stopping test and alpha (cv_scalars of km_twolevel.hip)
+        const double rvv = tot[0];
+        rr = tot[1];
+        if (it == 0) {
+            rho = rr;
+            r0 = rr;
+        }
+        if (it == 0 && tot[2] != 0.0) status = kUnsupported;
+        else if (!fin(rr)) status = KM_NONFINITE;
+        else if (it == 0 && rr == 0.0) status = KM_OK;
+        else if (it > 0 && sqrt(rr / r0) < s.eps) status = KM_OK;      // bicgsolver.py:130
+        else if (it > 0 && omega == 0.0) status = KM_BREAKDOWN;
+        else if (it >= s.max_iter) status = KM_MAXITER;
+        else if (!fin(rho)) status = KM_NONFINITE;
+        else if (rho == 0.0) status = KM_BREAKDOWN;
+        else if (!fin(rvv)) status = KM_NONFINITE;
+        else if (rvv == 0.0) status = KM_BREAKDOWN;
+        const bool better = rr < 0.81 * best;
+        if (status < 0 && !better && it - best_it >= kStallWindow) status = KM_STALL;
+        if (status >= 0) break;
+        if (better) {
+            best = rr;
+            best_it = it;
+        }
+        alpha = rho / rvv;                                              // bicgsolver.py:108
+        if (COARSE) {
+            rows([&](int k, double y) {
+                yv[k] = y;                      // Y(v)
+                ysv[k] = yr[k] - alpha * y;     // Y(s)
+            });
+        }
+        {
+            const T fa = (T)alpha;
+#pragma unroll
+            for (int q = 0; q < Q; ++q)
+#pragma unroll
+                for (int cc = 0; cc < 2; ++cc) r[q][cc] = r[q][cc] - fa * v[q][cc];   // s (bicgsolver.py:110)
+        }
+        if (COARSE) __syncthreads();
+        // ---- s^ = M(s), t = A s^; <t,s>, <t,t>, <s,r~>, <t,r~>
+        if (shared) share(ysv, s.Ys, round + 1);
+        start_z(shared ? yl : ysv);
+        sweep(r);
+        T th[Q][2];
+        {
+            double sum[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int q = 0; q < QI; ++q)
+#pragma unroll
+                for (int cc = 0; cc < 2; ++cc) {
+                    const uint32_t bit = 1u << (2 * q + cc);
+                    CT y = CT(0);
+                    th[q][cc] = T(0);
+                    if (own & bit) {
+                        y = matvec(q, cc);
+                        th[q][cc] = (T)y;
+                        if (edge & bit) put(s.t + kq[q][cc], (T)y);
+                        const double sk = (double)r[q][cc], rk = (double)rts[(2 * q + cc) * NT + t];
+                        sum[0] += (double)y * sk;
+                        sum[1] += (double)y * (double)y;
+                        sum[2] += sk * rk;
+                        sum[3] += (double)y * rk;
+                    }
+                    if (COARSE && t + q * NT < NPI) into_yb(q, cc, (double)y);
+                }
+            if (COARSE) restrict_yb(s.rct);
+            publish<4, NT>(sum, s.pb + 4 * L, red);
+        }
+        if (!meet<NT>(s.flags, L, G, ++round, s.abort, &bad)) { status = kAborted; break; }
+        double pt[4];
+        {
+            double mine[4] = {0.0, 0.0, 0.0, 0.0};
+            if (t < G)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) mine[q] = get_at(s.pb, 4 * t + q);
+#pragma unroll
+            for (int q = 0; q < Q; ++q)
+#pragma unroll
+                for (int cc = 0; cc < 2; ++cc) {
+                    if (q >= QI) th[q][cc] = T(0);
+                    if (dq[q][cc] > 0 && dq[q][cc] <= NS) th[q][cc] = get_at(s.t, kq[q][cc]);
+                }
+            if (COARSE) gather(s.rct);
+            totals<4, NT>(mine, G, pt, red2);
+        }
+        // omega, rho, beta (ct_scalars of km_twolevel.hip)
+        omega = pt[1] != 0.0 ? pt[0] / pt[1] : 0.0;                          // bicgsolver.py:118
+        const double rho1 = pt[2] - omega * pt[3];                           // bicgsolver.py:95
+        const double beta = omega != 0.0 ? (rho1 / rho) * (alpha / omega) : 0.0;   // bicgsolver.py:102
+        rho = rho1;
+        if (COARSE) {
+            rows([&](int k, double y) {
+                const double v1 = ysv[k] - omega * y;                        // Y(r)
+                yr[k] = v1;
+                yp[k] = v1 + beta * (yp[k] - omega * yv[k]);                 // Y(p)
+            });
+        }
+        const T fo = (T)omega, fb = (T)beta;
+        rr = 0.0;
+#pragma unroll
+        for (int q = 0; q < Q; ++q)
+#pragma unroll
+            for (int cc = 0; cc < 2; ++cc) {
+                const T rn = r[q][cc] - fo * th[q][cc];                      // bicgsolver.py:134
+                r[q][cc] = rn;
+                p[q][cc] = rn + fb * (p[q][cc] - fo * v[q][cc]);             // bicgsolver.py:103
+                if (q < QI && ((own >> (2 * q + cc)) & 1u)) {
+                    // s^ is still in za
+                    const int o = (2 * q + cc) * NT + t;
+                    xs[o] = xs[o] + (T)(alpha * (double)hps[o] + omega * (double)za[pz[q][cc]]);
+                    rr += (double)rn * (double)rn;
+                }
+            }
+        ++it;
+        __syncthreads();   // za is read above and written by the next start_z, yp the other way round
+    }
+#pragma unroll
+    for (int q = 0; q < QI; ++q)
+#pragma unroll
+        for (int cc = 0; cc < 2; ++cc)
+            if ((own >> (2 * q + cc)) & 1u) s.x[kq[q][cc]] = status < kUnsupported ? xs[(2 * q + cc) * NT + t] : T(0);
+    if (t == 0 && (L == 0 || status == kAborted)) {
+        // the host's words (read after the stream has been waited for)
+        if (L == 0) {
+            __hip_atomic_store(s.hw + 1, it, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            __hip_atomic_store(s.hw + 2, status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            __hip_atomic_store(reinterpret_cast<double*>(s.hw + 4), r0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            __hip_atomic_store(reinterpret_cast<double*>(s.hw + 6), rr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+        if (status == kAborted) __hip_atomic_store(s.hw + 3, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (L == 0) __hip_atomic_store(s.hw, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+template <typename T, typename CT, int TI, int TJ, int NT, int SW, bool COARSE>
+__global__ void __launch_bounds__(NT) k_solve(PSys<T> s) {
+    solve_body<T, CT, TI, TJ, NT, SW, COARSE>(s, xcd_remap(blockIdx.x, s.G));
+}
+
+// Two independent systems: workgroups [0, a.G) the first, the rest the second.
+template <typename T, typename CT, int TI, int TJ, int NT, int SW>
+__global__ void __launch_bounds__(NT) k_solve2(PSys<T> a, PSys<T> b) {
+    const bool first = (int)blockIdx.x < a.G;
+    const PSys<T>& s = first ? a : b;
+    solve_body<T, CT, TI, TJ, NT, SW, false>(s, xcd_remap(first ? blockIdx.x : blockIdx.x - a.G, s.G));
+}
+
+// Launches of one device in one process follow each other: two of them side
+// by side could each hold compute units the other waits for.
+struct Gate {
+    std::mutex m;
+    hipEvent_t last = nullptr;
+    hipStream_t stream = nullptr;
+    bool any = false;
+};
+constexpr int kMaxDevices = 64;
+Gate g_gate[kMaxDevices];
+
+int tiles_of(int n, int T) { return (n + T - 1) / T; }
+
+int slots_along(int n, int B, int Tt) {
+    int most = 1;
+    for (int I = 0; I * B < n; ++I) {
+        const int e = ((I + 1) * B < n ? (I + 1) * B : n) - 1;
+        most = std::max(most, e / Tt - (I * B) / Tt + 1);
+    }
+    return most;
+}
+
+// At most this many aggregates of size B lie under a tile's z frame.
+int frame_rows(int B, int shape) {
+    const int h = 2 * (2 * kmcoarse::kSweeps + 1);
+    return ((kTI[shape] + h - 2) / B + 2) * ((kTJ[shape] + h - 2) / B + 2);
+}
+
+// Bytes of solve_body's LDS arrays with a coarse level, rounded up.
+size_t solve_lds(int TI, int TJ, int NT, int sweeps, size_t vec) {
+    const int h = 2 * (2 * sweeps + 1);
+    const size_t QI = (TI * TJ / 2 + NT - 1) / NT;
+    return (TI + h) * (TJ + h) * vec + (size_t)TI * TJ * 8 + 6 * QI * NT * vec + kMaxF * (5 * 8 + sizeof(Piece)) + 4096;
+}
+
+int compute_units(km_ctx* ctx) {
+    static std::mutex m;
+    static int cus[kMaxDevices] = {};
+    if (ctx->device < 0 || ctx->device >= kMaxDevices) return 0;
+    std::lock_guard<std::mutex> lk(m);
+    if (!cus[ctx->device]) {
+        int v = 0;
+        if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, ctx->device) != hipSuccess) v = 0;
+        cus[ctx->device] = v > 0 ? v : -1;
+    }
+    return std::max(0, cus[ctx->device]);
+}
+
+// The words that hold round numbers: flags, the abort word, Y.
+constexpr size_t kFlagBytes = (size_t)2 * kMaxWg * kFlagStride * sizeof(unsigned);
+constexpr size_t kWords = kFlagBytes + 256 + (size_t)4 * kMaxM * sizeof(uint64_t);
+
+int ensure(km_ctx* ctx) {
+    if (km_persist* K = ctx->persist) {
+        if (!K->clean || K->round > 0xe0000000u) {
+            KM_HIP(ctx, hipMemsetAsync(K->arena, 0, kWords, ctx->stream));
+            K->round = 0;
+        }
+        K->clean = false;   // until the launch has ended well
+        return KM_OK;
+    }
+    km_persist* K = new km_persist();
+    const size_t pt = (size_t)4 * kMaxWg * 4 * sizeof(double);
+    const size_t rc = (size_t)2 * kMaxSlots * kMaxM * sizeof(double);
+    void* q = nullptr;
+    hipError_t e;
+    {
+        KmHostLock lk(km_host_mutex());
+        e = hipSetDevice(ctx->device);
+        if (e == hipSuccess) e = hipMalloc(&q, kWords + pt + rc);
+    }
+    if (e == hipSuccess) e = hipMemsetAsync(q, 0, kWords, ctx->stream);
+    if (e != hipSuccess) {
+        if (q) (void)hipFree(q);
+        delete K;
+        return km_fail(ctx, KM_ENOMEM, "exchange buffers: %s", hipGetErrorString(e));
+    }
+    char* a = K->arena = static_cast<char*>(q);
+    K->flags = reinterpret_cast<unsigned*>(a);
+    K->abort = reinterpret_cast<unsigned*>(a + kFlagBytes);
+    K->Y = reinterpret_cast<uint64_t*>(a + kFlagBytes + 256);
+    K->part = reinterpret_cast<double*>(a + kWords);
+    K->rc = reinterpret_cast<double*>(a + kWords + pt);
+    ctx->persist = K;
+    return KM_OK;
+}
+
+template <typename T>
+PSys<T> system(km_ctx* ctx, int slot, int shape, int NX, int NY, const void* c, const T* b, T* x, T* ws, double eps,
+               int max_iter, double om) {
+    km_persist* K = ctx->persist;
+    const int64_t n = (int64_t)NX * NY;
+    PSys<T> s{};
+    s.NX = NX;
+    s.NY = NY;
+    s.tiles_j = tiles_of(NY - 2, kTJ[shape]);
+    s.G = tiles_of(NX - 2, kTI[shape]) * s.tiles_j;
+    s.c = c;
+    s.b = b;
+    s.x = x;
+    s.v = ws;
+    s.t = ws + n;
+    s.flags = K->flags + (size_t)(slot * kMaxWg) * kFlagStride;
+    s.abort = K->abort;
+    s.round = K->round;
+    s.pa = K->part + (size_t)(slot * 2) * kMaxWg * 4;
+    s.pb = s.pa + (size_t)kMaxWg * 4;
+    s.eps = eps;
+    s.max_iter = max_iter;
+    s.om = (T)om;
+    s.hw = ctx->d_flag + KM_HW * slot;
+    return s;
+}
+
+// Launch, the tail, and the final states; *ran = false if it gave up.
+int finish(km_ctx* ctx, int nsys, const std::function<void()>& launch, KState* out, const std::function<int()>* tail,
+           bool* ran) {
+    km_persist* K = ctx->persist;
+    volatile int* hf = ctx->h_flag;
+    for (int q = 0; q < nsys; ++q)
+        for (int k = 0; k < 4; ++k) hf[KM_HW * q + k] = 0;
+    std::atomic_thread_fence(std::memory_order_seq_cst);
+    {
+        Gate& g = g_gate[ctx->device];
+        std::lock_guard<std::mutex> lk(g.m);
+        if (!g.last) KM_HIP_SYNC(ctx, hipEventCreateWithFlags(&g.last, hipEventDisableTiming));
+        if (g.any && g.stream != ctx->stream) KM_HIP(ctx, hipStreamWaitEvent(ctx->stream, g.last, 0));
+        launch();
+        KM_CHECK_LAUNCH(ctx);
+        KM_HIP(ctx, hipEventRecord(g.last, ctx->stream));
+        g.any = true;
+        g.stream = ctx->stream;
+    }
+    if (tail)
+        if (int rc = (*tail)()) return rc;
+    KM_HIP_SYNC(ctx, hipStreamSynchronize(ctx->stream));
+    std::atomic_thread_fence(std::memory_order_acquire);
+    *ran = true;
+    bool aborted = false;
+    for (int q = 0; q < nsys; ++q) {
+        volatile int* w = hf + KM_HW * q;
+        KState& f = out[q];
+        f = KState{};
+        f.done = w[0];
+        f.iter = w[1];
+        f.status = w[2];
+        f.r0 = *reinterpret_cast<volatile double*>(w + 4);
+        f.rTr = *reinterpret_cast<volatile double*>(w + 6);
+        aborted = aborted || w[3];
+        if (!f.done) return km_fail(ctx, KM_EHIP, "solver stopped without reporting completion");
+        if (f.status >= kUnsupported) *ran = false;
+    }
+    if (aborted) {
+        *ran = false;
+        K->off++;
+        return KM_OK;
+    }
+    int most = 0;
+    for (int q = 0; q < nsys; ++q) most = std::max(most, out[q].iter);
+    K->round += 2 * (unsigned)most + 8;
+    K->clean = true;
+    return KM_OK;
+}
+
+}  // namespace
+
+namespace kmpersist {
+
+bool fits_twolevel(km_ctx* ctx, const km_coarse* C, int NX, int NY, int* shape) {
+    if (!C || C->m > kMaxM || (ctx->persist && ctx->persist->off >= 2)) return false;
+    const int cus = std::min(kMaxWg, compute_units(ctx));
+    const int nx = NX - 2, ny = NY - 2;
+    for (int k = 0; k < kNumShapes; ++k) {
+        const int64_t G = (int64_t)tiles_of(nx, kTI[k]) * tiles_of(ny, kTJ[k]);
+        if (G > cus) continue;
+        const int B = C->B;
+        if (C->m > kEpt * kNT[k]) return false;
+        if (slots_along(nx, B, kTI[k]) * slots_along(ny, B, kTJ[k]) > kMaxSlots) return false;
+        if (frame_rows(B, k) > kMaxF || (C->m + G - 1) / G > kMaxF) return false;
+        *shape = k;
+        return true;
+    }
+    return false;
+}
+
+// A system that fits half of the compute units with one of the first
+// kHalfShapes shapes takes the smallest that does, so that u and v share a
+// launch; a larger one takes the smallest that fits all of them.  The rule
+// looks at one system only: a pair's results are those of two solves.
+constexpr int kHalfShapes = 4;
+
+bool fits_smooth(km_ctx* ctx, int NX, int NY, int* shape) {
+    if (ctx->persist && ctx->persist->off >= 2) return false;
+    const int cus = std::min(kMaxWg, compute_units(ctx));
+    for (int half = 1; half >= 0; --half)
+        for (int k = 0; k < (half ? kHalfShapes : kNumShapes); ++k) {
+            const int64_t G = (int64_t)tiles_of(NX - 2, kTI[k]) * tiles_of(NY - 2, kTJ[k]);
+            if (G > (half ? cus / 2 : cus)) continue;
+            *shape = k;
+            return true;
+        }
+    return false;
+}
+
+#define KM_SHAPES(X) X(0) X(1) X(2) X(3) X(4) X(5)
+
+template <typename T>
+int twolevel(km_ctx* ctx, int shape, int NX, int NY, const double* coef, const T* rhs, T* xd, T* ws, double eps,
+             int max_iter, KState* out, const std::function<int()>* tail, bool* ran) {
+    if (int rc = ensure(ctx)) return rc;
+    const km_coarse* C = ctx->coarse;
+    km_persist* K = ctx->persist;
+    PSys<T> s = system<T>(ctx, 0, shape, NX, NY, coef, rhs, xd, ws, eps, max_iter, kmcoarse::kOmega);
+    s.B = C->B;
+    s.mJ = C->mJ;
+    s.m = C->m;
+    s.SJ = slots_along(NY - 2, C->B, kTJ[shape]);
+    s.mask = C->mask;
+    s.inv = C->inv;
+    s.rcv = K->rc;
+    s.rct = K->rc + (size_t)kMaxSlots * kMaxM;
+    // the restricted vector, then as many rows of A_c^-1 as fit
+    const size_t row = (size_t)C->m * sizeof(double);
+    const size_t fixed = solve_lds(kTI[shape], kTJ[shape], kNT[shape], kmcoarse::kSweeps, sizeof(T));
+    const int room = fixed + row < kLdsBytes ? (int)((kLdsBytes - fixed) / row) - 1 : 0;
+    const int under = std::min(frame_rows(C->B, shape), C->m);
+    s.R = room >= under ? 0 : (C->m + s.G - 1) / s.G;
+    s.cached = std::min(room, s.R > 0 ? s.R : under);
+    s.Yp = K->Y;
+    s.Ys = K->Y + 2 * kMaxM;
+    const size_t lds = row * (1 + s.cached);
+    auto launch = [&]() {
+        switch (shape) {
+#define KM_CASE(I)                                                                                                 \
+    case I:                                                                                                        \
+        hipLaunchKernelGGL((k_solve<T, double, kTI[I], kTJ[I], kNT[I], kmcoarse::kSweeps, true>), dim3(s.G),       \
+                           dim3(kNT[I]), lds, ctx->stream, s);                                                     \
+        break;
+            KM_SHAPES(KM_CASE)
+#undef KM_CASE
+        }
+    };
+    return finish(ctx, 1, launch, out, tail, ran);
+}
+
+template <typename T>
+int smooth(km_ctx* ctx, int nsys, const int* NX, const int* NY, const T* const* coef, const T* const* rhs,
+           T* const* xd, T* const* ws, double eps, const int* max_iter, int sweeps, KState* out,
+           const std::function<int()>* tail, bool* ran) {
+    if (int rc = ensure(ctx)) return rc;
+    PSys<T> s[2] = {};
+    int shape[2] = {0, 0};
+    for (int q = 0; q < nsys; ++q) {
+        KM_REQUIRE(ctx, fits_smooth(ctx, NX[q], NY[q], &shape[q]), "system %d does not fit one launch", q);
+        s[q] = system<T>(ctx, q, shape[q], NX[q], NY[q], coef[q], rhs[q], xd[q], ws[q], eps, max_iter[q], 1.0);
+    }
+    const bool together = nsys == 2 && shape[0] == shape[1] && s[0].G + s[1].G <= std::min(kMaxWg, compute_units(ctx));
+    auto one = [&](int sh, const PSys<T>& a, const PSys<T>& b) {
+        switch (sh * 2 + (sweeps == 2 ? 1 : 0)) {
+#define KM_CASE(I)                                                                                                 \
+    case 2 * I:                                                                                                    \
+        hipLaunchKernelGGL((k_solve2<T, T, kTI[I], kTJ[I], kNT[I], 1>), dim3(a.G + b.G), dim3(kNT[I]), 0,          \
+                           ctx->stream, a, b);                                                                     \
+        break;                                                                                                     \
+    case 2 * I + 1:                                                                                                \
+        hipLaunchKernelGGL((k_solve2<T, T, kTI[I], kTJ[I], kNT[I], 2>), dim3(a.G + b.G), dim3(kNT[I]), 0,          \
+                           ctx->stream, a, b);                                                                     \
+        break;
+            KM_SHAPES(KM_CASE)
+#undef KM_CASE
+        }
+    };
+    auto launch = [&]() {
+        const PSys<T> none{};
+        if (together) {
+            one(shape[0], s[0], s[1]);
+        } else {
+            for (int q = 0; q < nsys; ++q) one(shape[q], s[q], none);
+        }
+    };
+    return finish(ctx, nsys, launch, out, tail, ran);
+}
+
+template int twolevel<double>(km_ctx*, int, int, int, const double*, const double*, double*, double*, double, int,
+                              KState*, const std::function<int()>*, bool*);
+template int twolevel<float>(km_ctx*, int, int, int, const double*, const float*, float*, float*, double, int, KState*,
+                             const std::function<int()>*, bool*);
+template int smooth<double>(km_ctx*, int, const int*, const int*, const double* const*, const double* const*,
+                            double* const*, double* const*, double, const int*, int, KState*,
+                            const std::function<int()>*, bool*);
+template int smooth<float>(km_ctx*, int, const int*, const int*, const float* const*, const float* const*,
+                           float* const*, float* const*, double, const int*, int, KState*,
+                           const std::function<int()>*, bool*);
+
+}  // namespace kmpersist
+
+void km_persist_free(km_ctx* ctx) {
+    if (!ctx->persist) return;
+    KmHostLock lk(km_host_mutex());
+    if (ctx->persist->arena) (void)hipFree(ctx->persist->arena);
+    delete ctx->persist;
+    ctx->persist = nullptr;
+}

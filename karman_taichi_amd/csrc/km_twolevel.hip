@@ -32,6 +32,7 @@
 // into its own slot: slot (a - I B / TI) SJ + (b - J B / TJ) of aggregate
 // (I, J).  The coarse launches sum the slots in slot order.
 #include "km_coarse.h"
+#include "km_persist.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -1219,8 +1220,13 @@ int set_tile(km_ctx* ctx, int which) {
     for_each_level(ctx, [&](km_coarse* L) {
         for (int sz : {(int)sizeof(float), (int)sizeof(double)}) {
             const auto key = std::make_tuple(NX, NY, sz);
-            if (which < 0) L->tiles.erase(key);
-            else L->tiles[key] = which;
+            if (which < 0) {
+                L->tiles.erase(key);
+                L->pinned.erase(key);
+            } else {
+                L->tiles[key] = which;
+                L->pinned.insert(key);
+            }
         }
     });
     return KM_OK;
@@ -1463,6 +1469,13 @@ void record_solve(km_coarse* C, int iters) {
 
 }  // namespace
 
+// A level whose smoothing tile was pinned solves by launches with that tile.
+template <typename T>
+bool one_launch(km_ctx* ctx, const km_coarse* C, int* shape) {
+    return !C->pinned.count(std::make_tuple(C->NX, C->NY, (int)sizeof(T))) &&
+           kmpersist::fits_twolevel(ctx, C, C->NX, C->NY, shape);
+}
+
 template <typename T>
 int fused_inner(km_ctx* ctx, int NX, int NY, const T* coefT, const T* rhs, T* xd, T* ws, double eps, int max_iter,
                 bool use_graph, KState* out, const std::function<int()>* tail, bool sym, const double* coef64) {
@@ -1470,6 +1483,16 @@ int fused_inner(km_ctx* ctx, int NX, int NY, const T* coefT, const T* rhs, T* xd
     KM_REQUIRE(ctx, C && C->arena && C->NX == NX && C->NY == NY, "coarse level not set up for this system");
     if (sizeof(T) == sizeof(double)) coef64 = reinterpret_cast<const double*>(coefT);
     KM_REQUIRE(ctx, coef64, "the FP32-vector two-level solve needs the FP64 coefficients");
+    int shape = 0;
+    if (one_launch<T>(ctx, C, &shape)) {
+        bool ran = false;
+        if (int rc = kmpersist::twolevel<T>(ctx, shape, NX, NY, coef64, rhs, xd, ws, eps, max_iter, out, tail, &ran))
+            return rc;
+        if (ran) {
+            record_solve(C, out->iter);
+            return KM_OK;
+        }
+    }
     int tile = 0;
     if (int rc = tuned_tile<T>(ctx, coefT, rhs, ws, &tile, sym, coef64)) return rc;
     const Fused<T> f(ctx, NX, NY, coefT, ws, xd, tile, sym, coef64);
@@ -1813,6 +1836,13 @@ int smooth_inner(km_ctx* ctx, int NX, int NY, const T* coefT, const T* rhs, T* x
                  bool use_graph, KState* out, const std::function<int()>* tail) {
     KM_REQUIRE(ctx, (int64_t)NX * NY < kTileCellsMax, "system of %lld cells is too large for the tile kernels",
                (long long)NX * NY);
+    int shape = 0;
+    if (kmpersist::fits_smooth(ctx, NX, NY, &shape)) {
+        bool ran = false;
+        const int rc = kmpersist::smooth<T>(ctx, 1, &NX, &NY, &coefT, &rhs, &xd, &ws, eps, &max_iter,
+                                            mom_sweeps<T>(ctx, (int64_t)NX * NY), out, tail, &ran);
+        if (rc || ran) return rc;
+    }
     const SmoothFused<T> f(NX, NY, coefT, ws, xd, &ctx->st[4], ctx->partials, ctx->d_flag,
                            mom_sweeps<T>(ctx, (int64_t)NX * NY));
     f.init(ctx->stream, rhs, eps, max_iter);
@@ -1835,6 +1865,12 @@ int smooth_inner2(km_ctx* ctx, const int* NX, const int* NY, const T* const* coe
     // host words of the second system beyond the first's; both systems take
     // the larger one's sweep count (one kernel serves both)
     const int sw = mom_sweeps<T>(ctx, std::max((int64_t)NX[0] * NY[0], (int64_t)NX[1] * NY[1]));
+    int shape = 0;
+    if (kmpersist::fits_smooth(ctx, NX[0], NY[0], &shape) && kmpersist::fits_smooth(ctx, NX[1], NY[1], &shape)) {
+        bool ran = false;
+        const int rc = kmpersist::smooth<T>(ctx, 2, NX, NY, coefT, rhs, xd, ws, eps, max_iter, sw, out, tail, &ran);
+        if (rc || ran) return rc;
+    }
     const SmoothFused<T> a(NX[0], NY[0], coefT[0], ws[0], xd[0], &ctx->st[4], ctx->partials, ctx->d_flag, sw);
     const SmoothFused<T> b(NX[1], NY[1], coefT[1], ws[1], xd[1], &ctx->st[5], ctx->partials + kPairPartials,
                            ctx->d_flag + KM_HW, sw);
@@ -1859,6 +1895,7 @@ template int smooth_inner2<double>(km_ctx*, const int*, const int*, const double
                                    double* const*, double* const*, double, const int*, bool, KState*,
                                    const std::function<int()>*);
 
+template bool one_launch<double>(km_ctx*, const km_coarse*, int*);
 template int smooth<float>(km_ctx*, const float*, const float*, float*, hipStream_t);
 template int smooth<double>(km_ctx*, const double*, const double*, double*, hipStream_t);
 template int fused_inner<float>(km_ctx*, int, int, const float*, const float*, float*, float*, double, int, bool,

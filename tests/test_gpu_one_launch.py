@@ -1,0 +1,86 @@
+"""The preconditioned solves that run in one launch (csrc/km_persist.hip),
+against the direct solution, at the edges of its tile shapes.
+
+Tolerance: a solve ends with ||b - A x|| < eps ||b||, so its error is at most
+eps ||A^-1|| ||b||; with x* the direct solution that is eps cond(A) ||x*||
+at most.  With row sums of 0.01 or more and aP of at most 7, cond(A) <= 2 * 7 / 0.01
+< 1e4: the bound is 1e4 eps, eps = 1e-10.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from karman_taichi_amd import _lib
+from karman_taichi_amd._lib import KmSolveInfo
+from oracle import krylov
+
+pytestmark = pytest.mark.gpu
+EPS = 1e-10
+
+
+def system(NX, NY, seed, diagonal):
+    """A symmetric system with links of 0.5 to 1.5, an obstacle of identity
+    rows where there is room, and `diagonal` added to every row."""
+    rng = np.random.default_rng(seed)
+    coef, b = np.zeros((5, NX, NY)), np.zeros((NX, NY))
+    coef[2, 1:NX - 2, 1:NY - 1] = -(rng.random((NX - 3, NY - 2)) + 0.5)
+    coef[3, 1:NX - 1, 1:NY - 2] = -(rng.random((NX - 2, NY - 3)) + 0.5)
+    solid = np.zeros((NX, NY), bool)
+    if NX > 12 and NY > 12:
+        solid[5:8, 6:9] = True
+    coef[2, :-1][solid[:-1] | solid[1:]] = 0.0
+    coef[3, :, :-1][solid[:, :-1] | solid[:, 1:]] = 0.0
+    coef[1, 1:], coef[4, :, 1:] = coef[2, :-1], coef[3, :, :-1]
+    coef[0, 1:-1, 1:-1] = diagonal - coef[1:, 1:-1, 1:-1].sum(axis=0)
+    coef[0][solid] = 1.0
+    b[1:-1, 1:-1] = rng.standard_normal((NX - 2, NY - 2))
+    b[solid] = 0.0
+    return coef, b
+
+
+def solve(dev, coef, b, flags):
+    c, bt = torch.tensor(coef, device=dev), torch.tensor(b, device=dev)
+    x = torch.full_like(bt, 7.0)     # every cell is written, boundary cells too
+    info = KmSolveInfo()
+    ctx = _lib.Context(torch.cuda.current_device(), torch.cuda.current_stream(dev).cuda_stream)
+    try:
+        ctx.call("km_fbicgstab", b.shape[0], b.shape[1], ctypes.c_void_p(c.data_ptr()), ctypes.c_void_p(bt.data_ptr()),
+                 ctypes.c_void_p(x.data_ptr()), EPS, 0, flags, None, ctypes.byref(info))
+        torch.cuda.synchronize()
+    finally:
+        ctx.close()
+    return x.cpu().numpy(), info
+
+
+def check(x, info, coef, b):
+    xd = krylov.direct_solve(coef, b)
+    err = np.linalg.norm(x - xd) / np.linalg.norm(xd)
+    print(f"{b.shape}: {info.iterations} it, true residual {info.rel_resid_true:.1e}, error {err:.1e}")
+    assert info.status == _lib.KM_OK and info.fallback == 0
+    assert info.rel_resid_true < EPS
+    assert err <= 1e4 * EPS
+
+
+# one cell over and under the tiles (16 x 16, 16 x 32, 32 x 32, 40 x 32, 48 x 32,
+# 48 x 48 cells), a single tile, and 256 tiles of a shape (where the next begins)
+SHAPES = [(6, 5), (18, 18), (19, 17), (50, 34), (49, 67), (258, 258), (259, 258), (258, 515), (514, 516)]
+
+
+@pytest.mark.parametrize("NX,NY", SHAPES)
+@pytest.mark.parametrize("mixed", [0, _lib.KM_FLAG_MIXED])
+@pytest.mark.parametrize("kind", [_lib.KM_FLAG_COARSE | _lib.KM_FLAG_SYMMETRIC, _lib.KM_FLAG_SMOOTH])
+def test_one_launch_matches_direct_solution(NX, NY, mixed, kind, dev):
+    coef, b = system(NX, NY, NX + NY, 1.0 if kind == _lib.KM_FLAG_SMOOTH else 0.01)
+    x, info = solve(dev, coef, b, kind | mixed)
+    check(x, info, coef, b)
+
+
+def test_coupled_boundary_rows_take_the_launches(dev):
+    """A system whose boundary rows are not empty is not the one-launch
+    kernel's: it says so and the solve by launches follows."""
+    coef, b = system(40, 36, 3, 1.0)
+    coef[0, 0, 5], b[0, 5] = 2.0, 1.0
+    x, info = solve(dev, coef, b, _lib.KM_FLAG_SMOOTH)
+    check(x, info, coef, b)
