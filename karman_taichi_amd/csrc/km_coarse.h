@@ -31,6 +31,7 @@ struct km_coarse {
     bool refresh = false;     // a solve ran long: factor on the next set-up
     int totals = -1;          // km_set_coarse_totals: -1 automatic, 0 never, 1 always
     int recent[8] = {};       // iteration counts of the last fused solves of this shape (0: none)
+    double paced[8] = {};     // the same per eight decades of residual (0: none)
     int chunk_big = 8, chunk_small = 2, chunk_lead = 2;   // km_set_coarse_chunks
     uint64_t used = 0;        // coarse_tick of the last solve that used this level
     // tile shape of the fused smoothing launches per (NX, NY, sizeof T)

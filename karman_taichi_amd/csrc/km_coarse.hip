@@ -641,7 +641,7 @@ int setup(km_ctx* ctx, int NX, int NY, const double* coef, hipStream_t s, bool s
     // the held inverse belongs to a coarse level of the same shape: try the update
     const bool same = C->held && C->NX == NX && C->NY == NY && C->B == B;
     if (!(C->NX == NX && C->NY == NY && C->B == B))   // another system shape
-        for (int& c : C->recent) c = 0;
+        for (int k = 0; k < 8; ++k) C->recent[k] = 0, C->paced[k] = 0.0;
     // a solve of the system set up last time (same coefficient array) may run
     // with a lagged coarse inverse: the flexible solve only needs an
     // approximate one

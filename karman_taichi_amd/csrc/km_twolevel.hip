@@ -1455,16 +1455,26 @@ int expected_iterations(const km_coarse* C) {
     return expect;
 }
 
-// The level's record of a finished solve: its iteration count, and a solve
-// over twice as long as the shortest recent one asks for a refactorisation
-// (the lagged coarse inverse no longer serves).
-void record_solve(km_coarse* C, int iters) {
+// The level's record of a finished solve to eps: its iteration count (for
+// expected_iterations), and whether the lagged coarse inverse still serves.  A
+// solve over twice as long as the shortest recent one, both counted per eight
+// decades of residual, asks for a refactorisation.  Per decade because the
+// sweeps of one FP64 refinement stop at different depths: by plain counts a
+// last sweep of two iterations made the next first sweep of ten look slow, and
+// 11 of 24 solves of a 717 x 143 mixed-precision run refactored (3 ms each;
+// 4.2 -> 1.5 ms per outer step).  Sweeps of less than two decades say nothing.
+void record_solve(km_coarse* C, int iters, double eps) {
     for (int k = 7; k > 0; --k) C->recent[k] = C->recent[k - 1];
     C->recent[0] = iters;
-    int shortest = 0;
-    for (int k = 1; k < 8; ++k)
-        if (C->recent[k] > 0 && (shortest == 0 || C->recent[k] < shortest)) shortest = C->recent[k];
-    if (shortest > 0 && iters > 2 * shortest + 4) C->refresh = true;
+    const double decades = -std::log10(eps);
+    if (!(decades >= 2.0)) return;
+    const double paced = iters * (8.0 / decades);
+    double shortest = 0.0;
+    for (double p : C->paced)
+        if (p > 0.0 && (shortest == 0.0 || p < shortest)) shortest = p;
+    for (int k = 7; k > 0; --k) C->paced[k] = C->paced[k - 1];
+    C->paced[0] = paced;
+    if (shortest > 0.0 && paced > 2.0 * shortest + 4.0) C->refresh = true;
 }
 
 }  // namespace
@@ -1489,7 +1499,7 @@ int fused_inner(km_ctx* ctx, int NX, int NY, const T* coefT, const T* rhs, T* xd
         if (int rc = kmpersist::twolevel<T>(ctx, shape, NX, NY, coef64, rhs, xd, ws, eps, max_iter, out, tail, &ran))
             return rc;
         if (ran) {
-            record_solve(C, out->iter);
+            record_solve(C, out->iter, eps);
             return KM_OK;
         }
     }
@@ -1507,7 +1517,7 @@ int fused_inner(km_ctx* ctx, int NX, int NY, const T* coefT, const T* rhs, T* xd
     const int expect = expected_iterations(C);
     const int rc = run_chunks_flag(ctx, key, use_graph, C->chunk_big, C->chunk_small, expect, max_iter,
                                    enqueue, out, tail);
-    if (rc == KM_OK) record_solve(C, out->iter);
+    if (rc == KM_OK) record_solve(C, out->iter, eps);
     return rc;
 }
 
@@ -1557,7 +1567,7 @@ int fused_inner_n(km_ctx* ctx, int n, km_coarse* const* C, const int* NX, const 
     const int rc = run_chunks_flag(ctx, key, use_graph, C[0]->chunk_big, C[0]->chunk_small, history ? expect : 0, mi,
                                    enqueue, out, tail, n);
     if (rc == KM_OK)
-        for (int k = 0; k < n; ++k) record_solve(C[k], out[k].iter);
+        for (int k = 0; k < n; ++k) record_solve(C[k], out[k].iter, eps);
     return rc;
 }
 
