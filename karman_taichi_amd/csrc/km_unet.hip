@@ -270,121 +270,218 @@ k_conv3x3(int H, int W, const bf16* __restrict__ src0, const bf16* __restrict__ 
     }
 }
 
-// Weight gradient: one wave accumulates RT x CT output tiles (16 x 16) over
-// its share of the pixels (K = pixels, 32 per MFMA); partial sums per wave go
-// to part[(split * 4 + wave)][COUT][KP] and are summed in a fixed order by
-// k_wgrad_reduce.  Workgroup (split, column group).
+// Weight gradient: a workgroup (split, column group) runs over its share of the
+// pixels (K = pixels, 32 per MFMA), each wave accumulating RT x CT output tiles
+// (16 x 16) of its own columns; the workgroup's partial sums go to
+// part[split][COUT][KP] and are summed in a fixed order by k_wgrad_reduce.
+//
+// An operand fragment is eight pixels of one channel, and memory holds the
+// channels of a pixel side by side: fetched two bytes at a time from memory
+// every fragment took eight loads with their own index arithmetic, and the
+// kernel waited for them (609 us for the 48-channel layer at 4 x 1280 x 256
+// pixels, 1.1 TFLOP/s).  Now the workgroup brings kWgPx pixels of dY and, for
+// the three rows of taps, kWgPx + 2 pixels of the input into LDS with 16-byte
+// loads, once for all nine taps and all waves, and the fragments are gathered
+// there.  Pixels are taken in linear order (a tap is a shift of dy W + dx); a
+// tap that leaves the image is cleared by each lane's pixel masks.  The pixel
+// stride in LDS is CIN + 2 values: the four 8-pixel groups of a fragment then
+// start 8 banks apart.
+constexpr int kWgPx = 64;
+
 template <int MODE, int C0, int C1, int COUT, int CT>
 __global__ void __launch_bounds__(KM_BLOCK)
 k_wgrad(int H, int W, int B, const bf16* __restrict__ src0, const bf16* __restrict__ src1,
-        const bf16* __restrict__ dY, int64_t pps, float* __restrict__ part) {
+        const bf16* __restrict__ dY, int pps, float* __restrict__ part) {
     constexpr int CIN = C0 + C1;
     constexpr int KP = round32(9 * CIN);
     constexpr int NCT = KP / 16;
     constexpr int RT = COUT / 16;
+    constexpr int LX = CIN + 2, LY = COUT + 2;          // pixel strides in LDS
+    constexpr int VX = CIN / 8, VY = COUT / 8;          // 16-byte vectors per pixel
+    constexpr int NX3 = 3 * (kWgPx + 2) * VX, NY1 = kWgPx * VY;
+    __shared__ bf16 xs[3 * (kWgPx + 2) * LX];
+    __shared__ bf16 ys[kWgPx * LY];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int g = lane >> 4, col = lane & 15;
-    const int64_t HW = (int64_t)H * W, NPX = (int64_t)B * HW;
-    const int split = blockIdx.x, cg = blockIdx.y;
-    const int64_t wpps = pps / 4;
-    const int64_t lo = (int64_t)split * pps + wave * wpps;
-    const int64_t hi = lo + wpps < NPX ? lo + wpps : NPX;
+    const int HW = H * W, NPX = B * HW;
+    const int split = blockIdx.x, ct0 = (blockIdx.y * 4 + wave) * CT;
+    const int lo = split * pps, hi = lo + pps < NPX ? lo + pps : NPX;
     const int Wc = W >> 1;
-    int cdy[CT], cdx[CT], cc[CT];
-    bool cval[CT];
+    int off[CT];        // LDS offset of this lane's column at pixel 0
+    int tdy[CT], tdx[CT];
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) {
-        const int kcol = (cg * CT + ct) * 16 + col;
-        const int tap = kcol / CIN;
-        cc[ct] = kcol - tap * CIN;
-        cval[ct] = (cg * CT + ct) < NCT && tap < 9;
-        cdy[ct] = tap / 3 - 1;
-        cdx[ct] = tap - (tap / 3) * 3 - 1;
+        const int kcol = (ct0 + ct) * 16 + col;
+        int tap = kcol / CIN;
+        const int c = kcol - tap * CIN;
+        // columns past the nine taps (KP is a multiple of 32) are not used: any valid offset
+        if (tap > 8) tap = 8;
+        tdy[ct] = tap / 3 - 1;
+        tdx[ct] = tap - (tap / 3) * 3 - 1;
+        off[ct] = ((tdy[ct] + 1) * (kWgPx + 2) + tdx[ct] + 1) * LX + c;
     }
+    auto store8 = [](bf16* p, const bf16x8& v) {        // 4-byte aligned
+        const int4 q = *reinterpret_cast<const int4*>(&v);
+        int* d = reinterpret_cast<int*>(p);
+        d[0] = q.x;
+        d[1] = q.y;
+        d[2] = q.z;
+        d[3] = q.w;
+    };
     floatx4 acc[RT][CT];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) acc[rt][ct] = floatx4{0.f, 0.f, 0.f, 0.f};
-    for (int64_t base = lo; base < hi; base += 32) {
-        const int64_t P0 = base + g * 8;
-        int b = 0, i = 0, j = 0;
-        if (P0 < NPX) {
-            b = (int)(P0 / HW);
-            const int64_t rem = P0 - (int64_t)b * HW;
-            i = (int)(rem / W);
-            j = (int)(rem - (int64_t)i * W);
+    for (int base = lo; base < hi; base += kWgPx) {
+        __syncthreads();
+        for (int u = threadIdx.x; u < NX3; u += KM_BLOCK) {
+            const int px = u / VX, vc = (u - px * VX) * 8;
+            const int row = px / (kWgPx + 2), k = px - row * (kWgPx + 2);
+            const int q = base + (row - 1) * W + k - 1;     // linear pixel, perhaps of another row: masked later
+            bf16x8 v = zero8();
+            if (q >= 0 && q < NPX) {
+                if (MODE == 0) {
+                    v = *reinterpret_cast<const bf16x8*>(src0 + (int64_t)q * C0 + vc);
+                } else if (vc < C0) {
+                    const int b = q / HW, rem = q - b * HW, i = rem / W, j = rem - i * W;
+                    v = *reinterpret_cast<const bf16x8*>(
+                        src0 + ((int64_t)b * (HW / 4) + (int64_t)(i >> 1) * Wc + (j >> 1)) * C0 + vc);
+                } else {
+                    v = *reinterpret_cast<const bf16x8*>(src1 + (int64_t)q * C1 + (vc - C0));
+                }
+            }
+            store8(xs + px * LX + vc, v);
         }
-        bf16x8 av[RT], bv[CT];
+        for (int u = threadIdx.x; u < NY1; u += KM_BLOCK) {
+            const int px = u / VY, vc = (u - px * VY) * 8;
+            bf16x8 v = zero8();
+            if (base + px < hi) v = *reinterpret_cast<const bf16x8*>(dY + (int64_t)(base + px) * COUT + vc);
+            store8(ys + px * LY + vc, v);
+        }
+        __syncthreads();
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const bool ok = P0 + e < hi;
+        for (int ch = 0; ch < kWgPx / 32; ++ch) {
+            const int p0 = ch * 32 + g * 8;     // this lane's first pixel of the chunk
+            // bit e: pixel e has a neighbour above, below, left, right
+            int up = 0, down = 0, left = 0, right = 0;
+            {
+                const int P = base + p0 < NPX ? base + p0 : NPX - 1;
+                const int rem = P % HW;
+                int i = rem / W, j = rem - i * W;
 #pragma unroll
-            for (int rt = 0; rt < RT; ++rt) av[rt][e] = ok ? dY[(P0 + e) * COUT + rt * 16 + col] : (bf16)0.0f;
+                for (int e = 0; e < 8; ++e) {
+                    up |= (i > 0) << e;
+                    down |= (i < H - 1) << e;
+                    left |= (j > 0) << e;
+                    right |= (j < W - 1) << e;
+                    if (++j == W) {
+                        j = 0;
+                        if (++i == H) i = 0;
+                    }
+                }
+            }
+            bf16x8 av[RT];
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) av[rt][e] = ys[(p0 + e) * LY + rt * 16 + col];
 #pragma unroll
             for (int ct = 0; ct < CT; ++ct) {
-                bf16 val = (bf16)0.0f;
-                const int ii = i + cdy[ct], jj = j + cdx[ct];
-                if (ok && cval[ct] && ii >= 0 && ii < H && jj >= 0 && jj < W) {
-                    const int c = cc[ct];
-                    if (MODE == 0)
-                        val = src0[(((int64_t)b * H + ii) * W + jj) * C0 + c];
-                    else if (c < C0)
-                        val = src0[((int64_t)b * (HW / 4) + (int64_t)(ii >> 1) * Wc + (jj >> 1)) * C0 + c];
-                    else
-                        val = src1[(((int64_t)b * H + ii) * W + jj) * C1 + (c - C0)];
+                if (ct0 + ct >= NCT) continue;
+                bf16x8 bv;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) bv[e] = xs[off[ct] + (p0 + e) * LX];
+                const int in = (tdy[ct] < 0 ? up : tdy[ct] > 0 ? down : 0xff) &
+                               (tdx[ct] < 0 ? left : tdx[ct] > 0 ? right : 0xff);
+                if (__any(in != 0xff)) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        if (!((in >> e) & 1)) bv[e] = (bf16)0.0f;
                 }
-                bv[ct][e] = val;
-            }
-            if (++j == W) {
-                j = 0;
-                if (++i == H) { i = 0; ++b; }
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt)
+                    acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[rt], bv, acc[rt][ct], 0, 0, 0);
             }
         }
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-            for (int ct = 0; ct < CT; ++ct)
-                if (cg * CT + ct < NCT)
-                    acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[rt], bv[ct], acc[rt][ct], 0, 0, 0);
     }
-    float* dst = part + (int64_t)(split * 4 + wave) * COUT * KP;
+    float* dst = part + (int64_t)split * COUT * KP;
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) {
-            if (cg * CT + ct >= NCT) continue;
-            const int kcol = (cg * CT + ct) * 16 + col;
+            if (ct0 + ct >= NCT) continue;
+            const int kcol = (ct0 + ct) * 16 + col;
 #pragma unroll
             for (int i = 0; i < 4; ++i) dst[(int64_t)(rt * 16 + g * 4 + i) * KP + kcol] = acc[rt][ct][i];
         }
 }
 
-__global__ void __launch_bounds__(KM_BLOCK)
+// The parts' sums in FP64: 32 weights by 32 slices of the parts per workgroup,
+// eight loads of a thread in flight, the slices added in order (one thread per
+// weight walking all parts: 310 us per layer on average, almost all of it
+// load latency).
+constexpr int kWrSlices = 32;
+__global__ void __launch_bounds__(32 * kWrSlices)
 k_wgrad_reduce(int nparts, int cout, int kp, int cin, int cin_p, const float* __restrict__ part, float* __restrict__ gw) {
+    __shared__ double sh[kWrSlices][33];
     const int64_t n = (int64_t)cout * kp;
-    for (int64_t idx = (int64_t)blockIdx.x * KM_BLOCK + threadIdx.x; idx < n; idx += (int64_t)gridDim.x * KM_BLOCK) {
-        const int co = (int)(idx / kp), kcol = (int)(idx % kp);
-        const int tap = kcol / cin_p, c = kcol % cin_p;
-        if (tap >= 9 || c >= cin) continue;
-        double s = 0.0;
-        for (int p = 0; p < nparts; ++p) s += (double)part[(int64_t)p * n + idx];
-        gw[((int64_t)co * 9 + tap) * cin + c] = (float)s;
+    const int c32 = threadIdx.x & 31, sl = threadIdx.x >> 5;
+    const int64_t idx = (int64_t)blockIdx.x * 32 + c32;     // n is a multiple of 32
+    const int per = (nparts + kWrSlices - 1) / kWrSlices;
+    const int p0 = sl * per, p1 = p0 + per < nparts ? p0 + per : nparts;
+    const float* q = part + idx;
+    double s = 0.0;
+    int p = p0;
+    for (; p + 8 <= p1; p += 8) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = q[(int64_t)(p + u) * n];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) s += (double)v[u];
     }
+    for (; p < p1; ++p) s += (double)q[(int64_t)p * n];
+    sh[sl][c32] = s;
+    __syncthreads();
+    if (sl != 0) return;
+    double a = 0.0;
+#pragma unroll
+    for (int k = 0; k < kWrSlices; ++k) a += sh[k][c32];
+    const int co = (int)(idx / kp), kcol = (int)(idx % kp);
+    const int tap = kcol / cin_p, c = kcol % cin_p;
+    if (tap >= 9 || c >= cin) return;
+    gw[((int64_t)co * 9 + tap) * cin + c] = (float)a;
 }
 
-// Per-channel sums of a (npx, C) BF16 tensor: partials P[c * G + block].
+// Per-channel sums of a (npx, C) BF16 tensor: partials P[c * G + block].  A
+// thread adds eight channels of a pixel at a time (one 16-byte load, four in
+// flight): 433 us for 128 channels with two-byte loads one after another.
 template <int C>
 __global__ void __launch_bounds__(KM_BLOCK) k_chan_sum(int64_t npx, const bf16* __restrict__ dY, double* __restrict__ P, int G) {
-    __shared__ double sh[KM_BLOCK];
-    constexpr int R = KM_BLOCK / C;
-    const int c = threadIdx.x % C, r0 = threadIdx.x / C;
+    constexpr int V = C / 8, R = KM_BLOCK / V;
+    __shared__ double sh[KM_BLOCK * 8];
+    const int vc = threadIdx.x % V, r0 = threadIdx.x / V;
     const int64_t chunk = (npx + G - 1) / G;
     const int64_t lo = (int64_t)blockIdx.x * chunk;
     const int64_t hi = lo + chunk < npx ? lo + chunk : npx;
-    double s = 0.0;
-    for (int64_t p = lo + r0; p < hi; p += R) s += (double)(float)dY[p * C + c];
-    sh[threadIdx.x] = s;
+    double s[8] = {};
+    int64_t p = lo + r0;
+    for (; p + 3 * R < hi; p += 4 * R) {
+        bf16x8 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = *reinterpret_cast<const bf16x8*>(dY + (p + u * R) * C + vc * 8);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) s[e] += (double)(float)v[u][e];
+    }
+    for (; p < hi; p += R) {
+        const bf16x8 v = *reinterpret_cast<const bf16x8*>(dY + p * C + vc * 8);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s[e] += (double)(float)v[e];
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) sh[r0 * C + vc * 8 + e] = s[e];
     __syncthreads();
     if (threadIdx.x < C) {
         double a = 0.0;
@@ -393,13 +490,14 @@ __global__ void __launch_bounds__(KM_BLOCK) k_chan_sum(int64_t npx, const bf16* 
     }
 }
 
-// out[v] = sum_g P[v * G + g] (fixed order)
-__global__ void __launch_bounds__(KM_BLOCK) k_reduce_rows(int nv, int G, const double* __restrict__ P, float* __restrict__ out) {
-    const int v = blockIdx.x * KM_BLOCK + threadIdx.x;
-    if (v >= nv) return;
+// out[v] = sum_g P[v * G + g] (fixed order): one workgroup per row
+__global__ void __launch_bounds__(KM_BLOCK) k_reduce_rows(int G, const double* __restrict__ P, float* __restrict__ out) {
+    __shared__ double sh[8];
+    const double* q = P + (int64_t)blockIdx.x * G;
     double s = 0.0;
-    for (int g = 0; g < G; ++g) s += P[(int64_t)v * G + g];
-    out[v] = (float)s;
+    for (int g = threadIdx.x; g < G; g += KM_BLOCK) s += q[g];
+    s = block_sum(s, sh);
+    if (threadIdx.x == 0) out[blockIdx.x] = (float)s;
 }
 
 // ------------------------------------------------------------ pools, splits
@@ -796,26 +894,30 @@ template <int MODE, int C0, int C1, int COUT>
 void wgrad(km_net* N, int l, int H, int W, int B, const bf16* s0, const bf16* s1, const bf16* dY, float* grad,
            hipStream_t st) {
     constexpr int CIN = C0 + C1, KP = round32(9 * CIN), NCT = KP / 16;
-    constexpr int CT = COUT >= 128 ? 4 : 8;
-    const int ncg = (NCT + CT - 1) / CT;
+    // accumulators of a wave: at most 32 tiles (128 registers)
+    constexpr int most_ct = 32 / (COUT / 16), CT = (NCT + 3) / 4 < most_ct ? (NCT + 3) / 4 : most_ct;
+    const int ncg = (NCT + 4 * CT - 1) / (4 * CT);
     const int64_t npx = (int64_t)B * H * W;
-    int64_t nsplit = (1024 + ncg - 1) / ncg;
-    const int64_t cap = kWpartMax / (4LL * COUT * KP);
+    // as many splits as keep four workgroups of each column group per compute
+    // unit and the FP32 sums short, within the partial sums' buffer
+    int64_t nsplit = (4096 + ncg - 1) / ncg;
+    const int64_t cap = kWpartMax / (COUT * KP);
     if (nsplit > cap) nsplit = cap;
-    const int64_t most = (npx + 127) / 128;
+    const int64_t most = (npx + kWgPx - 1) / kWgPx;
     if (nsplit > most) nsplit = most;
-    if (nsplit < 1) nsplit = 1;
     int64_t pps = (npx + nsplit - 1) / nsplit;
-    pps = (pps + 127) / 128 * 128;
+    pps = (pps + kWgPx - 1) / kWgPx * kWgPx;
     nsplit = (npx + pps - 1) / pps;
     hipLaunchKernelGGL((k_wgrad<MODE, C0, C1, COUT, CT>), dim3((unsigned)nsplit, (unsigned)ncg), dim3(KM_BLOCK), 0, st,
-                       H, W, B, s0, s1, dY, pps, N->wpart);
+                       H, W, B, s0, s1, dY, (int)pps, N->wpart);
     const LayerOff& L = N->lay.L[l];
-    hipLaunchKernelGGL(k_wgrad_reduce, dim3(flat_blocks((int64_t)COUT * KP)), dim3(KM_BLOCK), 0, st,
-                       (int)(nsplit * 4), COUT, KP, L.cin, L.cin_p, (const float*)N->wpart, grad + L.w);
-    const int G = (int)(npx / 4096 + 1 < 1024 ? npx / 4096 + 1 : 1024);
+    static_assert(COUT * KP % 32 == 0, "k_wgrad_reduce takes 32 weights per workgroup");
+    hipLaunchKernelGGL(k_wgrad_reduce, dim3(COUT * KP / 32), dim3(32 * kWrSlices), 0, st, (int)nsplit, COUT, KP, L.cin,
+                       L.cin_p, (const float*)N->wpart, grad + L.w);
+    const int64_t gc = npx * COUT / 32768 + 1;
+    const int G = (int)(gc < 1024 ? gc : 1024);
     hipLaunchKernelGGL(k_chan_sum<COUT>, dim3(G), dim3(KM_BLOCK), 0, st, npx, dY, N->P, G);
-    hipLaunchKernelGGL(k_reduce_rows, dim3(1), dim3(KM_BLOCK), 0, st, COUT, G, (const double*)N->P, grad + L.b);
+    hipLaunchKernelGGL(k_reduce_rows, dim3(COUT), dim3(KM_BLOCK), 0, st, G, (const double*)N->P, grad + L.b);
 }
 
 size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
@@ -1125,7 +1227,7 @@ int km_unet_loss_grad(km_ctx* ctx, const float* params, int B, int NX, int NY, c
     hipLaunchKernelGGL(k_loss_grad, dim3(Gl), dim3(KM_BLOCK), 0, s, NX, NY, H, W, B, coef, 5 * n, (const float*)N->q,
                        corr ? (const float*)N->ae : nullptr, (const double*)N->stats, (const bf16*)N->d0,
                        params + N->lay.out_w, N->dy_d0, N->P, Gl);
-    hipLaunchKernelGGL(k_reduce_rows, dim3(1), dim3(KM_BLOCK), 0, s, 17, Gl, (const double*)N->P, grad + N->lay.out_w);
+    hipLaunchKernelGGL(k_reduce_rows, dim3(17), dim3(KM_BLOCK), 0, s, Gl, (const double*)N->P, grad + N->lay.out_w);
     backward(N, B, grad, s);
     KM_CHECK_LAUNCH(ctx);
     if (loss) {
