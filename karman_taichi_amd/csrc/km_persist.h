@@ -29,6 +29,19 @@ int smooth(km_ctx* ctx, int nsys, const int* NX, const int* NY, const T* const* 
            T* const* xd, T* const* ws, double eps, const int* max_iter, int sweeps, KState* out,
            const std::function<int()>* tail, bool* ran);
 
+// What orders these launches on one device; created with the first context there.
+int gate(int device);
+
+// Plain BiCGSTAB, or CG, of a system whose first residual is rin (from_x: x
+// holds x0, else x = 0 and rin = b), relative to ref = ||b||^2 (0: to ||rin||^2),
+// as bicgstab_typed / cg_typed of km_krylov.hip.  ws: 2 n values.  words: null,
+// or plain_words_bytes() of the caller's for the exchange.
+bool fits_plain(km_ctx* ctx, int NX, int NY, int* shape);
+size_t plain_words_bytes();
+int plain(km_ctx* ctx, int shape, bool cg, int NX, int NY, const double* coef, const double* rin, double* x, bool from_x,
+          double* ws, void* words, double eps, int max_iter, double ref, KState* out, const std::function<int()>* tail,
+          bool* ran);
+
 }  // namespace kmpersist
 
 void km_persist_free(km_ctx* ctx);

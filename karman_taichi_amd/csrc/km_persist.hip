@@ -42,6 +42,7 @@
 #include <algorithm>
 #include <mutex>
 #include <type_traits>
+#include <vector>
 
 // Per-context exchange buffers (allocated at the first such solve).
 struct km_persist {
@@ -794,8 +795,283 @@ __global__ void __launch_bounds__(NT) k_solve2(PSys<T> a, PSys<T> b) {
     solve_body<T, CT, TI, TJ, NT, SW, false>(s, xcd_remap(first ? blockIdx.x : blockIdx.x - a.G, s.G));
 }
 
+// ------------------------------------------------------------ plain solves
+//
+// The reference's BiCGSTAB (bicgsolver.py:88-136) and CG (cgsolver.py:83-114) of
+// a whole system in one launch, with the scalars, order of tests and
+// recurrences of km_krylov.hip.  A thread holds coefficients and vectors of
+// its tile's cells in registers; the stencil's input lies in LDS with a one-cell
+// halo, whose cells (at most one per thread) advance like the tile's.  An
+// iteration is two or three rounds (one per reduction).  A system of one tile
+// needs none: 16 us per iteration by launches at 34 x 34 cells is three
+// launches' latency, whatever they do.
+struct PPlain {
+    int NX, NY, tiles_j, G;
+    const double* c;
+    const double* rin;    // the first residual: b, or b - A x0
+    double* x;
+    int from_x;           // 1: x holds x0
+    double* v;            // edge cells of v (A p), t
+    double* t;
+    unsigned* flags;
+    unsigned* abort;
+    unsigned round;
+    double* part[3];      // partial sums of the rounds in turn
+    double eps, ref;      // ref > 0: the stopping test's denominator
+    int max_iter;
+    int* hw;
+};
+
+constexpr int kNumPlain = 5;
+constexpr int kPlainOne = 2;     // shapes that a whole system may fill alone
+constexpr int kPTI[kNumPlain] = {16, 32, 40, 48, 64};
+constexpr int kPTJ[kNumPlain] = {16, 32, 32, 48, 64};
+constexpr int kPNT[kNumPlain] = {256, 512, 640, 768, 1024};
+
+template <int TI, int TJ, int NT, bool CG>
+__global__ void __launch_bounds__(NT) k_plain(PPlain s) {
+    constexpr int W = TJ + 2, Q = (TI * TJ + NT - 1) / NT, NW = NT / 64;
+    constexpr int RING = 2 * (TI + TJ);
+    static_assert(RING <= NT && NT >= kMaxWg, "one halo cell per thread, one flag per thread");
+    __shared__ double z[(TI + 2) * W];
+    __shared__ double red[2][2][NW], red2[2 * 4];   // two buffers: a sum's reads may overlap the next one's writes
+    __shared__ int bad;
+    const int t = threadIdx.x;
+    const int L = xcd_remap(blockIdx.x, s.G), G = s.G;
+    const int NX = s.NX, NY = s.NY, nx = NX - 2, ny = NY - 2;
+    const int64_t n = (int64_t)NX * NY;
+    const int ta = L / s.tiles_j, tb = L - ta * s.tiles_j;
+    const int ti0 = 1 + ta * TI, tj0 = 1 + tb * TJ;
+    unsigned round = s.round;
+    if (t == 0) bad = 0;
+    for (int k = t; k < (TI + 2) * W; k += NT) z[k] = 0.0;
+    // boundary rows must be empty (see solve_body)
+    const int j0 = tb == 0 ? 0 : tj0, j1 = tj0 + TJ > ny ? NY : tj0 + TJ;
+    const int i0 = ta == 0 ? 0 : ti0, i1 = ti0 + TI > nx ? NX : ti0 + TI;
+    auto boundary = [&](auto f) {
+        if (ta == 0)
+            for (int j = j0 + t; j < j1; j += NT) f((int64_t)j);
+        if (ti0 + TI > nx)
+            for (int j = j0 + t; j < j1; j += NT) f((int64_t)(NX - 1) * NY + j);
+        if (tb == 0)
+            for (int i = i0 + t; i < i1; i += NT) f((int64_t)i * NY);
+        if (tj0 + TJ > ny)
+            for (int i = i0 + t; i < i1; i += NT) f((int64_t)i * NY + NY - 1);
+    };
+    double odd = 0.0;
+    boundary([&](int64_t k) {
+        bool any = s.rin[k] != 0.0;
+        for (int e = 0; e < 5; ++e) any = any || s.c[e * n + k] != 0.0;
+        if (any) odd += 1.0;
+    });
+    double c[Q][5], r[Q], rt[Q], p[Q], v[Q], x[Q];
+    int kq[Q], lz[Q];
+    uint32_t own = 0, edge = 0;
+    double rr = 0.0;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        const int u = t + q * NT, a = u / TJ, b = u - a * TJ;
+        const int i = ti0 + a, j = tj0 + b;
+        const bool in = u < TI * TJ && i <= nx && j <= ny;
+        kq[q] = in ? i * NY + j : 0;
+        lz[q] = u < TI * TJ ? (a + 1) * W + b + 1 : 0;
+        if (in) own |= 1u << q;
+        if (in && (a == 0 || a == TI - 1 || b == 0 || b == TJ - 1)) edge |= 1u << q;
+#pragma unroll
+        for (int e = 0; e < 5; ++e) c[q][e] = in ? s.c[e * n + kq[q]] : 0.0;
+        r[q] = in ? s.rin[kq[q]] : 0.0;
+        x[q] = in && s.from_x ? s.x[kq[q]] : 0.0;
+        rt[q] = r[q];
+        p[q] = 0.0;
+        v[q] = 0.0;
+        rr += r[q] * r[q];
+    }
+    // the halo cell of this thread
+    int hk = -1, hz = 0;
+    if (t < RING) {
+        const int a = t < TJ ? -1 : t < 2 * TJ ? TI : (t - 2 * TJ) % TI;
+        const int b = t < TJ ? t : t < 2 * TJ ? t - TJ : t < 2 * TJ + TI ? -1 : TJ;
+        const int i = ti0 + a, j = tj0 + b;
+        if (i >= 1 && i <= nx && j >= 1 && j <= ny) hk = i * NY + j;
+        hz = (a + 1) * W + b + 1;
+    }
+    double hr = hk >= 0 ? s.rin[hk] : 0.0, hp = 0.0, hv = 0.0;
+    // everyone's totals of (a, b): false when the launch gave up
+    double T0 = 0.0, T1 = 0.0;
+    int buf = 0;
+    auto sum = [&](double a, double b, double* P) {
+        const int lane = t & 63, w = t >> 6;
+        const double sa = wave_sum(a), sb = wave_sum(b);
+        buf ^= 1;
+        if (lane == 0) {
+            red[buf][0][w] = sa;
+            red[buf][1][w] = sb;
+        }
+        __syncthreads();
+        // pairwise, all loads first
+        auto waves = [&](const double* q) {
+            double y[NW];
+#pragma unroll
+            for (int k = 0; k < NW; ++k) y[k] = q[k];
+#pragma unroll
+            for (int d = 1; d < NW; d *= 2)
+#pragma unroll
+                for (int k = 0; k + d < NW; k += 2 * d) y[k] += y[k + d];
+            return y[0];
+        };
+        if (G == 1) {
+            T0 = waves(red[buf][0]);
+            T1 = waves(red[buf][1]);
+            return true;
+        }
+        if (t < 2) put(P + 2 * L + t, waves(red[buf][t]));
+        return meet<NT>(s.flags, L, G, ++round, s.abort, &bad);
+    };
+    // the totals after a round (G > 1), with this thread's halo value of h
+    auto total = [&](const double* P, const double* h, double* out) {
+        if (G == 1) return;
+        double mine[2] = {0.0, 0.0};
+        if (t < G) {
+            mine[0] = get_at(P, 2 * t);
+            mine[1] = get_at(P, 2 * t + 1);
+        }
+        if (h && hk >= 0) *out = get_at(h, hk);
+        double y[2];
+        totals<2, NT>(mine, G, y, red2);
+        T0 = y[0];
+        T1 = y[1];
+    };
+    auto apply = [&](int q) {
+        const int k = lz[q];
+        double y = c[q][0] * z[k];
+        y += c[q][1] * z[k - W];
+        y += c[q][2] * z[k + W];
+        y += c[q][3] * z[k + 1];
+        y += c[q][4] * z[k - 1];
+        return y;
+    };
+    int it = 0, status = -1;
+    double r0 = 0.0, rho = 0.0, rho0 = 1.0, alpha = 0.0, omega = 0.0, rTr = 0.0;
+    // <r,r> (and <r,r~>, the same at the start); the count of odd boundary cells first
+    bool ok = sum(odd, 0.0, s.part[1]);
+    if (ok) total(s.part[1], nullptr, nullptr);
+    if (!ok) status = kAborted;
+    else if (T0 != 0.0) status = kUnsupported;
+    if (status < 0) {
+        ok = sum(rr, rr, s.part[2]);
+        if (ok) total(s.part[2], nullptr, nullptr);
+        else status = kAborted;
+    }
+    while (status < 0) {
+        rTr = T0;
+        rho = CG ? T0 : T1;
+        if (it == 0) r0 = s.ref > 0.0 ? s.ref : rTr;
+        if (!fin(rTr)) status = KM_NONFINITE;
+        else if (it == 0 && rTr == 0.0) status = KM_OK;
+        else if (it > 0 && (CG ? sqrt(rTr) < sqrt(r0) * s.eps : sqrt(rTr / r0) < s.eps)) status = KM_OK;   // bicgsolver.py:130, cgsolver.py:240
+        else if (!CG && it > 0 && omega == 0.0) status = KM_BREAKDOWN;
+        else if (it >= s.max_iter) status = KM_MAXITER;
+        else if (!CG && !fin(rho)) status = KM_NONFINITE;
+        else if (!CG && rho == 0.0) status = KM_BREAKDOWN;                                     // bicgsolver.py:96-98
+        if (status >= 0) break;
+        const double beta = it == 0 ? 0.0 : CG ? rho / rho0 : (rho / rho0) * (alpha / omega);   // :102, cgsolver.py:245
+        const double om = it == 0 ? 0.0 : omega;
+        rho0 = rho;
+        // p = r + beta (p - omega v) (bicgsolver.py:43-46; CG: r + beta p)
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            p[q] = r[q] + beta * (CG ? p[q] : p[q] - om * v[q]);
+            if ((own >> q) & 1u) z[lz[q]] = p[q];
+        }
+        hp = hr + beta * (CG ? hp : hp - om * hv);
+        if (hk >= 0) z[hz] = hp;
+        __syncthreads();
+        double d0 = 0.0, d1 = 0.0;
+#pragma unroll
+        for (int q = 0; q < Q; ++q)
+            if ((own >> q) & 1u) {
+                v[q] = apply(q);
+                if (G > 1 && ((edge >> q) & 1u)) put(s.v + kq[q], v[q]);
+                d0 += (CG ? p[q] : rt[q]) * v[q];
+            }
+        if (!sum(d0, 0.0, s.part[0])) { status = kAborted; break; }
+        if (G > 1) total(s.part[0], s.v, &hv);
+        if (!fin(T0)) status = KM_NONFINITE;
+        else if (T0 == 0.0) status = KM_BREAKDOWN;
+        if (status >= 0) break;
+        alpha = rho / T0;                                     // bicgsolver.py:108, cgsolver.py:234
+        if (CG) {
+            rr = 0.0;
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                x[q] = x[q] + alpha * p[q];                   // cgsolver.py:206-209
+                r[q] = r[q] - alpha * v[q];                   // cgsolver.py:211-214
+                rr += r[q] * r[q];
+            }
+            if (G == 1) hv = 0.0;
+            hr = hr - alpha * hv;
+            d0 = d1 = rr;
+        } else {
+            // s = r - alpha v (bicgsolver.py:60-63)
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                r[q] = r[q] - alpha * v[q];
+                if ((own >> q) & 1u) z[lz[q]] = r[q];
+            }
+            hr = hr - alpha * hv;
+            if (hk >= 0) z[hz] = hr;
+            __syncthreads();
+            double th = 0.0, tq[Q];
+            d0 = d1 = 0.0;
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                tq[q] = 0.0;
+                if ((own >> q) & 1u) {
+                    tq[q] = apply(q);
+                    if (G > 1 && ((edge >> q) & 1u)) put(s.t + kq[q], tq[q]);
+                    d0 += tq[q] * r[q];                       // <t,s>, <t,t> (:116-117)
+                    d1 += tq[q] * tq[q];
+                }
+            }
+            if (!sum(d0, d1, s.part[1])) { status = kAborted; break; }
+            if (G > 1) total(s.part[1], s.t, &th);
+            omega = T1 != 0.0 ? T0 / T1 : 0.0;                // bicgsolver.py:118
+            d0 = d1 = 0.0;
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                x[q] = x[q] + (alpha * p[q] + omega * r[q]);  // bicgsolver.py:78-81
+                r[q] = r[q] - omega * tq[q];                  // :83-86
+                d0 += r[q] * r[q];
+                d1 += r[q] * rt[q];
+            }
+            hr = hr - omega * th;
+        }
+        if (!sum(d0, d1, s.part[2])) { status = kAborted; break; }
+        if (G > 1) total(s.part[2], nullptr, nullptr);
+        ++it;
+    }
+    if (status < kUnsupported) {
+#pragma unroll
+        for (int q = 0; q < Q; ++q)
+            if ((own >> q) & 1u) s.x[kq[q]] = x[q];
+        if (!s.from_x) boundary([&](int64_t k) { s.x[k] = 0.0; });
+    }
+    if (t == 0 && (L == 0 || status == kAborted)) {
+        if (L == 0) {
+            __hip_atomic_store(s.hw + 1, it, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            __hip_atomic_store(s.hw + 2, status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            __hip_atomic_store(reinterpret_cast<double*>(s.hw + 4), r0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            __hip_atomic_store(reinterpret_cast<double*>(s.hw + 6), rTr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+        if (status == kAborted) __hip_atomic_store(s.hw + 3, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (L == 0) __hip_atomic_store(s.hw, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
 // Launches of one device in one process follow each other: two of them side
-// by side could each hold compute units the other waits for.
+// by side could each hold compute units the other waits for.  (Letting those run
+// together whose workgroups fit the device at once gained 2% on 12 cases of 13k
+// to 210k cells on three streams, which is within its spread.)
 struct Gate {
     std::mutex m;
     hipEvent_t last = nullptr;
@@ -804,6 +1080,19 @@ struct Gate {
 };
 constexpr int kMaxDevices = 64;
 Gate g_gate[kMaxDevices];
+
+int admit(km_ctx* ctx, const std::function<void()>& launch) {
+    Gate& g = g_gate[ctx->device];
+    std::lock_guard<std::mutex> lk(g.m);
+    KM_REQUIRE(ctx, g.last, "device %d has no launch gate", ctx->device);
+    if (g.any && g.stream != ctx->stream) KM_HIP(ctx, hipStreamWaitEvent(ctx->stream, g.last, 0));
+    launch();
+    KM_CHECK_LAUNCH(ctx);
+    KM_HIP(ctx, hipEventRecord(g.last, ctx->stream));
+    g.any = true;
+    g.stream = ctx->stream;
+    return KM_OK;
+}
 
 int tiles_of(int n, int T) { return (n + T - 1) / T; }
 
@@ -910,23 +1199,12 @@ PSys<T> system(km_ctx* ctx, int slot, int shape, int NX, int NY, const void* c, 
 
 // Launch, the tail, and the final states; *ran = false if it gave up.
 int finish(km_ctx* ctx, int nsys, const std::function<void()>& launch, KState* out, const std::function<int()>* tail,
-           bool* ran) {
-    km_persist* K = ctx->persist;
+           bool* ran, km_persist* K, int rounds) {
     volatile int* hf = ctx->h_flag;
     for (int q = 0; q < nsys; ++q)
         for (int k = 0; k < 4; ++k) hf[KM_HW * q + k] = 0;
     std::atomic_thread_fence(std::memory_order_seq_cst);
-    {
-        Gate& g = g_gate[ctx->device];
-        std::lock_guard<std::mutex> lk(g.m);
-        if (!g.last) KM_HIP_SYNC(ctx, hipEventCreateWithFlags(&g.last, hipEventDisableTiming));
-        if (g.any && g.stream != ctx->stream) KM_HIP(ctx, hipStreamWaitEvent(ctx->stream, g.last, 0));
-        launch();
-        KM_CHECK_LAUNCH(ctx);
-        KM_HIP(ctx, hipEventRecord(g.last, ctx->stream));
-        g.any = true;
-        g.stream = ctx->stream;
-    }
+    if (int rc = admit(ctx, launch)) return rc;
     if (tail)
         if (int rc = (*tail)()) return rc;
     KM_HIP_SYNC(ctx, hipStreamSynchronize(ctx->stream));
@@ -948,13 +1226,15 @@ int finish(km_ctx* ctx, int nsys, const std::function<void()>& launch, KState* o
     }
     if (aborted) {
         *ran = false;
-        K->off++;
+        if (K) K->off++;
         return KM_OK;
     }
     int most = 0;
     for (int q = 0; q < nsys; ++q) most = std::max(most, out[q].iter);
-    K->round += 2 * (unsigned)most + 8;
-    K->clean = true;
+    if (K) {
+        K->round += (unsigned)rounds * (unsigned)most + 8;
+        K->clean = true;
+    }
     return KM_OK;
 }
 
@@ -1036,7 +1316,7 @@ int twolevel(km_ctx* ctx, int shape, int NX, int NY, const double* coef, const T
 #undef KM_CASE
         }
     };
-    return finish(ctx, 1, launch, out, tail, ran);
+    return finish(ctx, 1, launch, out, tail, ran, K, 2);
 }
 
 template <typename T>
@@ -1074,7 +1354,86 @@ int smooth(km_ctx* ctx, int nsys, const int* NX, const int* NY, const T* const* 
             for (int q = 0; q < nsys; ++q) one(shape[q], s[q], none);
         }
     };
-    return finish(ctx, nsys, launch, out, tail, ran);
+    return finish(ctx, nsys, launch, out, tail, ran, ctx->persist, 2);
+}
+
+int gate(int device) {
+    if (device < 0 || device >= kMaxDevices) return KM_OK;   // no path on that device (fits_*)
+    Gate& g = g_gate[device];
+    std::lock_guard<std::mutex> lk(g.m);
+    if (!g.last && hipEventCreateWithFlags(&g.last, hipEventDisableTiming) != hipSuccess) return KM_EHIP;
+    return KM_OK;
+}
+
+// One workgroup where the system fits one (no exchange: 2-3 us per iteration
+// against 16 by launches), else the smallest tiles that number at most one per
+// compute unit.  A tile chosen by km_set_tile asks for the launches.
+bool fits_plain(km_ctx* ctx, int NX, int NY, int* shape) {
+    if ((ctx->persist && ctx->persist->off >= 2) || NX < 3 || NY < 3 ||
+        ctx->tile_override.count(std::make_tuple(NX, NY, KM_F64)))
+        return false;
+    const int cus = std::min(kMaxWg, compute_units(ctx));
+    for (int one = 1; one >= 0; --one)
+        for (int k = 0; k < (one ? kPlainOne : kNumPlain); ++k) {
+            const int64_t G = (int64_t)tiles_of(NX - 2, kPTI[k]) * tiles_of(NY - 2, kPTJ[k]);
+            if (G > (one ? 1 : cus)) continue;
+            *shape = k;
+            return true;
+        }
+    return false;
+}
+
+size_t plain_words_bytes() { return kFlagBytes + 256 + (size_t)3 * kMaxWg * 2 * sizeof(double); }
+
+int plain(km_ctx* ctx, int shape, bool cg, int NX, int NY, const double* coef, const double* rin, double* x, bool from_x,
+          double* ws, void* words, double eps, int max_iter, double ref, KState* out, const std::function<int()>* tail,
+          bool* ran) {
+    km_persist* K = nullptr;
+    PPlain s{};
+    if (words) {
+        // the caller's memory: flags from zero
+        char* w = static_cast<char*>(words);
+        KM_HIP(ctx, hipMemsetAsync(w, 0, kFlagBytes + 256, ctx->stream));
+        s.flags = reinterpret_cast<unsigned*>(w);
+        s.abort = reinterpret_cast<unsigned*>(w + kFlagBytes);
+        for (int k = 0; k < 3; ++k)
+            s.part[k] = reinterpret_cast<double*>(w + kFlagBytes + 256) + (size_t)k * kMaxWg * 2;
+    } else {
+        if (int rc = ensure(ctx)) return rc;
+        K = ctx->persist;
+        s.flags = K->flags;
+        s.abort = K->abort;
+        s.round = K->round;
+        for (int k = 0; k < 3; ++k) s.part[k] = K->part + (size_t)k * kMaxWg * 2;
+    }
+    s.NX = NX;
+    s.NY = NY;
+    s.tiles_j = tiles_of(NY - 2, kPTJ[shape]);
+    s.G = tiles_of(NX - 2, kPTI[shape]) * s.tiles_j;
+    s.c = coef;
+    s.rin = rin;
+    s.x = x;
+    s.from_x = from_x ? 1 : 0;
+    s.v = ws;
+    s.t = ws + (size_t)NX * NY;
+    s.eps = eps;
+    s.ref = ref;
+    s.max_iter = max_iter;
+    s.hw = ctx->d_flag;
+    auto launch = [&]() {
+        switch (shape * 2 + (cg ? 1 : 0)) {
+#define KM_CASE(I)                                                                                                 \
+    case 2 * I:                                                                                                    \
+        hipLaunchKernelGGL((k_plain<kPTI[I], kPTJ[I], kPNT[I], false>), dim3(s.G), dim3(kPNT[I]), 0, ctx->stream, s); \
+        break;                                                                                                     \
+    case 2 * I + 1:                                                                                                \
+        hipLaunchKernelGGL((k_plain<kPTI[I], kPTJ[I], kPNT[I], true>), dim3(s.G), dim3(kPNT[I]), 0, ctx->stream, s); \
+        break;
+            KM_CASE(0) KM_CASE(1) KM_CASE(2) KM_CASE(3) KM_CASE(4)
+#undef KM_CASE
+        }
+    };
+    return finish(ctx, 1, launch, out, tail, ran, K, 3);
 }
 
 template int twolevel<double>(km_ctx*, int, int, int, const double*, const double*, double*, double*, double, int,

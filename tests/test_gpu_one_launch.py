@@ -84,3 +84,37 @@ def test_coupled_boundary_rows_take_the_launches(dev):
     coef[0, 0, 5], b[0, 5] = 2.0, 1.0
     x, info = solve(dev, coef, b, _lib.KM_FLAG_SMOOTH)
     check(x, info, coef, b)
+
+
+# one tile of 16 x 16 and of 32 x 32 (a single workgroup), one cell more,
+# remainders, and 256 tiles of the first shape and one cell more
+PLAIN = [(5, 4), (18, 18), (19, 18), (34, 34), (35, 34), (50, 71), (258, 258), (259, 260)]
+
+
+@pytest.mark.parametrize("NX,NY", PLAIN)
+@pytest.mark.parametrize("entry", ["km_bicgstab", "km_cg", "km_bicgstab_noalloc", "from_x"])
+def test_plain_one_launch_matches_direct_solution(NX, NY, entry, dev):
+    """The plain solves stop on the recursive residual, so the true one may
+    end a little above eps: ten times, as in the parity tests."""
+    coef, b = system(NX, NY, NX * NY, 0.01)
+    c, bt = torch.tensor(coef, device=dev), torch.tensor(b, device=dev)
+    x = torch.full_like(bt, 7.0)
+    flags = 0
+    if entry == "from_x":
+        entry, flags = "km_bicgstab", _lib.KM_FLAG_X0 | _lib.KM_FLAG_TRUE
+        x[:] = 0.0
+        x[1:-1, 1:-1] = torch.tensor(np.random.default_rng(1).standard_normal((NX - 2, NY - 2)), device=dev)
+    info = KmSolveInfo()
+    ctx = _lib.Context(torch.cuda.current_device(), torch.cuda.current_stream(dev).cuda_stream)
+    try:
+        ctx.call(entry, NX, NY, ctypes.c_void_p(c.data_ptr()), ctypes.c_void_p(bt.data_ptr()),
+                 ctypes.c_void_p(x.data_ptr()), EPS, 0, flags, ctypes.byref(info))
+        torch.cuda.synchronize()
+    finally:
+        ctx.close()
+    xd = krylov.direct_solve(coef, b)
+    err = np.linalg.norm(x.cpu().numpy() - xd) / np.linalg.norm(xd)
+    print(f"{entry} {b.shape}: {info.iterations} it, true residual {info.rel_resid_true:.1e}, error {err:.1e}")
+    assert info.status == _lib.KM_OK
+    assert info.rel_resid_true < 10 * EPS
+    assert err <= 1e5 * EPS
