@@ -4,7 +4,8 @@
 //
 // What bounds it.  The launch-per-stage iteration of km_twolevel.hip costs the
 // latency of four launches (three for the momentum systems), 45-50 us per
-// iteration at 1282 x 258 cells, however few bytes it moves.  Here one
+// iteration at 1282 x 258 cells (22 us here; 13 us at 320 x 64), however few
+// bytes it moves.  Here one
 // workgroup per tile stays on its compute unit for the whole solve: the five
 // coefficients, r, p and v of the tile and its halo and x, r~ of the tile live
 // in registers, z in LDS, and only what other workgroups need goes through
@@ -42,7 +43,6 @@
 #include <algorithm>
 #include <mutex>
 #include <type_traits>
-#include <vector>
 
 // Per-context exchange buffers (allocated at the first such solve).
 struct km_persist {
@@ -75,10 +75,37 @@ constexpr int kAborted = 101;
 // first: a solve takes the first shape whose tiles number at most one per
 // compute unit.  Threads: as many as the register frame (tile plus halo 4) has
 // pairs of cells, or half or a third of them.
-constexpr int kNumShapes = 6;
-constexpr int kTI[kNumShapes] = {16, 16, 32, 40, 48, 48};
-constexpr int kTJ[kNumShapes] = {16, 32, 32, 32, 32, 48};
-constexpr int kNT[kNumShapes] = {320, 512, 512, 512, 512, 512};
+constexpr int kNumShapes = 7;
+constexpr int kTI[kNumShapes] = {16, 16, 32, 40, 48, 48, 64};
+constexpr int kTJ[kNumShapes] = {16, 32, 32, 32, 32, 48, 56};
+constexpr int kNT[kNumShapes] = {320, 512, 512, 512, 512, 512, 512};
+
+// What of a tile's own cells lies where (vectors of size vec): v and t of the
+// slots that hold own cells only in LDS beside z and the restriction's y; then,
+// as long as the LDS lasts (keeping 20 KB for the restricted vector and the
+// tables), r~, x, and p^ until x takes it.  What does not fit: t takes y's
+// place in yb (and the free-cell mask a byte per cell), x stays in memory (the
+// die's L2: 5 us per iteration at 64 x 56 cells), and without p^ x takes
+// alpha p^ while z still is p^.  r~ always fits: read from memory it cost 5 us
+// per half-iteration.
+struct Plan {
+    bool t_in_yb, x_in_lds, p_in_lds;
+    size_t bytes;
+};
+__host__ __device__ constexpr Plan plan(int TI, int TJ, int NT, int sweeps, bool coarse, size_t vec) {
+    const size_t h = 2 * (2 * sweeps + 1), QI = (TI * TJ / 2 + NT - 1) / NT, QF = TI * TJ / 2 / NT;
+    const size_t own = 2 * QI * NT * vec, full = 2 * QF * NT * vec;
+    const size_t room = 160 * 1024 - (coarse ? 20 : 4) * 1024;
+    Plan p{};
+    p.bytes = (TI + h) * (TJ + h) * vec + (coarse ? (size_t)TI * TJ * 8 : 0) + full + own;
+    p.t_in_yb = coarse && vec == 8 && p.bytes + full > room;
+    p.bytes += p.t_in_yb ? (size_t)TI * TJ : full;
+    p.x_in_lds = p.bytes + own <= room;
+    if (p.x_in_lds) p.bytes += own;
+    p.p_in_lds = p.x_in_lds && p.bytes + own <= room;
+    if (p.p_in_lds) p.bytes += own;
+    return p;
+}
 
 template <typename T>
 struct PSys {
@@ -132,6 +159,11 @@ __device__ __forceinline__ V get(const V* p) {
 template <typename V>
 __device__ __forceinline__ V get_at(const V* base, int k) {
     return get(reinterpret_cast<const V*>(reinterpret_cast<const char*>(base) + (uint32_t)k * (uint32_t)sizeof(V)));
+}
+
+template <typename V>
+__device__ __forceinline__ void put_at(V* base, int k, V v) {
+    put(reinterpret_cast<V*>(reinterpret_cast<char*>(base) + (uint32_t)k * (uint32_t)sizeof(V)), v);
 }
 
 // One round: false when the wait ran into its limit here or elsewhere.
@@ -214,6 +246,15 @@ struct LdsRow {
     }
 };
 
+// v, as a value the compiler knows nothing about: what is computed from it in
+// the iteration is computed there, not kept in a register over all of it (the
+// predicates and addresses so kept cost 90 registers, and spills from 32 x 32
+// cells on).
+__device__ __forceinline__ int fresh(int v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
 // SW red-black sweeps (halo NS = 2 SW); COARSE: the two-level preconditioner.
 // CT: coefficient and arithmetic type (FP64 for the two-level solve of FP32
 // vectors, see k_tl_tile's C64).
@@ -228,6 +269,8 @@ __device__ __forceinline__ void solve_body(const PSys<T>& s, int L) {
     constexpr int BAND = NS * (WR / 2);
     constexpr int QZ = (HZ * WZ + NT - 1) / NT;
     constexpr int NW = NT / 64;
+    constexpr int QF = NPI / NT;     // slots that hold own cells only: their v and t lie in LDS
+    constexpr Plan PL = plan(TI, TJ, NT, SW, COARSE, sizeof(T));
     static_assert(TJ % 2 == 0 && TI >= NS && TJ >= NS && NT % 64 == 0 && NT >= kMaxWg, "tile");
     extern __shared__ double dyn[];            // COARSE: m restricted values, then the cached rows of A_c^-1
     __shared__ T za[HZ * WZ];
@@ -240,7 +283,9 @@ __device__ __forceinline__ void solve_body(const PSys<T>& s, int L) {
     __shared__ double red[4 * (NW > 4 ? NW : 4)];
     __shared__ double red2[4 * 4];
     // x, r~ and p^ of the own cells: each thread reads back what it wrote
-    __shared__ T xs[2 * QI * NT], rts[2 * QI * NT], hps[2 * QI * NT];
+    __shared__ T xs[PL.x_in_lds ? 2 * QI * NT : 1], rts[2 * QI * NT], hps[PL.p_in_lds ? 2 * QI * NT : 1];
+    __shared__ T vs[QF ? 2 * QF * NT : 1], ts[QF && !PL.t_in_yb ? 2 * QF * NT : 1];
+    __shared__ uint8_t mk[PL.t_in_yb ? TI * TJ : 1];   // free own cells
     __shared__ int bad;
 
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
@@ -278,10 +323,15 @@ __device__ __forceinline__ void solve_body(const PSys<T>& s, int L) {
 
     // the frame: pair slots as k_tl_tile's, the tile's own block first
     CT cr[Q][2][5], wd[Q][2];
-    T r[Q][2], p[Q][2], v[Q][2];
+    T r[Q][2], p[Q][2], v[Q - QF][2];
     int kq[Q][2];
+    auto rtv = [&](int q, int cc) { return rts[(2 * q + cc) * NT + t]; };   // r~ of an own cell
     short dq[Q][2], pz[Q][2];   // distance outside the tile (99: not in the system), z index
     uint32_t own = 0, edge = 0, fm = 0;   // bit 2 q + c: own cell; read by a neighbour; free cell
+    auto yb_at = [&](int q, int cc) {        // place of a pair cell of the tile's own block in yb
+        const int P = fresh(t) + q * NT, lr = P / (TJ / 2);
+        return lr * TJ + pz[q][cc] - (lr + NS + 1) * WZ - (NS + 1);
+    };
     const int par0 = (ti0 + tj0) & 1;
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
@@ -337,14 +387,18 @@ __device__ __forceinline__ void solve_body(const PSys<T>& s, int L) {
             if (!in) r[q][cc] = T(0);
             wd[q][cc] = cr[q][cc][0] != CT(0) ? om * recip(cr[q][cc][0]) : CT(0);
             p[q][cc] = r[q][cc];
-            v[q][cc] = T(0);
+            if (q >= QF) v[q >= QF ? q - QF : 0][cc] = T(0);
+            else vs[(2 * q + cc) * NT + t] = T(0);
             if (q < QI) {
                 const bool o = (own >> (2 * q + cc)) & 1u;
                 const T b = o ? r[q][cc] : T(0);
-                xs[(2 * q + cc) * NT + t] = T(0);
                 rts[(2 * q + cc) * NT + t] = b;
+                if constexpr (PL.x_in_lds) xs[(2 * q + cc) * NT + t] = T(0);
+                else if (o) s.x[kq[q][cc]] = T(0);
                 rr += (double)b * (double)b;
                 if (COARSE && o && s.mask[kq[q][cc]]) fm |= 1u << (2 * q + cc);
+                if constexpr (PL.t_in_yb)
+                    if (t + q * NT < NPI) mk[yb_at(q, cc)] = (fm >> (2 * q + cc)) & 1u;
             }
         }
     // z frame: which cells take a coarse value, and from which aggregate
@@ -429,7 +483,7 @@ __device__ __forceinline__ void solve_body(const PSys<T>& s, int L) {
             int ec = lane - er * q.wdt, at = q.at + er * TJ + ec;
             double acc = 0.0;
             for (int e = lane; e < q.cnt; e += 64) {
-                acc += yb[at];
+                acc += PL.t_in_yb && !mk[PL.t_in_yb ? at : 0] ? 0.0 : yb[at];
                 ec += q.dc;
                 at += q.dr * TJ + q.dc;
                 if (ec >= q.wdt) {
@@ -450,10 +504,11 @@ __device__ __forceinline__ void solve_body(const PSys<T>& s, int L) {
     // iteration costs more than to share them (1280 x 256: 4 us and as much again
     // waiting for the workgroups with more rows, against 3 us), so each
     // workgroup computes R rows and shares them (R > 0).
-    // rows [f1, f2), row f at at(f)[k], NR rows per wave and U loads of each at a time
-    auto some_rows = [&](auto NRc, auto Uc, int f1, int f2, auto at, auto g) {
+    // rows [f1, f2), row f at at(f)[k], from wave w0 = 0 on, NR rows per wave and U
+    // loads of each at a time
+    auto some_rows = [&](auto NRc, auto Uc, int w0, int f1, int f2, auto at, auto g) {
         constexpr int NR = decltype(NRc)::value, U = decltype(Uc)::value;
-        for (int f0 = f1 + w; f0 < f2; f0 += NR * NW) {
+        for (int f0 = f1 + w0; f0 < f2; f0 += NR * NW) {
             decltype(at(0)) a[NR];
             double acc[NR];
 #pragma unroll
@@ -491,27 +546,30 @@ __device__ __forceinline__ void solve_body(const PSys<T>& s, int L) {
         using std::integral_constant;
         const auto mem = [&](int f) -> const double* { return s.inv + (int64_t)unknown(f) * s.m; };
         const auto lds = [&](int f) { return LdsRow{(f + 1) * s.m}; };
-        if (nc < nF) some_rows(integral_constant<int, 1>(), integral_constant<int, 8>(), nc, nF, mem, g);
-        if (nc <= NW) some_rows(integral_constant<int, 1>(), integral_constant<int, 8>(), 0, nc, lds, g);
-        else some_rows(integral_constant<int, 3>(), integral_constant<int, 4>(), 0, nc, lds, g);
+        // rows from memory on the first waves, those from LDS on the others
+        if (nc < nF) some_rows(integral_constant<int, 1>(), integral_constant<int, 16>(), w, nc, nF, mem, g);
+        const int w1 = (w + NW - (nF - nc) % NW) % NW;
+        if (nc <= NW) some_rows(integral_constant<int, 1>(), integral_constant<int, 8>(), w1, 0, nc, lds, g);
+        else some_rows(integral_constant<int, 3>(), integral_constant<int, 4>(), w1, 0, nc, lds, g);
     };
     // the restricted vector from its pieces, added in slot order; the loads of
     // a thread's first two pieces per value are in flight together
     auto gather = [&](const double* rcs) {
         double g0[kEpt], g1[kEpt];
+        const int tt = fresh(t);
 #pragma unroll
         for (int e = 0; e < kEpt; ++e) {
-            const uint32_t u = slots[e], u1 = u & (u - 1);
-            const int k = t + e * NT;
+            const uint32_t u = (uint32_t)fresh((int)slots[e]), u1 = u & (u - 1);
+            const int k = tt + e * NT;
             g0[e] = u ? get_at(rcs, (__ffs(u) - 1) * s.m + k) : 0.0;
             g1[e] = u1 ? get_at(rcs, (__ffs(u1) - 1) * s.m + k) : 0.0;
         }
 #pragma unroll
         for (int e = 0; e < kEpt; ++e) {
-            const int k = t + e * NT;
-            const uint32_t u1 = slots[e] & (slots[e] - 1);
+            const int k = tt + e * NT;
+            const uint32_t u = (uint32_t)fresh((int)slots[e]), u1 = u & (u - 1);
             double acc = g0[e] + g1[e];
-            for (uint32_t u = u1 & (u1 - 1); u; u &= u - 1) acc += get_at(rcs, (__ffs(u) - 1) * s.m + k);
+            for (uint32_t w2 = u1 & (u1 - 1); w2; w2 &= w2 - 1) acc += get_at(rcs, (__ffs(w2) - 1) * s.m + k);
             if (k < s.m) dyn[k] = acc;
         }
     };
@@ -545,10 +603,12 @@ __device__ __forceinline__ void solve_body(const PSys<T>& s, int L) {
     };
     // z = z1 from the frame's coarse values y, or 0
     auto start_z = [&](const double* y) {
+        const int tt = fresh(t);
+        const uint32_t zz = (uint32_t)fresh((int)zm);
 #pragma unroll
         for (int q = 0; q < QZ; ++q) {
-            const int idx = t + q * NT;
-            if (idx < HZ * WZ) za[idx] = COARSE && ((zm >> q) & 1u) ? (T)y[zi[COARSE ? q : 0]] : T(0);
+            const int idx = tt + q * NT;
+            if (idx < HZ * WZ) za[idx] = COARSE && ((zz >> q) & 1u) ? (T)y[fresh(zi[COARSE ? q : 0])] : T(0);
         }
         __syncthreads();
     };
@@ -558,7 +618,7 @@ __device__ __forceinline__ void solve_body(const PSys<T>& s, int L) {
             const int h = NS - hs, cc = hs & 1;
 #pragma unroll
             for (int q = 0; q < Q; ++q) {
-                if (dq[q][cc] > h) continue;
+                if (fresh(dq[q][cc]) > h) continue;
                 const int z0 = pz[q][cc];
                 const CT zc = za[z0];
                 CT az = cr[q][cc][0] * zc;
@@ -582,9 +642,7 @@ __device__ __forceinline__ void solve_body(const PSys<T>& s, int L) {
         return y;
     };
     auto into_yb = [&](int q, int cc, double y) {
-        const int P = t + q * NT, lr = P / (TJ / 2);
-        const int lc = pz[q][cc] - (lr + NS + 1) * WZ - (NS + 1);
-        yb[lr * TJ + lc] = ((fm >> (2 * q + cc)) & 1u) ? y : 0.0;
+        yb[yb_at(q, cc)] = PL.t_in_yb || (((uint32_t)fresh((int)fm) >> (2 * q + cc)) & 1u) ? y : 0.0;
     };
 
     double rho = 0.0, alpha = 0.0, omega = 1.0, r0 = 0.0, best = 1e300;
@@ -596,7 +654,7 @@ __device__ __forceinline__ void solve_body(const PSys<T>& s, int L) {
         for (int q = 0; q < QI; ++q)
 #pragma unroll
             for (int cc = 0; cc < 2; ++cc)
-                if (t + q * NT < NPI) into_yb(q, cc, (double)rts[(2 * q + cc) * NT + t]);
+                if (t + q * NT < NPI) into_yb(q, cc, ((own >> (2 * q + cc)) & 1u) ? (double)rtv(q, cc) : 0.0);
         // (through the second buffer, whose next words follow another round)
         restrict_yb(s.rct);
         if (!meet<NT>(s.flags, L, G, ++round, s.abort, &bad)) status = kAborted;
@@ -621,12 +679,13 @@ __device__ __forceinline__ void solve_body(const PSys<T>& s, int L) {
                 for (int cc = 0; cc < 2; ++cc) {
                     const uint32_t bit = 1u << (2 * q + cc);
                     CT y = CT(0);
-                    if (own & bit) {
+                    if ((uint32_t)fresh((int)own) & bit) {
                         y = matvec(q, cc);
-                        v[q][cc] = (T)y;
-                        hps[(2 * q + cc) * NT + t] = za[pz[q][cc]];
-                        if (edge & bit) put(s.v + kq[q][cc], (T)y);
-                        sum[0] += (double)rts[(2 * q + cc) * NT + t] * (double)y;
+                        if (q >= QF) v[q >= QF ? q - QF : 0][cc] = (T)y;
+                        else vs[(2 * q + cc) * NT + t] = (T)y;
+                        if constexpr (PL.p_in_lds) hps[(2 * q + cc) * NT + t] = za[pz[q][cc]];
+                        if ((uint32_t)fresh((int)edge) & bit) put_at(s.v, kq[q][cc], (T)y);
+                        sum[0] += (double)rtv(q, cc) * (double)y;
                     }
                     if (COARSE && t + q * NT < NPI) into_yb(q, cc, (double)y);
                 }
@@ -641,10 +700,12 @@ __device__ __forceinline__ void solve_body(const PSys<T>& s, int L) {
 #pragma unroll
                 for (int q = 0; q < 3; ++q) mine[q] = get_at(s.pa, 4 * t + q);
 #pragma unroll
-            for (int q = 0; q < Q; ++q)
+            for (int q = QF; q < Q; ++q)
 #pragma unroll
-                for (int cc = 0; cc < 2; ++cc)
-                    if (dq[q][cc] > 0 && dq[q][cc] <= NS) v[q][cc] = get_at(s.v, kq[q][cc]);
+                for (int cc = 0; cc < 2; ++cc) {
+                    const int d = fresh(dq[q][cc]);
+                    if (d > 0 && d <= NS) v[q - QF][cc] = get_at(s.v, kq[q][cc]);
+                }
             if (COARSE) gather(s.rcv);
             totals<3, NT>(mine, G, tot, red2);   // its barrier covers dyn
         }
@@ -684,14 +745,23 @@ __device__ __forceinline__ void solve_body(const PSys<T>& s, int L) {
 #pragma unroll
             for (int q = 0; q < Q; ++q)
 #pragma unroll
-                for (int cc = 0; cc < 2; ++cc) r[q][cc] = r[q][cc] - fa * v[q][cc];   // s (bicgsolver.py:110)
+                for (int cc = 0; cc < 2; ++cc) {
+                    const T vq = q >= QF ? v[q >= QF ? q - QF : 0][cc] : vs[(2 * q + cc) * NT + t];
+                    r[q][cc] = r[q][cc] - fa * vq;                      // s (bicgsolver.py:110)
+                    if constexpr (!PL.p_in_lds)
+                        if (q < QI && (((uint32_t)fresh((int)own) >> (2 * q + cc)) & 1u)) {
+                            const T dx = (T)(alpha * (double)za[pz[q][cc]]);
+                            if constexpr (PL.x_in_lds) xs[(2 * q + cc) * NT + t] += dx;
+                            else s.x[kq[q][cc]] += dx;
+                        }
+                }
         }
-        if (COARSE) __syncthreads();
+        if (COARSE || !PL.p_in_lds) __syncthreads();   // ysv, and z, which start_z writes
         // ---- s^ = M(s), t = A s^; <t,s>, <t,t>, <s,r~>, <t,r~>
         if (shared) share(ysv, s.Ys, round + 1);
         start_z(shared ? yl : ysv);
         sweep(r);
-        T th[Q][2];
+        T th[Q - QF][2];
         {
             double sum[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
@@ -700,12 +770,13 @@ __device__ __forceinline__ void solve_body(const PSys<T>& s, int L) {
                 for (int cc = 0; cc < 2; ++cc) {
                     const uint32_t bit = 1u << (2 * q + cc);
                     CT y = CT(0);
-                    th[q][cc] = T(0);
-                    if (own & bit) {
+                    if (q >= QF) th[q >= QF ? q - QF : 0][cc] = T(0);
+                    if ((uint32_t)fresh((int)own) & bit) {
                         y = matvec(q, cc);
-                        th[q][cc] = (T)y;
-                        if (edge & bit) put(s.t + kq[q][cc], (T)y);
-                        const double sk = (double)r[q][cc], rk = (double)rts[(2 * q + cc) * NT + t];
+                        if (q >= QF) th[q >= QF ? q - QF : 0][cc] = (T)y;
+                        else if constexpr (!PL.t_in_yb) ts[(2 * q + cc) * NT + t] = (T)y;
+                        if ((uint32_t)fresh((int)edge) & bit) put_at(s.t, kq[q][cc], (T)y);
+                        const double sk = (double)r[q][cc], rk = (double)rtv(q, cc);
                         sum[0] += (double)y * sk;
                         sum[1] += (double)y * (double)y;
                         sum[2] += sk * rk;
@@ -724,11 +795,12 @@ __device__ __forceinline__ void solve_body(const PSys<T>& s, int L) {
 #pragma unroll
                 for (int q = 0; q < 4; ++q) mine[q] = get_at(s.pb, 4 * t + q);
 #pragma unroll
-            for (int q = 0; q < Q; ++q)
+            for (int q = QF; q < Q; ++q)
 #pragma unroll
                 for (int cc = 0; cc < 2; ++cc) {
-                    if (q >= QI) th[q][cc] = T(0);
-                    if (dq[q][cc] > 0 && dq[q][cc] <= NS) th[q][cc] = get_at(s.t, kq[q][cc]);
+                    if (q >= QI) th[q - QF][cc] = T(0);
+                    const int d = fresh(dq[q][cc]);
+                    if (d > 0 && d <= NS) th[q - QF][cc] = get_at(s.t, kq[q][cc]);
                 }
             if (COARSE) gather(s.rct);
             totals<4, NT>(mine, G, pt, red2);
@@ -751,13 +823,21 @@ __device__ __forceinline__ void solve_body(const PSys<T>& s, int L) {
         for (int q = 0; q < Q; ++q)
 #pragma unroll
             for (int cc = 0; cc < 2; ++cc) {
-                const T rn = r[q][cc] - fo * th[q][cc];                      // bicgsolver.py:134
+                T tq;
+                if (q >= QF) tq = th[q >= QF ? q - QF : 0][cc];
+                else if constexpr (PL.t_in_yb) tq = (T)yb[yb_at(q, cc)];
+                else tq = ts[(2 * q + cc) * NT + t];
+                const T vq = q >= QF ? v[q >= QF ? q - QF : 0][cc] : vs[(2 * q + cc) * NT + t];
+                const T rn = r[q][cc] - fo * tq;                             // bicgsolver.py:134
                 r[q][cc] = rn;
-                p[q][cc] = rn + fb * (p[q][cc] - fo * v[q][cc]);             // bicgsolver.py:103
-                if (q < QI && ((own >> (2 * q + cc)) & 1u)) {
+                p[q][cc] = rn + fb * (p[q][cc] - fo * vq);                   // bicgsolver.py:103
+                if (q < QI && (((uint32_t)fresh((int)own) >> (2 * q + cc)) & 1u)) {
                     // s^ is still in za
                     const int o = (2 * q + cc) * NT + t;
-                    xs[o] = xs[o] + (T)(alpha * (double)hps[o] + omega * (double)za[pz[q][cc]]);
+                    const double dx = omega * (double)za[pz[q][cc]];
+                    if constexpr (PL.p_in_lds) xs[o] = xs[o] + (T)(alpha * (double)hps[o] + dx);
+                    else if constexpr (PL.x_in_lds) xs[o] += (T)dx;
+                    else s.x[kq[q][cc]] += (T)dx;
                     rr += (double)rn * (double)rn;
                 }
             }
@@ -768,7 +848,10 @@ __device__ __forceinline__ void solve_body(const PSys<T>& s, int L) {
     for (int q = 0; q < QI; ++q)
 #pragma unroll
         for (int cc = 0; cc < 2; ++cc)
-            if ((own >> (2 * q + cc)) & 1u) s.x[kq[q][cc]] = status < kUnsupported ? xs[(2 * q + cc) * NT + t] : T(0);
+            if ((own >> (2 * q + cc)) & 1u) {
+                if constexpr (PL.x_in_lds) s.x[kq[q][cc]] = status < kUnsupported ? xs[(2 * q + cc) * NT + t] : T(0);
+                else if (status >= kUnsupported) s.x[kq[q][cc]] = T(0);
+            }
     if (t == 0 && (L == 0 || status == kAborted)) {
         // the host's words (read after the stream has been waited for)
         if (L == 0) {
@@ -1113,9 +1196,7 @@ int frame_rows(int B, int shape) {
 
 // Bytes of solve_body's LDS arrays with a coarse level, rounded up.
 size_t solve_lds(int TI, int TJ, int NT, int sweeps, size_t vec) {
-    const int h = 2 * (2 * sweeps + 1);
-    const size_t QI = (TI * TJ / 2 + NT - 1) / NT;
-    return (TI + h) * (TJ + h) * vec + (size_t)TI * TJ * 8 + 6 * QI * NT * vec + kMaxF * (5 * 8 + sizeof(Piece)) + 4096;
+    return plan(TI, TJ, NT, sweeps, true, vec).bytes + kMaxF * (5 * 8 + sizeof(Piece)) + 2048;
 }
 
 int compute_units(km_ctx* ctx) {
@@ -1242,10 +1323,20 @@ int finish(km_ctx* ctx, int nsys, const std::function<void()>& launch, KState* o
 
 namespace kmpersist {
 
+// Longer systems stay by launches.  A p' solve takes 31 iterations at 1280 x 256,
+// 39 at 1500 x 300 and 50 to 62 at 1999 x 401; from about 40 on BiCGSTAB amplifies
+// the rounding of another summation order, in p' itself or in the momentum
+// solves before it, to the size of the tolerance, and the step's result, though
+// as accurate, is another one (eps = 1e-8: p' changes by 1e-12, 4e-10 and 1e-9 of
+// its norm at those sizes).  The gain would be 1.4x at 1500 x 300 (p' 50 us per
+// iteration against 72), 1.2x at 1999 x 401, and 2.5x for the momentum solves.
+constexpr int kMaxSide = 1300;
+
 bool fits_twolevel(km_ctx* ctx, const km_coarse* C, int NX, int NY, int* shape) {
     if (!C || C->m > kMaxM || (ctx->persist && ctx->persist->off >= 2)) return false;
     const int cus = std::min(kMaxWg, compute_units(ctx));
     const int nx = NX - 2, ny = NY - 2;
+    if (nx > kMaxSide || ny > kMaxSide) return false;
     for (int k = 0; k < kNumShapes; ++k) {
         const int64_t G = (int64_t)tiles_of(nx, kTI[k]) * tiles_of(ny, kTJ[k]);
         if (G > cus) continue;
@@ -1266,7 +1357,7 @@ bool fits_twolevel(km_ctx* ctx, const km_coarse* C, int NX, int NY, int* shape) 
 constexpr int kHalfShapes = 4;
 
 bool fits_smooth(km_ctx* ctx, int NX, int NY, int* shape) {
-    if (ctx->persist && ctx->persist->off >= 2) return false;
+    if ((ctx->persist && ctx->persist->off >= 2) || std::max(NX, NY) - 2 > kMaxSide + 1) return false;
     const int cus = std::min(kMaxWg, compute_units(ctx));
     for (int half = 1; half >= 0; --half)
         for (int k = 0; k < (half ? kHalfShapes : kNumShapes); ++k) {
@@ -1278,7 +1369,7 @@ bool fits_smooth(km_ctx* ctx, int NX, int NY, int* shape) {
     return false;
 }
 
-#define KM_SHAPES(X) X(0) X(1) X(2) X(3) X(4) X(5)
+#define KM_SHAPES(X) X(0) X(1) X(2) X(3) X(4) X(5) X(6)
 
 template <typename T>
 int twolevel(km_ctx* ctx, int shape, int NX, int NY, const double* coef, const T* rhs, T* xd, T* ws, double eps,

@@ -64,8 +64,11 @@ def check(x, info, coef, b):
 
 
 # one cell over and under the tiles (16 x 16, 16 x 32, 32 x 32, 40 x 32, 48 x 32,
-# 48 x 48 cells), a single tile, and 256 tiles of a shape (where the next begins)
-SHAPES = [(6, 5), (18, 18), (19, 17), (50, 34), (49, 67), (258, 258), (259, 258), (258, 515), (514, 516)]
+# 48 x 48, 64 x 56 cells), a single tile, 256 tiles of a shape (where the next
+# begins), systems of the two largest shapes, and the longest side and one past it
+# (by launches)
+SHAPES = [(6, 5), (18, 18), (19, 17), (50, 34), (49, 67), (258, 258), (259, 258), (258, 515), (514, 516), (602, 702),
+          (802, 802), (1302, 34), (1304, 35)]
 
 
 @pytest.mark.parametrize("NX,NY", SHAPES)
