@@ -99,11 +99,22 @@ k_prep_weights(const LayerOff* __restrict__ L, int64_t nwf, int64_t nwt, const f
 
 // ------------------------------------------------------------ convolution
 
-// One wave computes 16*Q pixels x 16*RTW output channels (row tiles
-// blockIdx.z*RTW ...); a workgroup is 4 waves along the pixels, so the grid is
-// (pixels / 64Q, batch, COUT / 16RTW) and low-resolution layers still launch
-// thousands of waves.  The operand fragments of the next 32-wide K chunk are
-// loaded while the MFMAs of the current one run (two register sets).
+// A workgroup computes TH rows of 16 pixels: WR waves share the rows and split
+// the output channels (RTW tiles of 16 each, blockIdx.z the rest), 4 / WR groups
+// of waves take Q rows each, so TH = Q 4 / WR.  The input of those rows, one
+// pixel around them included, is brought into LDS once, pooled, upsampled or
+// concatenated on the way; an operand fragment (8 channels of a pixel) is then
+// one 16-byte LDS read at an offset that a small table gives per K chunk.
+// Before, each wave fetched every fragment from memory for each of the nine
+// taps, with its own index arithmetic.  The layers of a 1280 x 256 system:
+// 116 us now, 200 then; the 192-channel one at 320 x 64 pixels 34 us (133
+// TFLOP/s) and 58, the last one at 1280 x 256 pixels 27 and 38.  What bounds it
+// now is filling the patch: one wait for memory per workgroup, and too few
+// workgroups per compute unit (one or two at the coarser levels) to hide it.  The
+// weights' fragments come from memory (the L1, all workgroups read the same),
+// one chunk ahead.  K runs in the same order for every output, so the results
+// have the bits of that kernel.  The pixel stride in LDS is an odd number of
+// 16-byte units: 16 pixels' reads fall on different banks.
 // MODE 0: input src0 (C0 channels) at the output resolution.
 // MODE 1: input = [2x nearest upsample of src0 (C0 channels, half resolution) | src1 (C1 channels)].
 // MODE 2: input = 2x2 average pool of src0 (C0 channels, double resolution), rounded to BF16 as k_pool does.
@@ -120,7 +131,7 @@ struct FusedOut {
     int accum;    // add to the output field instead of overwriting it
 };
 
-template <int MODE, int C0, int C1, int COUT, int OUTK, int Q, int RTW, typename T = float>
+template <int MODE, int C0, int C1, int COUT, int OUTK, int WR, int RTW, int Q, typename T = float>
 __global__ void __launch_bounds__(KM_BLOCK)
 k_conv3x3(int H, int W, const bf16* __restrict__ src0, const bf16* __restrict__ src1, const bf16* __restrict__ Wm,
           const float* __restrict__ bias, void* __restrict__ out, const int* __restrict__ skip, FusedOut fo) {
@@ -128,86 +139,84 @@ k_conv3x3(int H, int W, const bf16* __restrict__ src0, const bf16* __restrict__ 
     constexpr int CIN = C0 + C1;
     constexpr int KP = round32(9 * CIN);
     constexpr int NCH = KP / 32;
-    static_assert(C0 % 8 == 0 && C1 % 8 == 0 && COUT % (16 * RTW) == 0, "channel counts");
+    constexpr int TH = Q * 4 / WR, PW = 18;               // rows of the tile, columns of the patch
+    constexpr int LX = (CIN / 8) % 2 ? CIN : CIN + 8;     // pixel stride in LDS
+    constexpr int VX = CIN / 8;
+    static_assert(C0 % 8 == 0 && C1 % 8 == 0 && COUT % (16 * WR * RTW) == 0, "channel counts");
+    __shared__ __align__(16) bf16 xs[(TH + 2) * PW * LX];
+    __shared__ int koff[NCH * 4];                         // LDS offset of a K chunk's eight channels; < 0: past the taps
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int g = lane >> 4, col = lane & 15;
     const int64_t HW = (int64_t)H * W;
     const int b = blockIdx.y;
-    const int rt0 = blockIdx.z * RTW;
-    const int64_t px0 = ((int64_t)blockIdx.x * 4 + wave) * (16 * Q);
-    if (px0 >= HW) return;
-    int pi[Q], pj[Q];
-    bool pv[Q];
-#pragma unroll
-    for (int q = 0; q < Q; ++q) {
-        const int64_t p = px0 + q * 16 + col;
-        pv[q] = p < HW;
-        pi[q] = pv[q] ? (int)(p / W) : 0;
-        pj[q] = pv[q] ? (int)(p % W) : 0;
-    }
+    const int tw = (W + 15) / 16;
+    const int i0 = (blockIdx.x / tw) * TH, j0 = (blockIdx.x % tw) * 16;
+    const int rt0 = (blockIdx.z * WR + wave % WR) * RTW, q0 = wave / WR * Q;
     const bf16* s0 = src0 + (MODE == 0 ? (int64_t)b * HW * C0 : MODE == 1 ? (int64_t)b * (HW / 4) * C0
                                                                           : (int64_t)b * (4 * HW) * C0);
     const bf16* s1 = MODE == 1 ? src1 + (int64_t)b * HW * C1 : nullptr;
-    const bf16* wrow = Wm + (int64_t)(rt0 * 16 + col) * KP + g * 8;
     const int Wc = W >> 1;
-    auto load = [&](int kc, bf16x8 (&bv)[Q], bf16x8 (&av)[RTW]) {
-        const int k0 = kc + g * 8;
-        const int tap = k0 / CIN, c = k0 - tap * CIN;
-        const int dy = tap / 3 - 1, dx = tap - (tap / 3) * 3 - 1;
+    for (int u = threadIdx.x; u < NCH * 4; u += KM_BLOCK) {
+        const int k0 = u * 8, tap = k0 / CIN;
+        koff[u] = tap < 9 ? ((tap / 3) * PW + tap % 3) * LX + (k0 - tap * CIN) : -1;
+    }
+    for (int u = threadIdx.x; u < (TH + 2) * PW * VX; u += KM_BLOCK) {
+        const int px = u / VX, c = (u - px * VX) * 8;
+        const int ii = i0 - 1 + px / PW, jj = j0 - 1 + px % PW;
+        bf16x8 v = zero8();
+        if (ii >= 0 && ii < H && jj >= 0 && jj < W) {
+            if (MODE == 2) {
+                const bf16* f = s0 + ((int64_t)(2 * ii) * (2 * W) + 2 * jj) * C0 + c;
+                const bf16x8 x00 = *reinterpret_cast<const bf16x8*>(f);
+                const bf16x8 x01 = *reinterpret_cast<const bf16x8*>(f + C0);
+                const bf16x8 x10 = *reinterpret_cast<const bf16x8*>(f + (int64_t)2 * W * C0);
+                const bf16x8 x11 = *reinterpret_cast<const bf16x8*>(f + (int64_t)2 * W * C0 + C0);
 #pragma unroll
-        for (int q = 0; q < Q; ++q) {
-            const int ii = pi[q] + dy, jj = pj[q] + dx;
-            if (tap < 9 && pv[q] && ii >= 0 && ii < H && jj >= 0 && jj < W) {
-                if (MODE == 2) {
-                    const bf16* f = s0 + ((int64_t)(2 * ii) * (2 * W) + 2 * jj) * C0 + c;
-                    const bf16x8 x00 = *reinterpret_cast<const bf16x8*>(f);
-                    const bf16x8 x01 = *reinterpret_cast<const bf16x8*>(f + C0);
-                    const bf16x8 x10 = *reinterpret_cast<const bf16x8*>(f + (int64_t)2 * W * C0);
-                    const bf16x8 x11 = *reinterpret_cast<const bf16x8*>(f + (int64_t)2 * W * C0 + C0);
-                    bf16x8 o;
-#pragma unroll
-                    for (int e = 0; e < 8; ++e)
-                        o[e] = (bf16)(0.25f * ((((float)x00[e] + (float)x01[e]) + (float)x10[e]) + (float)x11[e]));
-                    bv[q] = o;
-                } else {
-                    const bf16* ptr;
-                    if (MODE == 0)
-                        ptr = s0 + ((int64_t)ii * W + jj) * C0 + c;
-                    else if (c < C0)
-                        ptr = s0 + ((int64_t)(ii >> 1) * Wc + (jj >> 1)) * C0 + c;
-                    else
-                        ptr = s1 + ((int64_t)ii * W + jj) * C1 + (c - C0);
-                    bv[q] = *reinterpret_cast<const bf16x8*>(ptr);
-                }
+                for (int e = 0; e < 8; ++e)
+                    v[e] = (bf16)(0.25f * ((((float)x00[e] + (float)x01[e]) + (float)x10[e]) + (float)x11[e]));
+            } else if (MODE == 0) {
+                v = *reinterpret_cast<const bf16x8*>(s0 + ((int64_t)ii * W + jj) * C0 + c);
+            } else if (c < C0) {
+                v = *reinterpret_cast<const bf16x8*>(s0 + ((int64_t)(ii >> 1) * Wc + (jj >> 1)) * C0 + c);
             } else {
-                bv[q] = zero8();
+                v = *reinterpret_cast<const bf16x8*>(s1 + ((int64_t)ii * W + jj) * C1 + (c - C0));
             }
         }
-#pragma unroll
-        for (int rt = 0; rt < RTW; ++rt) av[rt] = *reinterpret_cast<const bf16x8*>(wrow + (int64_t)rt * 16 * KP + kc);
-    };
+        *reinterpret_cast<bf16x8*>(xs + px * LX + c) = v;
+    }
+    const bf16* wrow = Wm + (int64_t)(rt0 * 16 + col) * KP + g * 8;
     floatx4 acc[RTW][Q];
 #pragma unroll
     for (int rt = 0; rt < RTW; ++rt)
 #pragma unroll
         for (int q = 0; q < Q; ++q) acc[rt][q] = floatx4{0.f, 0.f, 0.f, 0.f};
-    auto mma = [&](const bf16x8 (&bv)[Q], const bf16x8 (&av)[RTW]) {
+    bf16x8 av[2][RTW];
+#pragma unroll
+    for (int rt = 0; rt < RTW; ++rt) av[0][rt] = *reinterpret_cast<const bf16x8*>(wrow + (int64_t)rt * 16 * KP);
+    __syncthreads();
+    const bf16* x0 = xs + (q0 * PW + col) * LX;
+#pragma unroll 2
+    for (int ch = 0; ch < NCH; ++ch) {
+        const int cur = ch & 1;
+        if (ch + 1 < NCH)
+#pragma unroll
+            for (int rt = 0; rt < RTW; ++rt)
+                av[cur ^ 1][rt] = *reinterpret_cast<const bf16x8*>(wrow + (int64_t)rt * 16 * KP + (ch + 1) * 32);
+        const int ko = koff[ch * 4 + g];
+        bf16x8 bv[Q];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            bv[q] = *reinterpret_cast<const bf16x8*>(x0 + q * PW * LX + (ko < 0 ? 0 : ko));
+            if (9 * CIN % 32 != 0 && ko < 0) bv[q] = zero8();
+        }
 #pragma unroll
         for (int rt = 0; rt < RTW; ++rt)
 #pragma unroll
             for (int q = 0; q < Q; ++q)
-                acc[rt][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[rt], bv[q], acc[rt][q], 0, 0, 0);
-    };
-    bf16x8 b0[Q], a0[RTW], b1[Q], a1[RTW];
-    load(0, b0, a0);
-    for (int ch = 0; ch < NCH; ch += 2) {
-        if (ch + 1 < NCH) load((ch + 1) * 32, b1, a1);
-        mma(b0, a0);
-        if (ch + 1 < NCH) {
-            if (ch + 2 < NCH) load((ch + 2) * 32, b0, a0);
-            mma(b1, a1);
-        }
+                acc[rt][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[cur][rt], bv[q], acc[rt][q], 0, 0, 0);
     }
+    // this lane's pixel of row q: (i0 + q0 + q, j0 + col)
+    const bool jin = j0 + col < W;
     if constexpr (OUTK == 2) {
         static_assert(COUT == 16 && RTW == 1, "fused output needs all 16 channels in one wave");
         // lane (g, col) holds channels 4g .. 4g+3 of pixel col: gather the 16
@@ -229,9 +238,8 @@ k_conv3x3(int H, int W, const bf16* __restrict__ src0, const bf16* __restrict__ 
                 all[8 + i] = __shfl(y[i], col + 32, 64);
                 all[12 + i] = __shfl(y[i], col + 48, 64);
             }
-            if (g == 0 && pv[q]) {
-                const int64_t p = px0 + q * 16 + col;
-                const int a = (int)(p / W), cc = (int)(p % W);
+            if (g == 0 && jin && i0 + q0 + q < H) {
+                const int a = i0 + q0 + q, cc = j0 + col;
                 if (a < fo.NX - 2 && cc < fo.NY - 2) {
                     const int64_t k = (int64_t)(a + 1) * fo.NY + (cc + 1);
                     if (free_cell(fo.coef, n, k)) {
@@ -253,8 +261,8 @@ k_conv3x3(int H, int W, const bf16* __restrict__ src0, const bf16* __restrict__ 
         const int co = (rt0 + rt) * 16 + g * 4;
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
-            if (!pv[q]) continue;
-            const int64_t o = ((int64_t)b * HW + px0 + q * 16 + col) * COUT + co;
+            if (!jin || i0 + q0 + q >= H) continue;
+            const int64_t o = ((int64_t)b * HW + (int64_t)(i0 + q0 + q) * W + j0 + col) * COUT + co;
             if (OUTK == 0) {
                 bf16x4 v;
 #pragma unroll
@@ -873,12 +881,16 @@ int flat_blocks(int64_t n) {
     return g < 1 ? 1 : (int)g;
 }
 
-template <int MODE, int C0, int C1, int COUT, int OUTK, int Q, int RTW, typename T = float>
+// Waves on the output channels (WR, RTW tiles each) and rows per wave: a
+// fragment from LDS serves RTW products and one from memory Q.  Few pixels
+// (the coarser levels) take fewer rows per workgroup, so that there are
+// several hundred workgroups.
+template <int MODE, int C0, int C1, int COUT, int OUTK, int WR, int RTW, int Q, typename T = float>
 void conv(int H, int W, int B, const bf16* s0, const bf16* s1, const bf16* Wm, const float* bias, void* out,
-          const int* skip, hipStream_t st, FusedOut fo = FusedOut{}) {
-    const int64_t HW = (int64_t)H * W;
-    const dim3 grid((unsigned)((HW + 64 * Q - 1) / (64 * Q)), (unsigned)B, (unsigned)(COUT / (16 * RTW)));
-    hipLaunchKernelGGL((k_conv3x3<MODE, C0, C1, COUT, OUTK, Q, RTW, T>), grid, dim3(KM_BLOCK), 0, st, H, W, s0, s1,
+          const int* skip, hipStream_t st, const FusedOut& fo = FusedOut{}) {
+    constexpr int TH = Q * 4 / WR;
+    const dim3 grid((unsigned)(((H + TH - 1) / TH) * ((W + 15) / 16)), (unsigned)B, COUT / (16 * WR * RTW));
+    hipLaunchKernelGGL((k_conv3x3<MODE, C0, C1, COUT, OUTK, WR, RTW, Q, T>), grid, dim3(KM_BLOCK), 0, st, H, W, s0, s1,
                        Wm, bias, out, skip, fo);
 }
 
@@ -1001,16 +1013,16 @@ void forward(km_net* N, int B, const float* params, const int* skip, hipStream_t
     const int H1 = H / 2, W1 = W / 2, H2 = H / 4, W2 = W / 4, H3 = H / 8, W3 = W / 8;
     const LayerOff* L = N->lay.L;
     const bf16* wf = N->wf;
-    conv<0, 8, 0, 16, 0, 4, 1>(H, W, B, N->X0, nullptr, wf + L[E0].wf, params + L[E0].b, N->e0, skip, st);
+    conv<0, 8, 0, 16, 0, 1, 1, 4>(H, W, B, N->X0, nullptr, wf + L[E0].wf, params + L[E0].b, N->e0, skip, st);
     pool<16>(H1, W1, B, N->e0, N->p1, skip, st);
-    conv<0, 16, 0, 32, 0, 4, 1>(H1, W1, B, N->p1, nullptr, wf + L[E1].wf, params + L[E1].b, N->e1, skip, st);
+    conv<0, 16, 0, 32, 0, 1, 2, 2>(H1, W1, B, N->p1, nullptr, wf + L[E1].wf, params + L[E1].b, N->e1, skip, st);
     pool<32>(H2, W2, B, N->e1, N->p2, skip, st);
-    conv<0, 32, 0, 64, 0, 1, 2>(H2, W2, B, N->p2, nullptr, wf + L[E2].wf, params + L[E2].b, N->e2, skip, st);
+    conv<0, 32, 0, 64, 0, 2, 2, 2>(H2, W2, B, N->p2, nullptr, wf + L[E2].wf, params + L[E2].b, N->e2, skip, st);
     pool<64>(H3, W3, B, N->e2, N->p3, skip, st);
-    conv<0, 64, 0, 128, 0, 1, 2>(H3, W3, B, N->p3, nullptr, wf + L[E3].wf, params + L[E3].b, N->e3, skip, st);
-    conv<1, 128, 64, 64, 0, 1, 1>(H2, W2, B, N->e3, N->e2, wf + L[D2].wf, params + L[D2].b, N->d2, skip, st);
-    conv<1, 64, 32, 32, 0, 2, 1>(H1, W1, B, N->d2, N->e1, wf + L[D1].wf, params + L[D1].b, N->d1, skip, st);
-    conv<1, 32, 16, 16, 0, 4, 1>(H, W, B, N->d1, N->e0, wf + L[D0].wf, params + L[D0].b, N->d0, skip, st);
+    conv<0, 64, 0, 128, 0, 2, 2, 1>(H3, W3, B, N->p3, nullptr, wf + L[E3].wf, params + L[E3].b, N->e3, skip, st);
+    conv<1, 128, 64, 64, 0, 2, 2, 2>(H2, W2, B, N->e3, N->e2, wf + L[D2].wf, params + L[D2].b, N->d2, skip, st);
+    conv<1, 64, 32, 32, 0, 1, 2, 2>(H1, W1, B, N->d2, N->e1, wf + L[D1].wf, params + L[D1].b, N->d1, skip, st);
+    conv<1, 32, 16, 16, 0, 1, 1, 4>(H, W, B, N->d1, N->e0, wf + L[D0].wf, params + L[D0].b, N->d0, skip, st);
 }
 
 // Inference: pools folded into the next convolution's gather and the output
@@ -1022,14 +1034,14 @@ void forward_infer(km_net* N, const float* params, const int* skip, hipStream_t 
     const int H1 = H / 2, W1 = W / 2, H2 = H / 4, W2 = W / 4, H3 = H / 8, W3 = W / 8;
     const LayerOff* L = N->lay.L;
     const bf16* wf = N->wf;
-    conv<0, 8, 0, 16, 0, 4, 1>(H, W, 1, N->X0, nullptr, wf + L[E0].wf, params + L[E0].b, N->e0, skip, st);
-    conv<2, 16, 0, 32, 0, 4, 1>(H1, W1, 1, N->e0, nullptr, wf + L[E1].wf, params + L[E1].b, N->e1, skip, st);
-    conv<2, 32, 0, 64, 0, 1, 2>(H2, W2, 1, N->e1, nullptr, wf + L[E2].wf, params + L[E2].b, N->e2, skip, st);
-    conv<2, 64, 0, 128, 0, 1, 2>(H3, W3, 1, N->e2, nullptr, wf + L[E3].wf, params + L[E3].b, N->e3, skip, st);
-    conv<1, 128, 64, 64, 0, 1, 1>(H2, W2, 1, N->e3, N->e2, wf + L[D2].wf, params + L[D2].b, N->d2, skip, st);
-    conv<1, 64, 32, 32, 0, 2, 1>(H1, W1, 1, N->d2, N->e1, wf + L[D1].wf, params + L[D1].b, N->d1, skip, st);
+    conv<0, 8, 0, 16, 0, 1, 1, 4>(H, W, 1, N->X0, nullptr, wf + L[E0].wf, params + L[E0].b, N->e0, skip, st);
+    conv<2, 16, 0, 32, 0, 1, 2, 2>(H1, W1, 1, N->e0, nullptr, wf + L[E1].wf, params + L[E1].b, N->e1, skip, st);
+    conv<2, 32, 0, 64, 0, 2, 2, 2>(H2, W2, 1, N->e1, nullptr, wf + L[E2].wf, params + L[E2].b, N->e2, skip, st);
+    conv<2, 64, 0, 128, 0, 2, 2, 1>(H3, W3, 1, N->e2, nullptr, wf + L[E3].wf, params + L[E3].b, N->e3, skip, st);
+    conv<1, 128, 64, 64, 0, 2, 2, 2>(H2, W2, 1, N->e3, N->e2, wf + L[D2].wf, params + L[D2].b, N->d2, skip, st);
+    conv<1, 64, 32, 32, 0, 1, 2, 2>(H1, W1, 1, N->d2, N->e1, wf + L[D1].wf, params + L[D1].b, N->d1, skip, st);
     const FusedOut fo{params + N->lay.out_w, coef, (const double*)N->stats, NX, NY, accum};
-    conv<1, 32, 16, 16, 2, 4, 1, T>(H, W, 1, N->d1, N->e0, wf + L[D0].wf, params + L[D0].b, z, skip, st, fo);
+    conv<1, 32, 16, 16, 2, 1, 1, 4, T>(H, W, 1, N->d1, N->e0, wf + L[D0].wf, params + L[D0].b, z, skip, st, fo);
 }
 
 // Backward from dy_d0 (already written by k_loss_grad) to every parameter.
@@ -1040,32 +1052,32 @@ void backward(km_net* N, int B, float* grad, hipStream_t st) {
     const bf16* wt = N->wt;
     // d0: input [up(d1) | e0]
     wgrad<1, 32, 16, 16>(N, D0, H, W, B, N->d1, N->e0, N->dy_d0, grad, st);
-    conv<0, 16, 0, 48, 1, 4, 1>(H, W, B, N->dy_d0, nullptr, wt + L[D0].wt, nullptr, N->dX0, nullptr, st);
+    conv<0, 16, 0, 48, 1, 1, 3, 2>(H, W, B, N->dy_d0, nullptr, wt + L[D0].wt, nullptr, N->dX0, nullptr, st);
     hipLaunchKernelGGL((k_split_up<32, 16>), dim3(flat_blocks((int64_t)B * H1 * W1 * 32)), dim3(KM_BLOCK), 0, st, H1, W1,
                        B, (const float*)N->dX0, (const bf16*)N->d1, N->dy_d1);
     // d1: input [up(d2) | e1]
     wgrad<1, 64, 32, 32>(N, D1, H1, W1, B, N->d2, N->e1, N->dy_d1, grad, st);
-    conv<0, 32, 0, 96, 1, 2, 1>(H1, W1, B, N->dy_d1, nullptr, wt + L[D1].wt, nullptr, N->dX1, nullptr, st);
+    conv<0, 32, 0, 96, 1, 2, 3, 2>(H1, W1, B, N->dy_d1, nullptr, wt + L[D1].wt, nullptr, N->dX1, nullptr, st);
     hipLaunchKernelGGL((k_split_up<64, 32>), dim3(flat_blocks((int64_t)B * H2 * W2 * 64)), dim3(KM_BLOCK), 0, st, H2, W2,
                        B, (const float*)N->dX1, (const bf16*)N->d2, N->dy_d2);
     // d2: input [up(e3) | e2]
     wgrad<1, 128, 64, 64>(N, D2, H2, W2, B, N->e3, N->e2, N->dy_d2, grad, st);
-    conv<0, 64, 0, 192, 1, 1, 2>(H2, W2, B, N->dy_d2, nullptr, wt + L[D2].wt, nullptr, N->dX2, nullptr, st);
+    conv<0, 64, 0, 192, 1, 4, 3, 4>(H2, W2, B, N->dy_d2, nullptr, wt + L[D2].wt, nullptr, N->dX2, nullptr, st);
     hipLaunchKernelGGL((k_split_up<128, 64>), dim3(flat_blocks((int64_t)B * H3 * W3 * 128)), dim3(KM_BLOCK), 0, st, H3,
                        W3, B, (const float*)N->dX2, (const bf16*)N->e3, N->dy_e3);
     // e3: input p3
     wgrad<0, 64, 0, 128>(N, E3, H3, W3, B, N->p3, nullptr, N->dy_e3, grad, st);
-    conv<0, 128, 0, 64, 1, 1, 1>(H3, W3, B, N->dy_e3, nullptr, wt + L[E3].wt, nullptr, N->dp3, nullptr, st);
+    conv<0, 128, 0, 64, 1, 2, 2, 2>(H3, W3, B, N->dy_e3, nullptr, wt + L[E3].wt, nullptr, N->dp3, nullptr, st);
     hipLaunchKernelGGL(k_combine<64>, dim3(flat_blocks((int64_t)B * H2 * W2 * 64)), dim3(KM_BLOCK), 0, st, H2, W2, B,
                        (const float*)(N->dX2 + 128), 192, (const float*)N->dp3, (const bf16*)N->e2, N->dy_e2);
     // e2: input p2
     wgrad<0, 32, 0, 64>(N, E2, H2, W2, B, N->p2, nullptr, N->dy_e2, grad, st);
-    conv<0, 64, 0, 32, 1, 1, 1>(H2, W2, B, N->dy_e2, nullptr, wt + L[E2].wt, nullptr, N->dp2, nullptr, st);
+    conv<0, 64, 0, 32, 1, 1, 2, 2>(H2, W2, B, N->dy_e2, nullptr, wt + L[E2].wt, nullptr, N->dp2, nullptr, st);
     hipLaunchKernelGGL(k_combine<32>, dim3(flat_blocks((int64_t)B * H1 * W1 * 32)), dim3(KM_BLOCK), 0, st, H1, W1, B,
                        (const float*)(N->dX1 + 64), 96, (const float*)N->dp2, (const bf16*)N->e1, N->dy_e1);
     // e1: input p1
     wgrad<0, 16, 0, 32>(N, E1, H1, W1, B, N->p1, nullptr, N->dy_e1, grad, st);
-    conv<0, 32, 0, 16, 1, 4, 1>(H1, W1, B, N->dy_e1, nullptr, wt + L[E1].wt, nullptr, N->dp1, nullptr, st);
+    conv<0, 32, 0, 16, 1, 1, 1, 4>(H1, W1, B, N->dy_e1, nullptr, wt + L[E1].wt, nullptr, N->dp1, nullptr, st);
     hipLaunchKernelGGL(k_combine<16>, dim3(flat_blocks((int64_t)B * H * W * 16)), dim3(KM_BLOCK), 0, st, H, W, B,
                        (const float*)(N->dX0 + 32), 48, (const float*)N->dp1, (const bf16*)N->e0, N->dy_e0);
     // e0: input X0
