@@ -35,7 +35,7 @@ struct km_net {
     bf16 *X0, *e0, *p1, *e1, *p2, *e2, *p3, *e3, *d2, *d1, *d0;
     bf16 *dy_d0, *dy_d1, *dy_d2, *dy_e3, *dy_e2, *dy_e1, *dy_e0;
     float *z, *q, *ae, *dX0, *dX1, *dX2, *dp3, *dp2, *dp1, *wpart;
-    float *c32, *r32, *z32;     // FP32 staging of one system (km_unet_apply)
+    float *c32, *r32;           // FP32 staging of one system (km_unet_apply)
     double *P, *stats, *loss;
     int64_t wpart_n = 0;
 };
@@ -617,6 +617,46 @@ k_net_stats(int NX, int NY, const T* __restrict__ r, int64_t rstride, const floa
     }
 }
 
+// The FP32 copies of a system's FP64 coefficients and right-hand side, and the
+// sums of k_net_stats over them, in one pass: 48 bytes read and 24 written per
+// cell, 8 us at 1280 x 256.  The copies and the sums in two launches of each
+// took 38 us, 30 of them in the sums, whose 81 workgroups walked 4096 cells
+// each, one load after another.
+__global__ void __launch_bounds__(KM_BLOCK)
+k_ingest(int NX, int NY, const double* __restrict__ coef, const double* __restrict__ r, float* __restrict__ c32,
+         float* __restrict__ r32, double* __restrict__ P, int G) {
+    __shared__ double sh[4];
+    const int64_t n = (int64_t)NX * NY;
+    const int64_t chunk = (n + G - 1) / G;
+    const int64_t lo = (int64_t)blockIdx.x * chunk;
+    const int64_t hi = lo + chunk < n ? lo + chunk : n;
+    double s0 = 0.0, s1 = 0.0, s2 = 0.0;
+    for (int64_t k = lo + threadIdx.x; k < hi; k += KM_BLOCK) {
+        float c[5];
+#pragma unroll
+        for (int q = 0; q < 5; ++q) c[q] = (float)coef[q * n + k];
+        const float v = (float)r[k];
+#pragma unroll
+        for (int q = 0; q < 5; ++q) c32[q * n + k] = c[q];
+        r32[k] = v;
+        s0 += (double)v * (double)v;
+        const int i = (int)(k / NY), j = (int)(k % NY);
+        if (i >= 1 && i <= NX - 2 && j >= 1 && j <= NY - 2 &&
+            (c[1] != 0.f || c[2] != 0.f || c[3] != 0.f || c[4] != 0.f)) {
+            s1 += (double)c[0];
+            s2 += 1.0;
+        }
+    }
+    s0 = block_sum(s0, sh);
+    s1 = block_sum(s1, sh);
+    s2 = block_sum(s2, sh);
+    if (threadIdx.x == 0) {
+        P[blockIdx.x] = s0;
+        P[G + blockIdx.x] = s1;
+        P[2 * G + blockIdx.x] = s2;
+    }
+}
+
 // stats[b*8 + ...]: 0 r.r, 1 rs = sqrt(r.r / n_free), 3 abar, 4 rs / abar, 5 n_free.
 __global__ void __launch_bounds__(KM_BLOCK)
 k_net_stats_finish(int G, const double* __restrict__ P, int full, double* __restrict__ stats, const int* __restrict__ skip) {
@@ -651,16 +691,16 @@ k_net_stats_finish(int G, const double* __restrict__ P, int full, double* __rest
 // X0[b][a][c][0..7] = (r / rs, aP / abar on free cells, 1 on identity rows, 0 ...)
 // zc (may be null): an output field of B x NX x NY values cleared on the way
 // (the fused output layer then writes only free interior cells).
-template <typename T>
+template <typename T, typename Z = T>
 __global__ void __launch_bounds__(KM_BLOCK)
 k_features(int NX, int NY, int H, int W, int B, const T* __restrict__ r, int64_t rstride, const float* __restrict__ coef,
            int64_t cstride, const double* __restrict__ stats, bf16* __restrict__ X0, const int* __restrict__ skip,
-           T* __restrict__ zc) {
+           Z* __restrict__ zc) {
     if (skipped(skip)) return;
     const int64_t HW = (int64_t)H * W, n = (int64_t)NX * NY, tot = (int64_t)B * HW;
     if (zc)
         for (int64_t i = (int64_t)blockIdx.x * KM_BLOCK + threadIdx.x; i < (int64_t)B * n; i += (int64_t)gridDim.x * KM_BLOCK)
-            zc[i] = T(0);
+            zc[i] = Z(0);
     for (int64_t idx = (int64_t)blockIdx.x * KM_BLOCK + threadIdx.x; idx < tot; idx += (int64_t)gridDim.x * KM_BLOCK) {
         const int64_t b = idx / HW, p = idx % HW;
         const int a = (int)(p / W), c = (int)(p % W);
@@ -867,12 +907,6 @@ k_adam(int64_t n, float* __restrict__ p, const float* __restrict__ g, float* __r
     }
 }
 
-template <typename S, typename D>
-__global__ void __launch_bounds__(KM_BLOCK) k_convert(int64_t n, const S* __restrict__ a, D* __restrict__ out) {
-    for (int64_t i = (int64_t)blockIdx.x * KM_BLOCK + threadIdx.x; i < n; i += (int64_t)gridDim.x * KM_BLOCK)
-        out[i] = (D)a[i];
-}
-
 // ------------------------------------------------------------ host side
 
 int flat_blocks(int64_t n) {
@@ -958,7 +992,7 @@ int alloc(km_ctx* ctx, km_net* N, int B, int NX, int NY) {
         {(void**)&M.dX0, B * hw0 * 48 * fb}, {(void**)&M.dX1, B * hw1 * 96 * fb}, {(void**)&M.dX2, B * hw2 * 192 * fb},
         {(void**)&M.dp3, B * hw3 * 64 * fb}, {(void**)&M.dp2, B * hw2 * 32 * fb}, {(void**)&M.dp1, B * hw1 * 16 * fb},
         {(void**)&M.wpart, kWpartMax * fb},
-        {(void**)&M.c32, 5 * n * fb},        {(void**)&M.r32, n * fb},            {(void**)&M.z32, n * fb},
+        {(void**)&M.c32, 5 * n * fb},        {(void**)&M.r32, n * fb},
         {(void**)&M.P, kPartials * sizeof(double)}, {(void**)&M.stats, kMaxBatch * 8 * sizeof(double)},
         {(void**)&M.loss, kMaxBatch * sizeof(double)},
         {(void**)&M.wf, (size_t)M.lay.nwf * bb}, {(void**)&M.wt, (size_t)M.lay.nwt * bb},
@@ -993,8 +1027,8 @@ int alloc(km_ctx* ctx, km_net* N, int B, int NX, int NY) {
     N->NY = NY;
     N->H = H;
     N->W = W;
-    int64_t gs = n / 4096 + 1;
-    N->Gs = (int)(gs > 256 ? 256 : gs);
+    int64_t gs = n / 1024 + 1;
+    N->Gs = (int)(gs > 1024 ? 1024 : gs);
     KM_HIP_SYNC(ctx, hipMemcpy(N->dL, N->lay.L, sizeof(LayerOff) * NL, hipMemcpyHostToDevice));
     KM_HIP_SYNC(ctx, hipMemset(N->stats, 0, kMaxBatch * 8 * sizeof(double)));
     return KM_OK;
@@ -1202,12 +1236,14 @@ int km_unet_apply(km_ctx* ctx, const float* params, int NX, int NY, const double
     km_net* N = ctx->net;
     const int64_t n = (int64_t)NX * NY;
     hipStream_t s = ctx->stream;
-    hipLaunchKernelGGL((k_convert<double, float>), dim3(flat_blocks(5 * n)), dim3(KM_BLOCK), 0, s, 5 * n, coef, N->c32);
-    hipLaunchKernelGGL((k_convert<double, float>), dim3(flat_blocks(n)), dim3(KM_BLOCK), 0, s, n, r, N->r32);
-    KM_CHECK_LAUNCH(ctx);
-    if (int rc = kmnet::solve_stats(ctx, NX, NY, N->c32, s)) return rc;
-    if (int rc = kmnet::apply<float>(ctx, NX, NY, N->c32, N->r32, N->z32, nullptr, s, params)) return rc;
-    hipLaunchKernelGGL((k_convert<float, double>), dim3(flat_blocks(n)), dim3(KM_BLOCK), 0, s, n, (const float*)N->z32, z);
+    hipLaunchKernelGGL(k_ingest, dim3(N->Gs), dim3(KM_BLOCK), 0, s, NX, NY, coef, r, N->c32, N->r32, N->P, N->Gs);
+    hipLaunchKernelGGL(k_net_stats_finish, dim3(1), dim3(KM_BLOCK), 0, s, N->Gs, (const double*)N->P, 1, N->stats,
+                       (const int*)nullptr);
+    // z may be the caller's r or coef: nothing reads those from here on
+    hipLaunchKernelGGL((k_features<float, double>), dim3(flat_blocks((int64_t)N->H * N->W)), dim3(KM_BLOCK), 0, s, NX, NY,
+                       N->H, N->W, 1, (const float*)N->r32, (int64_t)0, (const float*)N->c32, (int64_t)0,
+                       (const double*)N->stats, N->X0, (const int*)nullptr, z);
+    forward_infer<double>(N, params, nullptr, s, z, N->c32, NX, NY);
     KM_CHECK_LAUNCH(ctx);
     return KM_OK;
 }

@@ -32,3 +32,15 @@ def test_forward_at_tile_edges(nx, ny, dev):
     err = np.linalg.norm(z - zo) / np.linalg.norm(zo)
     print(f"{nx}x{ny}: {err:.1e}")
     assert err < 1e-2
+
+
+def test_forward_in_place(dev):
+    """The output may be the right-hand side's own buffer."""
+    coef, r = small_system(71, nx=65, ny=33)
+    pt = torch.tensor(unet.init_params(6), device=dev)
+    ct, rt = torch.tensor(coef, device=dev), torch.tensor(r, device=dev)
+    zt = torch.empty_like(rt)
+    ctx = _lib.context_for(dev)
+    ctx.call("km_unet_apply", ptr(pt), 67, 35, ptr(ct), ptr(rt), ptr(zt))
+    ctx.call("km_unet_apply", ptr(pt), 67, 35, ptr(ct), ptr(rt), ptr(rt))
+    assert torch.equal(rt, zt)
