@@ -14,6 +14,7 @@
 #include "km_unet.h"
 
 #include <cmath>
+#include <type_traits>
 
 typedef __bf16 bf16;
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
@@ -287,96 +288,156 @@ k_conv3x3(int H, int W, const bf16* __restrict__ src0, const bf16* __restrict__ 
 // channels of a pixel side by side: fetched two bytes at a time from memory
 // every fragment took eight loads with their own index arithmetic, and the
 // kernel waited for them (609 us for the 48-channel layer at 4 x 1280 x 256
-// pixels, 1.1 TFLOP/s).  Now the workgroup brings kWgPx pixels of dY and, for
-// the three rows of taps, kWgPx + 2 pixels of the input into LDS with 16-byte
-// loads, once for all nine taps and all waves, and the fragments are gathered
-// there.  Pixels are taken in linear order (a tap is a shift of dy W + dx); a
-// tap that leaves the image is cleared by each lane's pixel masks.  The pixel
-// stride in LDS is CIN + 2 values: the four 8-pixel groups of a fragment then
-// start 8 banks apart.
+// pixels, 1.1 TFLOP/s).  Now the workgroup brings PX pixels of dY and, for
+// the three rows of taps, PX + 2 pixels of the input into LDS with 16-byte
+// loads, six of a thread in flight, once for all nine taps and all waves, and a
+// fragment is two transposing LDS reads (each hands a lane four pixels of its
+// channel).  Gathered two bytes at a time in LDS, with divisions for every
+// vector's place, the three decoder layers took 400, 319 and 302 us at that
+// size; now 243, 180 and 137 (75, 101 and 132 TFLOP/s; the FP32 partial sums'
+// 0.5 GB are 90 us of the first).  What bounds it: bringing and multiplying take
+// turns in a workgroup, and two workgroups fit a compute unit.
+// Pixels are taken in linear order (a tap is a shift of dy W + dx); a tap that
+// leaves the image is cleared by each lane's pixel masks.  The pixel stride in
+// LDS is CIN + 4 values: a quarter wave's reads are 8-byte aligned and its
+// pixels start on different banks.
 constexpr int kWgPx = 64;
 
 template <int MODE, int C0, int C1, int COUT, int CT>
-__global__ void __launch_bounds__(KM_BLOCK)
+__global__ void __launch_bounds__(KM_BLOCK, 2)
 k_wgrad(int H, int W, int B, const bf16* __restrict__ src0, const bf16* __restrict__ src1,
         const bf16* __restrict__ dY, int pps, float* __restrict__ part) {
     constexpr int CIN = C0 + C1;
+    constexpr int PX = CIN > 128 ? kWgPx / 2 : kWgPx;   // pixels in LDS: several workgroups per compute unit
+    constexpr int kInFlight = 6;
     constexpr int KP = round32(9 * CIN);
     constexpr int NCT = KP / 16;
     constexpr int RT = COUT / 16;
-    constexpr int LX = CIN + 2, LY = COUT + 2;          // pixel strides in LDS
+    constexpr int LX = CIN + 4, LY = COUT + 4;          // pixel strides in LDS
     constexpr int VX = CIN / 8, VY = COUT / 8;          // 16-byte vectors per pixel
-    constexpr int NX3 = 3 * (kWgPx + 2) * VX, NY1 = kWgPx * VY;
-    __shared__ bf16 xs[3 * (kWgPx + 2) * LX];
-    __shared__ bf16 ys[kWgPx * LY];
+    constexpr int NX3 = 3 * (PX + 2) * VX, NY1 = PX * VY;
+    __shared__ __align__(8) bf16 xs[3 * (PX + 2) * LX];
+    __shared__ __align__(8) bf16 ys[PX * LY];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int g = lane >> 4, col = lane & 15;
     const int HW = H * W, NPX = B * HW;
     const int split = blockIdx.x, ct0 = (blockIdx.y * 4 + wave) * CT;
     const int lo = split * pps, hi = lo + pps < NPX ? lo + pps : NPX;
     const int Wc = W >> 1;
-    int off[CT];        // LDS offset of this lane's column at pixel 0
+    // A lane reads four channels of one pixel and receives four pixels of one
+    // channel: it asks for pixel col / 4 (of four) and channels 4 (col % 4) ...,
+    // and the tap of its column is that of the masks below.
+    const int tp = col >> 2, tc = (col & 3) * 4;
+    int off[CT];        // LDS offset of the four channels this lane reads, at pixel tp
     int tdy[CT], tdx[CT];
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) {
-        const int kcol = (ct0 + ct) * 16 + col;
-        int tap = kcol / CIN;
-        const int c = kcol - tap * CIN;
-        // columns past the nine taps (KP is a multiple of 32) are not used: any valid offset
-        if (tap > 8) tap = 8;
+        auto tap_of = [](int kcol) {
+            // columns past the nine taps (KP is a multiple of 32) are not used: any valid offset
+            const int tap = kcol / CIN;
+            return tap > 8 ? 8 : tap;
+        };
+        const int kcol = (ct0 + ct) * 16 + col, kr = (ct0 + ct) * 16 + tc;
+        const int tap = tap_of(kcol), tr = tap_of(kr);
         tdy[ct] = tap / 3 - 1;
         tdx[ct] = tap - (tap / 3) * 3 - 1;
-        off[ct] = ((tdy[ct] + 1) * (kWgPx + 2) + tdx[ct] + 1) * LX + c;
+        off[ct] = ((tr / 3) * (PX + 2) + tr - (tr / 3) * 3 + tp) * LX + (kr / CIN > 8 ? tc % CIN : kr - tr * CIN);
     }
-    auto store8 = [](bf16* p, const bf16x8& v) {        // 4-byte aligned
+    auto store8 = [](bf16* p, const bf16x8& v) {        // 8-byte aligned
         const int4 q = *reinterpret_cast<const int4*>(&v);
-        int* d = reinterpret_cast<int*>(p);
-        d[0] = q.x;
-        d[1] = q.y;
-        d[2] = q.z;
-        d[3] = q.w;
+        int2* d = reinterpret_cast<int2*>(p);
+        d[0] = int2{q.x, q.y};
+        d[1] = int2{q.z, q.w};
+    };
+    // eight pixels of one channel: p is this lane's address for the first four
+    auto load8 = [](const bf16* p, int stride) {
+        typedef short s4 __attribute__((ext_vector_type(4)));
+        typedef __attribute__((address_space(3))) s4 lds4;
+        const s4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4*)p);
+        const s4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4*)(p + 4 * stride));
+        const int2 lo = *reinterpret_cast<const int2*>(&a), hi = *reinterpret_cast<const int2*>(&b);
+        return int4{lo.x, lo.y, hi.x, hi.y};
     };
     floatx4 acc[RT][CT];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) acc[rt][ct] = floatx4{0.f, 0.f, 0.f, 0.f};
-    for (int base = lo; base < hi; base += kWgPx) {
+    for (int base = lo; base < hi; base += PX) {
+        const int b0 = base / HW, i0 = (base - b0 * HW) / W, j0 = base % W;    // the chunk's first pixel
         __syncthreads();
-        for (int u = threadIdx.x; u < NX3; u += KM_BLOCK) {
-            const int px = u / VX, vc = (u - px * VX) * 8;
-            const int row = px / (kWgPx + 2), k = px - row * (kWgPx + 2);
-            const int q = base + (row - 1) * W + k - 1;     // linear pixel, perhaps of another row: masked later
-            bf16x8 v = zero8();
-            if (q >= 0 && q < NPX) {
-                if (MODE == 0) {
-                    v = *reinterpret_cast<const bf16x8*>(src0 + (int64_t)q * C0 + vc);
-                } else if (vc < C0) {
-                    const int b = q / HW, rem = q - b * HW, i = rem / W, j = rem - i * W;
-                    v = *reinterpret_cast<const bf16x8*>(
-                        src0 + ((int64_t)b * (HW / 4) + (int64_t)(i >> 1) * Wc + (j >> 1)) * C0 + vc);
-                } else {
-                    v = *reinterpret_cast<const bf16x8*>(src1 + (int64_t)q * C1 + (vc - C0));
+        // kInFlight vectors of a thread at a time
+        auto bring = [&](auto total, auto load, auto put) {
+            constexpr int N = decltype(total)::value;
+            int t = threadIdx.x;
+            // where the accumulators fill the registers, form the addresses here
+            // and not before the loop over the pixels (spilled: 252 us for 243)
+            if constexpr (COUT >= 64) asm volatile("" : "+v"(t));
+#pragma unroll
+            for (int u0 = 0; u0 < N; u0 += kInFlight * KM_BLOCK) {
+                bf16x8 v[kInFlight];
+#pragma unroll
+                for (int q = 0; q < kInFlight; ++q) {
+                    const int u = u0 + q * KM_BLOCK + t;
+                    v[q] = u < N ? load(u) : zero8();
+                }
+#pragma unroll
+                for (int q = 0; q < kInFlight; ++q) {
+                    const int u = u0 + q * KM_BLOCK + t;
+                    if (u < N) put(u, v[q]);
                 }
             }
-            store8(xs + px * LX + vc, v);
-        }
-        for (int u = threadIdx.x; u < NY1; u += KM_BLOCK) {
+        };
+        bring(std::integral_constant<int, NX3>{}, [&](int u) {
+            const int px = u / VX, vc = (u - px * VX) * 8;
+            const int row = px / (PX + 2), k = px - row * (PX + 2);
+            const int q = base + (row - 1) * W + k - 1;     // linear pixel, perhaps of another row: masked later
+            if (q < 0 || q >= NPX) return zero8();
+            if (MODE == 0) return *reinterpret_cast<const bf16x8*>(src0 + (int64_t)q * C0 + vc);
+            if (vc >= C0) return *reinterpret_cast<const bf16x8*>(src1 + (int64_t)q * C1 + (vc - C0));
+            int b = b0, i = i0 + row - 1, j = j0 + k - 1;
+            if (j < 0) {
+                j += W;
+                --i;
+            }
+            while (j >= W) {
+                j -= W;
+                ++i;
+            }
+            while (i < 0) {
+                i += H;
+                --b;
+            }
+            while (i >= H) {
+                i -= H;
+                ++b;
+            }
+            return *reinterpret_cast<const bf16x8*>(
+                src0 + ((int64_t)b * (HW / 4) + (int64_t)(i >> 1) * Wc + (j >> 1)) * C0 + vc);
+        }, [&](int u, const bf16x8& v) {
+            const int px = u / VX;
+            store8(xs + px * LX + (u - px * VX) * 8, v);
+        });
+        bring(std::integral_constant<int, NY1>{}, [&](int u) {
             const int px = u / VY, vc = (u - px * VY) * 8;
-            bf16x8 v = zero8();
-            if (base + px < hi) v = *reinterpret_cast<const bf16x8*>(dY + (int64_t)(base + px) * COUT + vc);
-            store8(ys + px * LY + vc, v);
-        }
+            if (base + px >= hi) return zero8();
+            return *reinterpret_cast<const bf16x8*>(dY + (int64_t)(base + px) * COUT + vc);
+        }, [&](int u, const bf16x8& v) {
+            const int px = u / VY;
+            store8(ys + px * LY + (u - px * VY) * 8, v);
+        });
         __syncthreads();
 #pragma unroll
-        for (int ch = 0; ch < kWgPx / 32; ++ch) {
+        for (int ch = 0; ch < PX / 32; ++ch) {
             const int p0 = ch * 32 + g * 8;     // this lane's first pixel of the chunk
             // bit e: pixel e has a neighbour above, below, left, right
             int up = 0, down = 0, left = 0, right = 0;
             {
-                const int P = base + p0 < NPX ? base + p0 : NPX - 1;
-                const int rem = P % HW;
-                int i = rem / W, j = rem - i * W;
+                int i = i0, j = j0 + p0;
+                while (j >= W) {
+                    j -= W;
+                    if (++i == H) i = 0;
+                }
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     up |= (i > 0) << e;
@@ -391,22 +452,25 @@ k_wgrad(int H, int W, int B, const bf16* __restrict__ src0, const bf16* __restri
             }
             bf16x8 av[RT];
 #pragma unroll
-            for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-                for (int e = 0; e < 8; ++e) av[rt][e] = ys[(p0 + e) * LY + rt * 16 + col];
+            for (int rt = 0; rt < RT; ++rt) {
+                const int4 a = load8(ys + (p0 + tp) * LY + rt * 16 + tc, LY);
+                av[rt] = *reinterpret_cast<const bf16x8*>(&a);
+            }
 #pragma unroll
             for (int ct = 0; ct < CT; ++ct) {
                 if (ct0 + ct >= NCT) continue;
-                bf16x8 bv;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) bv[e] = xs[off[ct] + (p0 + e) * LX];
+                int4 x = load8(xs + off[ct] + p0 * LX, LX);
                 const int in = (tdy[ct] < 0 ? up : tdy[ct] > 0 ? down : 0xff) &
                                (tdx[ct] < 0 ? left : tdx[ct] > 0 ? right : 0xff);
                 if (__any(in != 0xff)) {
-#pragma unroll
-                    for (int e = 0; e < 8; ++e)
-                        if (!((in >> e) & 1)) bv[e] = (bf16)0.0f;
+                    // two pixels per word: a bit of the mask becomes a half word
+                    auto two = [in](int e) { return (int)((in >> e & 1) * 0xffffu | (in >> (e + 1) & 1) * 0xffff0000u); };
+                    x.x &= two(0);
+                    x.y &= two(2);
+                    x.z &= two(4);
+                    x.w &= two(6);
                 }
+                const bf16x8 bv = *reinterpret_cast<const bf16x8*>(&x);
 #pragma unroll
                 for (int rt = 0; rt < RT; ++rt)
                     acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[rt], bv, acc[rt][ct], 0, 0, 0);
