@@ -35,7 +35,7 @@ struct km_net {
     bf16 *wf = nullptr, *wt = nullptr;
     bf16 *X0, *e0, *p1, *e1, *p2, *e2, *p3, *e3, *d2, *d1, *d0;
     bf16 *dy_d0, *dy_d1, *dy_d2, *dy_e3, *dy_e2, *dy_e1, *dy_e0;
-    float *z, *q, *ae, *dX0, *dX1, *dX2, *dp3, *dp2, *dp1, *wpart;
+    float *z, *q, *ae, *dX0, *dX1, *dX2, *wpart;
     float *c32, *r32;           // FP32 staging of one system (km_unet_apply)
     double *P, *stats, *loss;
     int64_t wpart_n = 0;
@@ -119,18 +119,31 @@ k_prep_weights(const LayerOff* __restrict__ L, int64_t nwf, int64_t nwt, const f
 // MODE 0: input src0 (C0 channels) at the output resolution.
 // MODE 1: input = [2x nearest upsample of src0 (C0 channels, half resolution) | src1 (C1 channels)].
 // MODE 2: input = 2x2 average pool of src0 (C0 channels, double resolution), rounded to BF16 as k_pool does.
-// OUTK 0: out = bf16(relu(acc + bias)); OUTK 1: out = acc in FP32 (input gradients);
-// OUTK 2 (COUT 16, RTW 1): the network output fused in: the 1x1 layer over
-// bf16(relu(acc + bias)) scaled as k_out does, written to the padded FP32 or
-// FP64 field ``out`` (type T) on free interior cells (fo: output parameters,
-// coef / stats / NX / NY: the system).
+// OUTK 0: out = bf16(relu(acc + bias)).
+// OUTK 1 (input gradients of [up(coarse) | skip], two thirds and one third of
+// the channels): the gradient of the coarse activation, out = bf16(sum over the
+// 2x2 children if fo.act > 0 else 0) on the half grid, and the skip's in FP32
+// to fo.skipg.
+// OUTK 3 (input gradient dp of a pooled activation): the activation's gradient
+// on the double grid, out = bf16((fo.skipg + dp / 4) if fo.act > 0 else 0).
+// A lane holds four channels of a pixel of each of its rows, so the 2x2 sum
+// takes its neighbour's registers and no memory.  With both in kernels of their
+// own, and the gradients stored in FP32 in between, the six layers of four
+// samples of 1280 x 256 took 229 + 185 us; now 259.
 struct FusedOut {
     const float* pw;
     const float* coef;
     const double* stats;
     int NX, NY;
     int accum;    // add to the output field instead of overwriting it
+    const bf16* act = nullptr;
+    float* skipg = nullptr;
 };
+
+// The value of the other column of a pair (lanes 2k and 2k + 1).
+__device__ __forceinline__ float next_lane(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, true));
+}
 
 template <int MODE, int C0, int C1, int COUT, int OUTK, int WR, int RTW, int Q, typename T = float>
 __global__ void __launch_bounds__(KM_BLOCK)
@@ -260,20 +273,63 @@ k_conv3x3(int H, int W, const bf16* __restrict__ src0, const bf16* __restrict__ 
 #pragma unroll
     for (int rt = 0; rt < RTW; ++rt) {
         const int co = (rt0 + rt) * 16 + g * 4;
+        if constexpr (OUTK == 1) {
+            constexpr int CU = COUT / 3 * 2, CS = COUT / 3;
+            static_assert(COUT % 48 == 0 && Q % 2 == 0, "whole tiles of each part, rows in pairs");
+            if ((rt0 + rt) * 16 < CU) {
 #pragma unroll
-        for (int q = 0; q < Q; ++q) {
-            if (!jin || i0 + q0 + q >= H) continue;
-            const int64_t o = ((int64_t)b * HW + (int64_t)(i0 + q0 + q) * W + j0 + col) * COUT + co;
-            if (OUTK == 0) {
-                bf16x4 v;
+                for (int q = 0; q < Q; q += 2) {
+                    float s[4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const float y = acc[rt][q][i] + bias[co + i];
-                    v[i] = (bf16)(y > 0.f ? y : 0.f);
+                    for (int i = 0; i < 4; ++i) {
+                        const float a0 = acc[rt][q][i], a1 = acc[rt][q + 1][i];
+                        s[i] = ((a0 + next_lane(a0)) + a1) + next_lane(a1);     // used by the even columns
+                    }
+                    const int i = i0 + q0 + q, j = j0 + col;
+                    if ((col & 1) || !jin || i >= H) continue;
+                    const int64_t o = (((int64_t)b * (H / 2) + (i >> 1)) * (W / 2) + (j >> 1)) * CU + co;
+                    const bf16x4 y = *reinterpret_cast<const bf16x4*>(fo.act + o);
+                    bf16x4 v;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] = (bf16)((float)y[e] > 0.f ? s[e] : 0.f);
+                    *reinterpret_cast<bf16x4*>(static_cast<bf16*>(out) + o) = v;
                 }
-                *reinterpret_cast<bf16x4*>(static_cast<bf16*>(out) + o) = v;
             } else {
-                *reinterpret_cast<floatx4*>(static_cast<float*>(out) + o) = acc[rt][q];
+#pragma unroll
+                for (int q = 0; q < Q; ++q)
+                    if (jin && i0 + q0 + q < H)
+                        *reinterpret_cast<floatx4*>(fo.skipg + ((int64_t)b * HW + (int64_t)(i0 + q0 + q) * W + j0 + col) * CS +
+                                                    (co - CU)) = acc[rt][q];
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                if (!jin || i0 + q0 + q >= H) continue;
+                const int i = i0 + q0 + q, j = j0 + col;
+                if constexpr (OUTK == 0) {
+                    bf16x4 v;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float y = acc[rt][q][e] + bias[co + e];
+                        v[e] = (bf16)(y > 0.f ? y : 0.f);
+                    }
+                    *reinterpret_cast<bf16x4*>(static_cast<bf16*>(out) + ((int64_t)b * HW + (int64_t)i * W + j) * COUT + co) = v;
+                } else if constexpr (OUTK == 3) {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const int64_t o =
+                            (((int64_t)b * (2 * H) + 2 * i + (k >> 1)) * (2 * (int64_t)W) + 2 * j + (k & 1)) * COUT + co;
+                        const floatx4 sg = *reinterpret_cast<const floatx4*>(fo.skipg + o);
+                        const bf16x4 y = *reinterpret_cast<const bf16x4*>(fo.act + o);
+                        bf16x4 v;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const float d = sg[e] + 0.25f * acc[rt][q][e];
+                            v[e] = (bf16)((float)y[e] > 0.f ? d : 0.f);
+                        }
+                        *reinterpret_cast<bf16x4*>(static_cast<bf16*>(out) + o) = v;
+                    }
+                }
             }
         }
     }
@@ -598,47 +654,6 @@ k_pool(int Ho, int Wo, int B, const bf16* __restrict__ in, bf16* __restrict__ ou
         for (int e = 0; e < 8; ++e)
             o[e] = (bf16)(0.25f * ((((float)x00[e] + (float)x01[e]) + (float)x10[e]) + (float)x11[e]));
         *reinterpret_cast<bf16x8*>(out + ((b * Ho + i) * (int64_t)Wo + j) * C + gc * 8) = o;
-    }
-}
-
-// Gradient of [up(coarse) | skip] -> gradient of the coarse activation:
-// dy = bf16(sum over the 2x2 children of dX[..., c] if act > 0 else 0).
-template <int CU, int CS>
-__global__ void __launch_bounds__(KM_BLOCK)
-k_split_up(int Hc, int Wc, int B, const float* __restrict__ dX, const bf16* __restrict__ act, bf16* __restrict__ dy) {
-    constexpr int CT_ = CU + CS;
-    const int64_t n = (int64_t)B * Hc * Wc * CU;
-    const int Wf = 2 * Wc;
-    for (int64_t idx = (int64_t)blockIdx.x * KM_BLOCK + threadIdx.x; idx < n; idx += (int64_t)gridDim.x * KM_BLOCK) {
-        const int c = (int)(idx % CU);
-        int64_t p = idx / CU;
-        const int jc = (int)(p % Wc);
-        p /= Wc;
-        const int ic = (int)(p % Hc);
-        const int64_t b = p / Hc;
-        const float* d = dX + ((b * 2 * Hc + 2 * ic) * (int64_t)Wf + 2 * jc) * CT_ + c;
-        const float s = ((d[0] + d[CT_]) + d[(int64_t)Wf * CT_]) + d[(int64_t)Wf * CT_ + CT_];
-        dy[idx] = (bf16)((float)act[idx] > 0.f ? s : 0.f);
-    }
-}
-
-// Encoder activation gradient: dy = bf16((skip gradient + unpool(dp)) if act > 0 else 0).
-template <int C>
-__global__ void __launch_bounds__(KM_BLOCK)
-k_combine(int H, int W, int B, const float* __restrict__ skipg, int sstride, const float* __restrict__ dp,
-          const bf16* __restrict__ act, bf16* __restrict__ dy) {
-    const int64_t n = (int64_t)B * H * W * C;
-    for (int64_t idx = (int64_t)blockIdx.x * KM_BLOCK + threadIdx.x; idx < n; idx += (int64_t)gridDim.x * KM_BLOCK) {
-        const int c = (int)(idx % C);
-        const int64_t p = idx / C;
-        const int j = (int)(p % W);
-        const int64_t pi = p / W;
-        const int i = (int)(pi % H);
-        const int64_t b = pi / H;
-        const float sg = skipg[p * sstride + c];
-        const float dv = dp[((b * (H / 2) + i / 2) * (int64_t)(W / 2) + j / 2) * C + c];
-        const float v = sg + 0.25f * dv;
-        dy[idx] = (bf16)((float)act[idx] > 0.f ? v : 0.f);
     }
 }
 
@@ -1053,8 +1068,7 @@ int alloc(km_ctx* ctx, km_net* N, int B, int NX, int NY) {
         {(void**)&M.dy_e2, B * hw2 * 64 * bb}, {(void**)&M.dy_e1, B * hw1 * 32 * bb},
         {(void**)&M.dy_e0, B * hw0 * 16 * bb},
         {(void**)&M.z, B * n * fb},          {(void**)&M.q, B * n * fb},          {(void**)&M.ae, B * n * fb},
-        {(void**)&M.dX0, B * hw0 * 48 * fb}, {(void**)&M.dX1, B * hw1 * 96 * fb}, {(void**)&M.dX2, B * hw2 * 192 * fb},
-        {(void**)&M.dp3, B * hw3 * 64 * fb}, {(void**)&M.dp2, B * hw2 * 32 * fb}, {(void**)&M.dp1, B * hw1 * 16 * fb},
+        {(void**)&M.dX0, B * hw0 * 16 * fb}, {(void**)&M.dX1, B * hw1 * 32 * fb}, {(void**)&M.dX2, B * hw2 * 64 * fb},
         {(void**)&M.wpart, kWpartMax * fb},
         {(void**)&M.c32, 5 * n * fb},        {(void**)&M.r32, n * fb},
         {(void**)&M.P, kPartials * sizeof(double)}, {(void**)&M.stats, kMaxBatch * 8 * sizeof(double)},
@@ -1148,36 +1162,36 @@ void backward(km_net* N, int B, float* grad, hipStream_t st) {
     const int H1 = H / 2, W1 = W / 2, H2 = H / 4, W2 = W / 4, H3 = H / 8, W3 = W / 8;
     const LayerOff* L = N->lay.L;
     const bf16* wt = N->wt;
+    auto grad_out = [](const bf16* act, float* skipg) {
+        FusedOut fo{};
+        fo.act = act;
+        fo.skipg = skipg;
+        return fo;
+    };
     // d0: input [up(d1) | e0]
     wgrad<1, 32, 16, 16>(N, D0, H, W, B, N->d1, N->e0, N->dy_d0, grad, st);
-    conv<0, 16, 0, 48, 1, 1, 3, 2>(H, W, B, N->dy_d0, nullptr, wt + L[D0].wt, nullptr, N->dX0, nullptr, st);
-    hipLaunchKernelGGL((k_split_up<32, 16>), dim3(flat_blocks((int64_t)B * H1 * W1 * 32)), dim3(KM_BLOCK), 0, st, H1, W1,
-                       B, (const float*)N->dX0, (const bf16*)N->d1, N->dy_d1);
+    conv<0, 16, 0, 48, 1, 1, 3, 2>(H, W, B, N->dy_d0, nullptr, wt + L[D0].wt, nullptr, N->dy_d1, nullptr, st,
+                                   grad_out(N->d1, N->dX0));
     // d1: input [up(d2) | e1]
     wgrad<1, 64, 32, 32>(N, D1, H1, W1, B, N->d2, N->e1, N->dy_d1, grad, st);
-    conv<0, 32, 0, 96, 1, 2, 3, 2>(H1, W1, B, N->dy_d1, nullptr, wt + L[D1].wt, nullptr, N->dX1, nullptr, st);
-    hipLaunchKernelGGL((k_split_up<64, 32>), dim3(flat_blocks((int64_t)B * H2 * W2 * 64)), dim3(KM_BLOCK), 0, st, H2, W2,
-                       B, (const float*)N->dX1, (const bf16*)N->d2, N->dy_d2);
+    conv<0, 32, 0, 96, 1, 2, 3, 2>(H1, W1, B, N->dy_d1, nullptr, wt + L[D1].wt, nullptr, N->dy_d2, nullptr, st,
+                                   grad_out(N->d2, N->dX1));
     // d2: input [up(e3) | e2]
     wgrad<1, 128, 64, 64>(N, D2, H2, W2, B, N->e3, N->e2, N->dy_d2, grad, st);
-    conv<0, 64, 0, 192, 1, 4, 3, 4>(H2, W2, B, N->dy_d2, nullptr, wt + L[D2].wt, nullptr, N->dX2, nullptr, st);
-    hipLaunchKernelGGL((k_split_up<128, 64>), dim3(flat_blocks((int64_t)B * H3 * W3 * 128)), dim3(KM_BLOCK), 0, st, H3,
-                       W3, B, (const float*)N->dX2, (const bf16*)N->e3, N->dy_e3);
+    conv<0, 64, 0, 192, 1, 4, 3, 4>(H2, W2, B, N->dy_d2, nullptr, wt + L[D2].wt, nullptr, N->dy_e3, nullptr, st,
+                                    grad_out(N->e3, N->dX2));
     // e3: input p3
     wgrad<0, 64, 0, 128>(N, E3, H3, W3, B, N->p3, nullptr, N->dy_e3, grad, st);
-    conv<0, 128, 0, 64, 1, 2, 2, 2>(H3, W3, B, N->dy_e3, nullptr, wt + L[E3].wt, nullptr, N->dp3, nullptr, st);
-    hipLaunchKernelGGL(k_combine<64>, dim3(flat_blocks((int64_t)B * H2 * W2 * 64)), dim3(KM_BLOCK), 0, st, H2, W2, B,
-                       (const float*)(N->dX2 + 128), 192, (const float*)N->dp3, (const bf16*)N->e2, N->dy_e2);
+    conv<0, 128, 0, 64, 3, 2, 2, 2>(H3, W3, B, N->dy_e3, nullptr, wt + L[E3].wt, nullptr, N->dy_e2, nullptr, st,
+                                    grad_out(N->e2, N->dX2));
     // e2: input p2
     wgrad<0, 32, 0, 64>(N, E2, H2, W2, B, N->p2, nullptr, N->dy_e2, grad, st);
-    conv<0, 64, 0, 32, 1, 1, 2, 2>(H2, W2, B, N->dy_e2, nullptr, wt + L[E2].wt, nullptr, N->dp2, nullptr, st);
-    hipLaunchKernelGGL(k_combine<32>, dim3(flat_blocks((int64_t)B * H1 * W1 * 32)), dim3(KM_BLOCK), 0, st, H1, W1, B,
-                       (const float*)(N->dX1 + 64), 96, (const float*)N->dp2, (const bf16*)N->e1, N->dy_e1);
+    conv<0, 64, 0, 32, 3, 1, 2, 2>(H2, W2, B, N->dy_e2, nullptr, wt + L[E2].wt, nullptr, N->dy_e1, nullptr, st,
+                                   grad_out(N->e1, N->dX1));
     // e1: input p1
     wgrad<0, 16, 0, 32>(N, E1, H1, W1, B, N->p1, nullptr, N->dy_e1, grad, st);
-    conv<0, 32, 0, 16, 1, 1, 1, 4>(H1, W1, B, N->dy_e1, nullptr, wt + L[E1].wt, nullptr, N->dp1, nullptr, st);
-    hipLaunchKernelGGL(k_combine<16>, dim3(flat_blocks((int64_t)B * H * W * 16)), dim3(KM_BLOCK), 0, st, H, W, B,
-                       (const float*)(N->dX0 + 32), 48, (const float*)N->dp1, (const bf16*)N->e0, N->dy_e0);
+    conv<0, 32, 0, 16, 3, 1, 1, 4>(H1, W1, B, N->dy_e1, nullptr, wt + L[E1].wt, nullptr, N->dy_e0, nullptr, st,
+                                   grad_out(N->e0, N->dX0));
     // e0: input X0
     wgrad<0, 8, 0, 16>(N, E0, H, W, B, N->X0, nullptr, N->dy_e0, grad, st);
 }
