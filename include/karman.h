@@ -154,11 +154,19 @@ int km_residual(km_ctx* ctx, int NX, int NY, const double* coef, const double* b
 /* BICGSolver.solve (bicgsolver.py:88-136): FP64 coefficients, right-hand side and solution. */
 int km_bicgstab(km_ctx* ctx, int NX, int NY, const double* coef, const double* b, double* x,
                 double eps, int max_iter, int flags, km_solve_info* info);
+/* One launch: km_bicgstab, km_cg and km_fbicgstab (with KM_FLAG_COARSE or
+ * KM_FLAG_SMOOTH and no network) run a whole solve as one launch of at most one
+ * workgroup per compute unit where the system's tiles fit the GPU, its boundary
+ * rows and columns are empty and no tile was set by the caller; other systems,
+ * and a launch that could not get all its workgroups resident within two
+ * seconds, are solved by launches.  The results do not depend on what else runs.
+ * Launches of this kind wait for one another on a device. */
 /* km_bicgstab without any allocation: no counterpart in the reference.  For
  * callers that cannot allocate device memory (code under stream capture, tight
  * serving loops, harnesses that forbid hipMalloc).  The same plain BiCGSTAB
- * kernels as km_bicgstab, launched directly (no graphs), with the solver's
- * state, partial sums and eight Krylov vectors in a device array the library
+ * kernels as km_bicgstab (in one launch where the system fits the GPU, else
+ * launched directly, no graphs), with the solver's state, partial sums and
+ * eight Krylov vectors in a device array the library
  * reserves once per GPU (KM_NOALLOC_SCRATCH_BYTES = 32 MiB; at most
  * KM_NOALLOC_MAX_CELLS = NX*NY cells, e.g. the 1282 x 258 p' system of a
  * 1280 x 256 grid).  Larger systems and KM_FLAG_MIXED return KM_EINVAL.  The
@@ -225,10 +233,11 @@ int km_adam_step(km_ctx* ctx, int64_t n, float* params, const float* grad, float
  * B x B aggregates of free cells (Galerkin A_c, its inverse held across
  * solves, km_set_coarse_update), then the network on r - A z1, added to z1 --
  * or, without a network, two red-black SOR sweeps (omega 1.3) on A z = r from
- * z1, run as a fused four-launch iteration.  KM_FLAG_SMOOTH: one or two
+ * z1, run in one launch or as a fused four-launch iteration.  KM_FLAG_SMOOTH: one or two
  * red-black Gauss-Seidel sweeps (km_set_momentum_sweeps) on A z = r from
  * zero as the preconditioner (no network,
- * no coarse level; the momentum systems), a fused three-launch iteration.
+ * no coarse level; the momentum systems), in one launch or as a fused
+ * three-launch iteration.
  * FP64 solves from x = 0 with either fused iteration solve straight into x. */
 int km_fbicgstab(km_ctx* ctx, int NX, int NY, const double* coef, const double* b, double* x, double eps,
                  int max_iter, int flags, const float* params, km_solve_info* info);
@@ -236,7 +245,7 @@ int km_fbicgstab(km_ctx* ctx, int NX, int NY, const double* coef, const double* 
  * calls BICGSolver.solve on each in turn): two independent km_fbicgstab
  * solves with the same eps, max_iter and flags, results and info as two
  * separate calls.  With KM_FLAG_SMOOTH and none of KM_FLAG_MIXED, KM_FLAG_X0,
- * KM_FLAG_COARSE the two systems' first sweeps iterate in the same launches
+ * KM_FLAG_COARSE the two systems' first sweeps iterate in the same launch or launches
  * (each workgroup serves one system; each system stops on its own test);
  * otherwise the two solves run one after the other. */
 int km_fbicgstab2(km_ctx* ctx, int NX0, int NY0, const double* coef0, const double* b0, double* x0, int NX1, int NY1,
@@ -249,7 +258,8 @@ int km_fbicgstab2(km_ctx* ctx, int NX0, int NY0, const double* coef0, const doub
  * several cases) every system keeps its own coarse level and smoothing tile,
  * and the first sweeps of systems of the same tile shape, up to four at a
  * time, iterate in the same launches, each workgroup serving one system and
- * each system stopping on its own test; otherwise the solves run one after
+ * each system stopping on its own test; otherwise, and for the systems that
+ * one launch holds whole, the solves run one after
  * the other.  n <= KM_MAX_GROUP_SOLVES; the systems must not share x or
  * coefficients.  No counterpart in the reference (one case per process). */
 #define KM_MAX_GROUP_SOLVES 256
