@@ -350,11 +350,13 @@ k_conv3x3(int H, int W, const bf16* __restrict__ src0, const bf16* __restrict__ 
 // fragment is two transposing LDS reads (each hands a lane four pixels of its
 // channel).  Gathered two bytes at a time in LDS, with divisions for every
 // vector's place, the three decoder layers took 400, 319 and 302 us at that
-// size; now 243, 180 and 137 (75, 101 and 132 TFLOP/s; the FP32 partial sums'
+// size; now 234, 167 and 118 (78, 109 and 153 TFLOP/s; the FP32 partial sums'
 // 0.5 GB are 90 us of the first).  What bounds it: bringing and multiplying take
 // turns in a workgroup, and two workgroups fit a compute unit.
 // Pixels are taken in linear order (a tap is a shift of dy W + dx); a tap that
-// leaves the image is cleared by each lane's pixel masks.  The pixel stride in
+// leaves the image is cleared by each lane's pixel masks (one word for the four
+// directions, formed from the first of the lane's eight pixels: bit by bit the
+// layers above took 243, 180 and 137).  The pixel stride in
 // LDS is CIN + 4 values: a quarter wave's reads are 8-byte aligned and its
 // pixels start on different banks.
 constexpr int kWgPx = 64;
@@ -385,7 +387,7 @@ k_wgrad(int H, int W, int B, const bf16* __restrict__ src0, const bf16* __restri
     // and the tap of its column is that of the masks below.
     const int tp = col >> 2, tc = (col & 3) * 4;
     int off[CT];        // LDS offset of the four channels this lane reads, at pixel tp
-    int tdy[CT], tdx[CT];
+    unsigned past[CT];  // bytes of the four directions this lane's tap does not look in: 0xff
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) {
         auto tap_of = [](int kcol) {
@@ -395,8 +397,8 @@ k_wgrad(int H, int W, int B, const bf16* __restrict__ src0, const bf16* __restri
         };
         const int kcol = (ct0 + ct) * 16 + col, kr = (ct0 + ct) * 16 + tc;
         const int tap = tap_of(kcol), tr = tap_of(kr);
-        tdy[ct] = tap / 3 - 1;
-        tdx[ct] = tap - (tap / 3) * 3 - 1;
+        past[ct] = (tap < 3 ? 0u : 0xffu) | (tap < 6 ? 0xff00u : 0u) | (tap % 3 == 0 ? 0u : 0xff0000u) |
+                   (tap % 3 == 2 ? 0u : 0xff000000u);
         off[ct] = ((tr / 3) * (PX + 2) + tr - (tr / 3) * 3 + tp) * LX + (kr / CIN > 8 ? tc % CIN : kr - tr * CIN);
     }
     auto store8 = [](bf16* p, const bf16x8& v) {        // 8-byte aligned
@@ -427,7 +429,7 @@ k_wgrad(int H, int W, int B, const bf16* __restrict__ src0, const bf16* __restri
             constexpr int N = decltype(total)::value;
             int t = threadIdx.x;
             // where the accumulators fill the registers, form the addresses here
-            // and not before the loop over the pixels (spilled: 252 us for 243)
+            // and not before the loop over the pixels (spilled: 252 us, 243 so)
             if constexpr (COUT >= 64) asm volatile("" : "+v"(t));
 #pragma unroll
             for (int u0 = 0; u0 < N; u0 += kInFlight * KM_BLOCK) {
@@ -486,23 +488,26 @@ k_wgrad(int H, int W, int B, const bf16* __restrict__ src0, const bf16* __restri
 #pragma unroll
         for (int ch = 0; ch < PX / 32; ++ch) {
             const int p0 = ch * 32 + g * 8;     // this lane's first pixel of the chunk
-            // bit e: pixel e has a neighbour above, below, left, right
-            int up = 0, down = 0, left = 0, right = 0;
+            // bit e of the bytes: pixel e has a neighbour above, below, left, right
+            unsigned has;
             {
                 int i = i0, j = j0 + p0;
                 while (j >= W) {
                     j -= W;
                     if (++i == H) i = 0;
                 }
+                if (__all(j + 8 <= W)) {                // eight pixels of one row
+                    has = (i > 0 ? 0xffu : 0u) | (i < H - 1 ? 0xff00u : 0u) | (j > 0 ? 0xff0000u : 0xfe0000u) |
+                          (j + 8 < W ? 0xff000000u : 0x7f000000u);
+                } else {
+                    has = 0;
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    up |= (i > 0) << e;
-                    down |= (i < H - 1) << e;
-                    left |= (j > 0) << e;
-                    right |= (j < W - 1) << e;
-                    if (++j == W) {
-                        j = 0;
-                        if (++i == H) i = 0;
+                    for (int e = 0; e < 8; ++e) {
+                        has |= ((i > 0) | (i < H - 1) << 8 | (j > 0) << 16 | (unsigned)(j < W - 1) << 24) << e;
+                        if (++j == W) {
+                            j = 0;
+                            if (++i == H) i = 0;
+                        }
                     }
                 }
             }
@@ -516,9 +521,9 @@ k_wgrad(int H, int W, int B, const bf16* __restrict__ src0, const bf16* __restri
             for (int ct = 0; ct < CT; ++ct) {
                 if (ct0 + ct >= NCT) continue;
                 int4 x = load8(xs + off[ct] + p0 * LX, LX);
-                const int in = (tdy[ct] < 0 ? up : tdy[ct] > 0 ? down : 0xff) &
-                               (tdx[ct] < 0 ? left : tdx[ct] > 0 ? right : 0xff);
-                if (__any(in != 0xff)) {
+                const unsigned look = has | past[ct];
+                if (__any(look != ~0u)) {
+                    const unsigned in = look & look >> 8 & look >> 16 & look >> 24;
                     // two pixels per word: a bit of the mask becomes a half word
                     auto two = [in](int e) { return (int)((in >> e & 1) * 0xffffu | (in >> (e + 1) & 1) * 0xffff0000u); };
                     x.x &= two(0);
