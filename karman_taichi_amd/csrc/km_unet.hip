@@ -36,6 +36,7 @@ struct km_net {
     bf16 *X0, *e0, *p1, *e1, *p2, *e2, *p3, *e3, *d2, *d1, *d0;
     bf16 *dy_d0, *dy_d1, *dy_d2, *dy_e3, *dy_e2, *dy_e1, *dy_e0;
     float *z, *q, *ae, *dX0, *dX1, *dX2, *wpart;
+    int cus = 1;                // compute units
     float *c32, *r32;           // FP32 staging of one system (km_unet_apply)
     double *P, *stats, *loss;
     int64_t wpart_n = 0;
@@ -46,7 +47,7 @@ namespace {
 constexpr int E0 = 0, E1 = 1, E2 = 2, E3 = 3, D2 = 4, D1 = 5, D0 = 6;
 constexpr int kMaxBatch = 64;
 constexpr int64_t kPartials = 1 << 20;          // doubles
-constexpr int64_t kWpartMax = (int64_t)16 << 20;  // floats
+constexpr int64_t kWpartMax = (int64_t)32 << 20;  // floats
 
 __host__ __device__ constexpr int round32(int v) { return (v + 31) / 32 * 32; }
 
@@ -350,13 +351,13 @@ k_conv3x3(int H, int W, const bf16* __restrict__ src0, const bf16* __restrict__ 
 // fragment is two transposing LDS reads (each hands a lane four pixels of its
 // channel).  Gathered two bytes at a time in LDS, with divisions for every
 // vector's place, the three decoder layers took 400, 319 and 302 us at that
-// size; now 234, 167 and 118 (78, 109 and 153 TFLOP/s; the FP32 partial sums'
-// 0.5 GB are 90 us of the first).  What bounds it: bringing and multiplying take
-// turns in a workgroup, and two workgroups fit a compute unit.
+// size; now 144, 143 and 118 (126, 127 and 153 TFLOP/s).  What bounds it: bringing
+// and multiplying take turns in a workgroup, and two or three workgroups fit a
+// compute unit.
 // Pixels are taken in linear order (a tap is a shift of dy W + dx); a tap that
 // leaves the image is cleared by each lane's pixel masks (one word for the four
 // directions, formed from the first of the lane's eight pixels: bit by bit the
-// layers above took 243, 180 and 137).  The pixel stride in
+// layers above took 9 to 19 us longer).  The pixel stride in
 // LDS is CIN + 4 values: a quarter wave's reads are 8-byte aligned and its
 // pixels start on different banks.
 constexpr int kWgPx = 64;
@@ -1028,15 +1029,36 @@ void wgrad(km_net* N, int l, int H, int W, int B, const bf16* s0, const bf16* s1
     constexpr int most_ct = 32 / (COUT / 16), CT = (NCT + 3) / 4 < most_ct ? (NCT + 3) / 4 : most_ct;
     const int ncg = (NCT + 4 * CT - 1) / (4 * CT);
     const int64_t npx = (int64_t)B * H * W;
-    // as many splits as keep four workgroups of each column group per compute
-    // unit and the FP32 sums short, within the partial sums' buffer
+    // The longest FP32 sums: those of 4096 workgroups, or of half the buffer.
     int64_t nsplit = (4096 + ncg - 1) / ncg;
     const int64_t cap = kWpartMax / (COUT * KP);
-    if (nsplit > cap) nsplit = cap;
+    if (nsplit > cap / 2) nsplit = cap / 2;
     const int64_t most = (npx + kWgPx - 1) / kWgPx;
     if (nsplit > most) nsplit = most;
     int64_t pps = (npx + nsplit - 1) / nsplit;
     pps = (pps + kWgPx - 1) / kWgPx * kWgPx;
+    // From there down, the pixels per workgroup whose rounds of resident
+    // workgroups take the fewest pixel steps (plus one chunk's for the partial
+    // sums of each round): with 576 the two wide decoder layers at
+    // 4 x 1280 x 256 ran 604 and 569 workgroups on 512 places, two rounds, the
+    // second nearly empty (234 and 167 us); 320 make two full ones (144 and 143).
+    static const int per_cu = [] {
+        int n = 0;
+        const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
+            &n, reinterpret_cast<const void*>(&k_wgrad<MODE, C0, C1, COUT, CT>), KM_BLOCK, 0);
+        return e == hipSuccess && n > 0 ? n : 2;
+    }();
+    const int64_t places = (int64_t)per_cu * N->cus;
+    int64_t least = INT64_MAX;
+    for (int64_t k = pps; k >= kWgPx; k -= kWgPx) {
+        const int64_t parts = (npx + k - 1) / k;
+        if (parts > cap) break;
+        const int64_t steps = (parts * ncg + places - 1) / places * (k + kWgPx);
+        if (steps < least) {
+            least = steps;
+            pps = k;
+        }
+    }
     nsplit = (npx + pps - 1) / pps;
     hipLaunchKernelGGL((k_wgrad<MODE, C0, C1, COUT, CT>), dim3((unsigned)nsplit, (unsigned)ncg), dim3(KM_BLOCK), 0, st,
                        H, W, B, s0, s1, dY, (int)pps, N->wpart);
@@ -1105,6 +1127,9 @@ int alloc(km_ctx* ctx, km_net* N, int B, int NX, int NY) {
         *it.ptr = N->arena + off;
         off += align256(it.bytes);
     }
+    int cus = 0;
+    KM_HIP(ctx, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
+    N->cus = cus > 0 ? cus : 1;
     N->B = B;
     N->NX = NX;
     N->NY = NY;
