@@ -109,7 +109,7 @@ k_prep_weights(const LayerOff* __restrict__ L, int64_t nwf, int64_t nwt, const f
 // one 16-byte LDS read at an offset that a small table gives per K chunk.
 // Before, each wave fetched every fragment from memory for each of the nine
 // taps, with its own index arithmetic.  The layers of a 1280 x 256 system:
-// 116 us now, 200 then; the 192-channel one at 320 x 64 pixels 34 us (133
+// 96 us now, 200 then; the 192-channel one at 320 x 64 pixels 23 us (194
 // TFLOP/s) and 58, the last one at 1280 x 256 pixels 27 and 38.  What bounds it
 // now is filling the patch: one wait for memory per workgroup, and too few
 // workgroups per compute unit (one or two at the coarser levels) to hide it.  The
@@ -130,7 +130,8 @@ k_prep_weights(const LayerOff* __restrict__ L, int64_t nwf, int64_t nwt, const f
 // A lane holds four channels of a pixel of each of its rows, so the 2x2 sum
 // takes its neighbour's registers and no memory.  With both in kernels of their
 // own, and the gradients stored in FP32 in between, the six layers of four
-// samples of 1280 x 256 took 229 + 185 us; now 259.
+// samples of 1280 x 256 took 229 + 185 us; so 259, and 223 with the waves split
+// as now.
 struct FusedOut {
     const float* pw;
     const float* coef;
@@ -1000,10 +1001,14 @@ int flat_blocks(int64_t n) {
     return g < 1 ? 1 : (int)g;
 }
 
-// Waves on the output channels (WR, RTW tiles each) and rows per wave: a
-// fragment from LDS serves RTW products and one from memory Q.  Few pixels
-// (the coarser levels) take fewer rows per workgroup, so that there are
-// several hundred workgroups.
+// Waves on the output channels (WR, RTW tiles each) and rows per wave (Q): a
+// fragment from LDS serves RTW products and one from memory Q, and one fetched
+// from memory is what a wave waits for.  So a wave takes one tile of channels and
+// four rows (two where pooling shrinks the images: more workgroups), and the
+// input gradients, whose 48 to 192 channels would read the patch again, three
+// tiles.  With two tiles and two rows the 192-channel layer took 34 us in an
+// inference at 1280 x 256 (23 now), the 96-channel one 20 (15), the pooled ones
+// 28 (22); over a training pass of four samples those changed took 379 us (285).
 template <int MODE, int C0, int C1, int COUT, int OUTK, int WR, int RTW, int Q, typename T = float>
 void conv(int H, int W, int B, const bf16* s0, const bf16* s1, const bf16* Wm, const float* bias, void* out,
           const int* skip, hipStream_t st, const FusedOut& fo = FusedOut{}) {
@@ -1157,13 +1162,13 @@ void forward(km_net* N, int B, const float* params, const int* skip, hipStream_t
     const bf16* wf = N->wf;
     conv<0, 8, 0, 16, 0, 1, 1, 4>(H, W, B, N->X0, nullptr, wf + L[E0].wf, params + L[E0].b, N->e0, skip, st);
     pool<16>(H1, W1, B, N->e0, N->p1, skip, st);
-    conv<0, 16, 0, 32, 0, 1, 2, 2>(H1, W1, B, N->p1, nullptr, wf + L[E1].wf, params + L[E1].b, N->e1, skip, st);
+    conv<0, 16, 0, 32, 0, 2, 1, 4>(H1, W1, B, N->p1, nullptr, wf + L[E1].wf, params + L[E1].b, N->e1, skip, st);
     pool<32>(H2, W2, B, N->e1, N->p2, skip, st);
-    conv<0, 32, 0, 64, 0, 2, 2, 2>(H2, W2, B, N->p2, nullptr, wf + L[E2].wf, params + L[E2].b, N->e2, skip, st);
+    conv<0, 32, 0, 64, 0, 4, 1, 4>(H2, W2, B, N->p2, nullptr, wf + L[E2].wf, params + L[E2].b, N->e2, skip, st);
     pool<64>(H3, W3, B, N->e2, N->p3, skip, st);
-    conv<0, 64, 0, 128, 0, 2, 2, 1>(H3, W3, B, N->p3, nullptr, wf + L[E3].wf, params + L[E3].b, N->e3, skip, st);
-    conv<1, 128, 64, 64, 0, 2, 2, 2>(H2, W2, B, N->e3, N->e2, wf + L[D2].wf, params + L[D2].b, N->d2, skip, st);
-    conv<1, 64, 32, 32, 0, 1, 2, 2>(H1, W1, B, N->d2, N->e1, wf + L[D1].wf, params + L[D1].b, N->d1, skip, st);
+    conv<0, 64, 0, 128, 0, 4, 1, 4>(H3, W3, B, N->p3, nullptr, wf + L[E3].wf, params + L[E3].b, N->e3, skip, st);
+    conv<1, 128, 64, 64, 0, 4, 1, 4>(H2, W2, B, N->e3, N->e2, wf + L[D2].wf, params + L[D2].b, N->d2, skip, st);
+    conv<1, 64, 32, 32, 0, 2, 1, 4>(H1, W1, B, N->d2, N->e1, wf + L[D1].wf, params + L[D1].b, N->d1, skip, st);
     conv<1, 32, 16, 16, 0, 1, 1, 4>(H, W, B, N->d1, N->e0, wf + L[D0].wf, params + L[D0].b, N->d0, skip, st);
 }
 
@@ -1177,11 +1182,11 @@ void forward_infer(km_net* N, const float* params, const int* skip, hipStream_t 
     const LayerOff* L = N->lay.L;
     const bf16* wf = N->wf;
     conv<0, 8, 0, 16, 0, 1, 1, 4>(H, W, 1, N->X0, nullptr, wf + L[E0].wf, params + L[E0].b, N->e0, skip, st);
-    conv<2, 16, 0, 32, 0, 1, 2, 2>(H1, W1, 1, N->e0, nullptr, wf + L[E1].wf, params + L[E1].b, N->e1, skip, st);
-    conv<2, 32, 0, 64, 0, 2, 2, 2>(H2, W2, 1, N->e1, nullptr, wf + L[E2].wf, params + L[E2].b, N->e2, skip, st);
-    conv<2, 64, 0, 128, 0, 2, 2, 1>(H3, W3, 1, N->e2, nullptr, wf + L[E3].wf, params + L[E3].b, N->e3, skip, st);
-    conv<1, 128, 64, 64, 0, 2, 2, 2>(H2, W2, 1, N->e3, N->e2, wf + L[D2].wf, params + L[D2].b, N->d2, skip, st);
-    conv<1, 64, 32, 32, 0, 1, 2, 2>(H1, W1, 1, N->d2, N->e1, wf + L[D1].wf, params + L[D1].b, N->d1, skip, st);
+    conv<2, 16, 0, 32, 0, 2, 1, 2>(H1, W1, 1, N->e0, nullptr, wf + L[E1].wf, params + L[E1].b, N->e1, skip, st);
+    conv<2, 32, 0, 64, 0, 4, 1, 2>(H2, W2, 1, N->e1, nullptr, wf + L[E2].wf, params + L[E2].b, N->e2, skip, st);
+    conv<2, 64, 0, 128, 0, 4, 1, 2>(H3, W3, 1, N->e2, nullptr, wf + L[E3].wf, params + L[E3].b, N->e3, skip, st);
+    conv<1, 128, 64, 64, 0, 4, 1, 4>(H2, W2, 1, N->e3, N->e2, wf + L[D2].wf, params + L[D2].b, N->d2, skip, st);
+    conv<1, 64, 32, 32, 0, 2, 1, 4>(H1, W1, 1, N->d2, N->e1, wf + L[D1].wf, params + L[D1].b, N->d1, skip, st);
     const FusedOut fo{params + N->lay.out_w, coef, (const double*)N->stats, NX, NY, accum};
     conv<1, 32, 16, 16, 2, 1, 1, 4, T>(H, W, 1, N->d1, N->e0, wf + L[D0].wf, params + L[D0].b, z, skip, st, fo);
 }
@@ -1200,11 +1205,11 @@ void backward(km_net* N, int B, float* grad, hipStream_t st) {
     };
     // d0: input [up(d1) | e0]
     wgrad<1, 32, 16, 16>(N, D0, H, W, B, N->d1, N->e0, N->dy_d0, grad, st);
-    conv<0, 16, 0, 48, 1, 1, 3, 2>(H, W, B, N->dy_d0, nullptr, wt + L[D0].wt, nullptr, N->dy_d1, nullptr, st,
+    conv<0, 16, 0, 48, 1, 1, 3, 4>(H, W, B, N->dy_d0, nullptr, wt + L[D0].wt, nullptr, N->dy_d1, nullptr, st,
                                    grad_out(N->d1, N->dX0));
     // d1: input [up(d2) | e1]
     wgrad<1, 64, 32, 32>(N, D1, H1, W1, B, N->d2, N->e1, N->dy_d1, grad, st);
-    conv<0, 32, 0, 96, 1, 2, 3, 2>(H1, W1, B, N->dy_d1, nullptr, wt + L[D1].wt, nullptr, N->dy_d2, nullptr, st,
+    conv<0, 32, 0, 96, 1, 2, 3, 4>(H1, W1, B, N->dy_d1, nullptr, wt + L[D1].wt, nullptr, N->dy_d2, nullptr, st,
                                    grad_out(N->d2, N->dX1));
     // d2: input [up(e3) | e2]
     wgrad<1, 128, 64, 64>(N, D2, H2, W2, B, N->e3, N->e2, N->dy_d2, grad, st);
@@ -1212,11 +1217,11 @@ void backward(km_net* N, int B, float* grad, hipStream_t st) {
                                     grad_out(N->e3, N->dX2));
     // e3: input p3
     wgrad<0, 64, 0, 128>(N, E3, H3, W3, B, N->p3, nullptr, N->dy_e3, grad, st);
-    conv<0, 128, 0, 64, 3, 2, 2, 2>(H3, W3, B, N->dy_e3, nullptr, wt + L[E3].wt, nullptr, N->dy_e2, nullptr, st,
+    conv<0, 128, 0, 64, 3, 4, 1, 2>(H3, W3, B, N->dy_e3, nullptr, wt + L[E3].wt, nullptr, N->dy_e2, nullptr, st,
                                     grad_out(N->e2, N->dX2));
     // e2: input p2
     wgrad<0, 32, 0, 64>(N, E2, H2, W2, B, N->p2, nullptr, N->dy_e2, grad, st);
-    conv<0, 64, 0, 32, 3, 1, 2, 2>(H2, W2, B, N->dy_e2, nullptr, wt + L[E2].wt, nullptr, N->dy_e1, nullptr, st,
+    conv<0, 64, 0, 32, 3, 2, 1, 4>(H2, W2, B, N->dy_e2, nullptr, wt + L[E2].wt, nullptr, N->dy_e1, nullptr, st,
                                    grad_out(N->e1, N->dX1));
     // e1: input p1
     wgrad<0, 16, 0, 32>(N, E1, H1, W1, B, N->p1, nullptr, N->dy_e1, grad, st);
