@@ -158,8 +158,8 @@ int km_bicgstab(km_ctx* ctx, int NX, int NY, const double* coef, const double* b
  * KM_FLAG_SMOOTH and no network) run a whole solve as one launch of at most one
  * workgroup per compute unit where the system's tiles fit the GPU, its boundary
  * rows and columns are empty and no tile was set by the caller; other systems,
- * and a launch that could not get all its workgroups resident within two
- * seconds, are solved by launches.  The results do not depend on what else runs.
+ * and a launch that got no memory for its exchange words or could not get all
+ * its workgroups resident within two seconds, are solved by launches.  The results do not depend on what else runs.
  * Launches of this kind wait for one another on a device. */
 /* km_bicgstab without any allocation: no counterpart in the reference.  For
  * callers that cannot allocate device memory (code under stream capture, tight

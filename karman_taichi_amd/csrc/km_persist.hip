@@ -1237,9 +1237,10 @@ int ensure(km_ctx* ctx) {
     }
     if (e == hipSuccess) e = hipMemsetAsync(q, 0, kWords, ctx->stream);
     if (e != hipSuccess) {
+        (void)hipGetLastError();     // not the caller's error: the solve runs by launches
         if (q) (void)hipFree(q);
         delete K;
-        return km_fail(ctx, KM_ENOMEM, "exchange buffers: %s", hipGetErrorString(e));
+        return KM_ENOMEM;
     }
     char* a = K->arena = static_cast<char*>(q);
     K->flags = reinterpret_cast<unsigned*>(a);
@@ -1374,7 +1375,10 @@ bool fits_smooth(km_ctx* ctx, int NX, int NY, int* shape) {
 template <typename T>
 int twolevel(km_ctx* ctx, int shape, int NX, int NY, const double* coef, const T* rhs, T* xd, T* ws, double eps,
              int max_iter, KState* out, const std::function<int()>* tail, bool* ran) {
-    if (int rc = ensure(ctx)) return rc;
+    if (int rc = ensure(ctx)) {
+        *ran = false;
+        return rc == KM_ENOMEM ? KM_OK : rc;
+    }
     const km_coarse* C = ctx->coarse;
     km_persist* K = ctx->persist;
     PSys<T> s = system<T>(ctx, 0, shape, NX, NY, coef, rhs, xd, ws, eps, max_iter, kmcoarse::kOmega);
@@ -1414,7 +1418,10 @@ template <typename T>
 int smooth(km_ctx* ctx, int nsys, const int* NX, const int* NY, const T* const* coef, const T* const* rhs,
            T* const* xd, T* const* ws, double eps, const int* max_iter, int sweeps, KState* out,
            const std::function<int()>* tail, bool* ran) {
-    if (int rc = ensure(ctx)) return rc;
+    if (int rc = ensure(ctx)) {
+        *ran = false;
+        return rc == KM_ENOMEM ? KM_OK : rc;
+    }
     PSys<T> s[2] = {};
     int shape[2] = {0, 0};
     for (int q = 0; q < nsys; ++q) {
@@ -1490,7 +1497,10 @@ int plain(km_ctx* ctx, int shape, bool cg, int NX, int NY, const double* coef, c
         for (int k = 0; k < 3; ++k)
             s.part[k] = reinterpret_cast<double*>(w + kFlagBytes + 256) + (size_t)k * kMaxWg * 2;
     } else {
-        if (int rc = ensure(ctx)) return rc;
+        if (int rc = ensure(ctx)) {
+            *ran = false;
+            return rc == KM_ENOMEM ? KM_OK : rc;
+        }
         K = ctx->persist;
         s.flags = K->flags;
         s.abort = K->abort;
