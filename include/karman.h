@@ -72,8 +72,10 @@ extern "C" {
                                * Results are undefined for a system that is not (no counterpart in the reference) */
 #define KM_FLAG_TRUE 32       /* km_bicgstab: after the reference's stop on the recursive residual, check the true
                                * residual ||b - A x|| / ||b|| and restart from x (r = b - A x) while it is above eps
-                               * and each restart at least halves it (at most 8 restarts; no counterpart in the
-                               * reference, which stops on the recursive residual, bicgsolver.py:128-131) */
+                               * and each restart at least halves it (at most 8 restarts; one that ends between eps
+                               * and 2 eps without halving it is followed by one to eps / 2).  The status is KM_OK
+                               * whenever the true residual ends below eps.  No counterpart in the reference, which
+                               * stops on the recursive residual (bicgsolver.py:128-131) */
 
 /* east boundary kinds */
 #define KM_EAST_WALL 0        /* simple.py:184-186, :214-216 (with the bicgsimp.py:196 fix) */

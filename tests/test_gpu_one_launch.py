@@ -121,3 +121,38 @@ def test_plain_one_launch_matches_direct_solution(NX, NY, entry, dev):
     assert info.status == _lib.KM_OK
     assert info.rel_resid_true < 10 * EPS
     assert err <= 1e5 * EPS
+
+
+@pytest.mark.parametrize("entry", ["km_bicgstab", "km_bicgstab_noalloc"])
+@pytest.mark.parametrize("launches", [False, True])
+def test_true_residual_decides_the_status(entry, launches, dev):
+    """KM_FLAG_TRUE from a start far off: x0 of 1e7 leaves a true residual that
+    the recursive one has drifted from, so restarts follow.  Wherever max_iter
+    cuts them, a true residual below eps is KM_OK."""
+    NX, NY = 50, 71
+    coef, b = system(NX, NY, 5, 0.01)
+    c, bt = torch.tensor(coef, device=dev), torch.tensor(b, device=dev)
+    x0 = torch.zeros_like(bt)
+    x0[1:-1, 1:-1] = 1e7 * torch.tensor(np.random.default_rng(1).standard_normal((NX - 2, NY - 2)), device=dev)
+    ctx = _lib.Context(torch.cuda.current_device(), torch.cuda.current_stream(dev).cuda_stream)
+
+    def run(max_iter):
+        x, info = x0.clone(), KmSolveInfo()
+        ctx.call(entry, NX, NY, ctypes.c_void_p(c.data_ptr()), ctypes.c_void_p(bt.data_ptr()),
+                 ctypes.c_void_p(x.data_ptr()), EPS, max_iter, _lib.KM_FLAG_X0 | _lib.KM_FLAG_TRUE, ctypes.byref(info))
+        torch.cuda.synchronize()
+        return info
+
+    try:
+        if launches:
+            ctx.call("km_set_tile", NX, NY, 0, 8, 32)
+        whole = run(0)
+        print(f"{whole.iterations} it, {whole.refinements} restarts, true residual {whole.rel_resid_true:.1e}")
+        assert whole.status == _lib.KM_OK and whole.rel_resid_true < EPS and whole.refinements >= 1
+        for cap in range(whole.iterations, whole.iterations // 2, -1):
+            info = run(cap)
+            print(f"  cap {cap}: {info.iterations} it, {info.refinements} restarts, status {info.status}, "
+                  f"{info.rel_resid_true:.2e}")
+            assert info.status == _lib.KM_OK or info.rel_resid_true >= EPS, cap
+    finally:
+        ctx.close()
