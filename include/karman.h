@@ -163,6 +163,14 @@ int km_bicgstab(km_ctx* ctx, int NX, int NY, const double* coef, const double* b
  * and a launch that got no memory for its exchange words or could not get all
  * its workgroups resident within two seconds, are solved by launches.  The results do not depend on what else runs.
  * Launches of this kind wait for one another on a device. */
+/* How many solves of this context ran in one launch, how many such launches
+ * refused their system (a boundary row that is not empty), and how many gave
+ * up waiting; any pointer may be null. */
+int km_one_launch_counts(const km_ctx* ctx, int64_t* run, int64_t* refused, int64_t* gave_up);
+/* For tests of the way back: the next n such launches of this context find
+ * that a wait has run into its limit, leave at their first exchange and are
+ * solved by launches (a solve of one workgroup has no exchange). */
+int km_one_launch_give_up(km_ctx* ctx, int n);
 /* km_bicgstab without any allocation: no counterpart in the reference.  For
  * callers that cannot allocate device memory (code under stream capture, tight
  * serving loops, harnesses that forbid hipMalloc).  The same plain BiCGSTAB

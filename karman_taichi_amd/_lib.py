@@ -86,6 +86,8 @@ SIGNATURES = {
     "km_bicgstab": [_CTX, _I, _I, _P, _P, _P, _D, _I, _I, _INFO],
     "km_bicgstab_noalloc": [_CTX, _I, _I, _P, _P, _P, _D, _I, _I, _INFO],
     "km_cg": [_CTX, _I, _I, _P, _P, _P, _D, _I, _I, _INFO],
+    "km_one_launch_counts": [_CTX] + [ctypes.POINTER(ctypes.c_int64)] * 3,
+    "km_one_launch_give_up": [_CTX, _I],
     "km_time_kernel": [_CTX, _I, _I, _I, _P, _P, _I, ctypes.POINTER(_D)],
     "km_unet_param_count": [ctypes.POINTER(ctypes.c_int64)],
     "km_unet_apply": [_CTX, _P, _I, _I, _P, _P, _P],

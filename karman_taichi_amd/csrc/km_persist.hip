@@ -296,7 +296,9 @@ __device__ __forceinline__ void solve_body(const PSys<T>& s, int L) {
     const int ta = L / s.tiles_j, tb = L - ta * s.tiles_j;
     const int ti0 = 1 + ta * TI, tj0 = 1 + tb * TJ;
     unsigned round = s.round;
-    if (t == 0) bad = 0;
+    // raised before this launch (by the one before it, say): leave at the first
+    // round instead of waiting too
+    if (t == 0) bad = (int)get(s.abort);
 
     // boundary cells of the system next to this tile: x = 0, and their rows
     // must be empty (checked: otherwise the launch gives up)
@@ -926,7 +928,7 @@ __global__ void __launch_bounds__(NT) k_plain(PPlain s) {
     const int ta = L / s.tiles_j, tb = L - ta * s.tiles_j;
     const int ti0 = 1 + ta * TI, tj0 = 1 + tb * TJ;
     unsigned round = s.round;
-    if (t == 0) bad = 0;
+    if (t == 0) bad = (int)get(s.abort);
     for (int k = t; k < (TI + 2) * W; k += NT) z[k] = 0.0;
     // boundary rows must be empty (see solve_body)
     const int j0 = tb == 0 ? 0 : tj0, j1 = tj0 + TJ > ny ? NY : tj0 + TJ;
@@ -1216,6 +1218,14 @@ int compute_units(km_ctx* ctx) {
 constexpr size_t kFlagBytes = (size_t)2 * kMaxWg * kFlagStride * sizeof(unsigned);
 constexpr size_t kWords = kFlagBytes + 256 + (size_t)4 * kMaxM * sizeof(uint64_t);
 
+// km_one_launch_give_up: this launch finds its abort word raised.
+int raise_abort(km_ctx* ctx, unsigned* abort) {
+    if (ctx->one_raise <= 0) return KM_OK;
+    ctx->one_raise--;
+    KM_HIP(ctx, hipMemsetAsync(abort, 1, sizeof(unsigned), ctx->stream));
+    return KM_OK;
+}
+
 int ensure(km_ctx* ctx) {
     if (km_persist* K = ctx->persist) {
         if (!K->clean || K->round > 0xe0000000u) {
@@ -1223,7 +1233,7 @@ int ensure(km_ctx* ctx) {
             K->round = 0;
         }
         K->clean = false;   // until the launch has ended well
-        return KM_OK;
+        return raise_abort(ctx, K->abort);
     }
     km_persist* K = new km_persist();
     const size_t pt = (size_t)4 * kMaxWg * 4 * sizeof(double);
@@ -1249,7 +1259,7 @@ int ensure(km_ctx* ctx) {
     K->part = reinterpret_cast<double*>(a + kWords);
     K->rc = reinterpret_cast<double*>(a + kWords + pt);
     ctx->persist = K;
-    return KM_OK;
+    return raise_abort(ctx, K->abort);
 }
 
 template <typename T>
@@ -1309,8 +1319,10 @@ int finish(km_ctx* ctx, int nsys, const std::function<void()>& launch, KState* o
     if (aborted) {
         *ran = false;
         if (K) K->off++;
+        ctx->one_count[2]++;
         return KM_OK;
     }
+    ctx->one_count[*ran ? 0 : 1] += nsys;
     int most = 0;
     for (int q = 0; q < nsys; ++q) most = std::max(most, out[q].iter);
     if (K) {
@@ -1494,6 +1506,7 @@ int plain(km_ctx* ctx, int shape, bool cg, int NX, int NY, const double* coef, c
         KM_HIP(ctx, hipMemsetAsync(w, 0, kFlagBytes + 256, ctx->stream));
         s.flags = reinterpret_cast<unsigned*>(w);
         s.abort = reinterpret_cast<unsigned*>(w + kFlagBytes);
+        if (int rc = raise_abort(ctx, s.abort)) return rc;
         for (int k = 0; k < 3; ++k)
             s.part[k] = reinterpret_cast<double*>(w + kFlagBytes + 256) + (size_t)k * kMaxWg * 2;
     } else {
@@ -1557,3 +1570,22 @@ void km_persist_free(km_ctx* ctx) {
     delete ctx->persist;
     ctx->persist = nullptr;
 }
+
+extern "C" {
+
+int km_one_launch_counts(const km_ctx* ctx, int64_t* run, int64_t* refused, int64_t* gave_up) {
+    if (!ctx) return KM_EINVAL;
+    if (run) *run = ctx->one_count[0];
+    if (refused) *refused = ctx->one_count[1];
+    if (gave_up) *gave_up = ctx->one_count[2];
+    return KM_OK;
+}
+
+int km_one_launch_give_up(km_ctx* ctx, int n) {
+    if (!ctx) return KM_EINVAL;
+    KM_REQUIRE(ctx, n >= 0, "%d launches", n);
+    ctx->one_raise = n;
+    return KM_OK;
+}
+
+}  // extern "C"
