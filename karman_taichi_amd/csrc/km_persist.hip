@@ -54,7 +54,6 @@ struct km_persist {
     double* rc = nullptr;        // [2][kMaxSlots][kMaxM] restriction pieces of P^T v, P^T t
     unsigned round = 0;          // the last round's number
     bool clean = false;          // flags and Y hold numbers up to ``round`` only
-    int off = 0;                 // launches that ran into the limit: the path closes after two
 };
 
 namespace {
@@ -1318,7 +1317,6 @@ int finish(km_ctx* ctx, int nsys, const std::function<void()>& launch, KState* o
     }
     if (aborted) {
         *ran = false;
-        if (K) K->off++;
         ctx->one_count[2]++;
         return KM_OK;
     }
@@ -1345,8 +1343,12 @@ namespace kmpersist {
 // iteration against 72), 1.2x at 1999 x 401, and 2.5x for the momentum solves.
 constexpr int kMaxSide = 1300;
 
+// Two launches that waited out their limit, of any entry: something holds the
+// compute units, and each further try would cost two seconds.
+bool closed(const km_ctx* ctx) { return ctx->one_count[2] >= 2; }
+
 bool fits_twolevel(km_ctx* ctx, const km_coarse* C, int NX, int NY, int* shape) {
-    if (!C || C->m > kMaxM || (ctx->persist && ctx->persist->off >= 2)) return false;
+    if (!C || C->m > kMaxM || closed(ctx)) return false;
     const int cus = std::min(kMaxWg, compute_units(ctx));
     const int nx = NX - 2, ny = NY - 2;
     if (nx > kMaxSide || ny > kMaxSide) return false;
@@ -1370,7 +1372,7 @@ bool fits_twolevel(km_ctx* ctx, const km_coarse* C, int NX, int NY, int* shape) 
 constexpr int kHalfShapes = 4;
 
 bool fits_smooth(km_ctx* ctx, int NX, int NY, int* shape) {
-    if ((ctx->persist && ctx->persist->off >= 2) || std::max(NX, NY) - 2 > kMaxSide + 1) return false;
+    if (closed(ctx) || std::max(NX, NY) - 2 > kMaxSide + 1) return false;
     const int cus = std::min(kMaxWg, compute_units(ctx));
     for (int half = 1; half >= 0; --half)
         for (int k = 0; k < (half ? kHalfShapes : kNumShapes); ++k) {
@@ -1479,7 +1481,7 @@ int gate(int device) {
 // against 16 by launches), else the smallest tiles that number at most one per
 // compute unit.  A tile chosen by km_set_tile asks for the launches.
 bool fits_plain(km_ctx* ctx, int NX, int NY, int* shape) {
-    if ((ctx->persist && ctx->persist->off >= 2) || NX < 3 || NY < 3 ||
+    if (closed(ctx) || NX < 3 || NY < 3 ||
         ctx->tile_override.count(std::make_tuple(NX, NY, KM_F64)))
         return false;
     const int cus = std::min(kMaxWg, compute_units(ctx));

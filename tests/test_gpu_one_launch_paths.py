@@ -116,7 +116,8 @@ def test_plain_shapes_take_one_launch(NX, NY, run, entry, dev):
         assert (counts[0] > 0) == bool(run)
 
 
-ENTRIES = ["km_bicgstab", "km_cg", "from_x", "coarse", "coarse_mixed", "smooth", "smooth_mixed", "pair", "group"]
+ENTRIES = ["km_bicgstab", "km_cg", "km_bicgstab_noalloc", "from_x", "coarse", "coarse_mixed", "smooth", "smooth_mixed", "pair",
+           "group"]
 
 
 @pytest.mark.parametrize("entry", ENTRIES)
@@ -139,3 +140,14 @@ def test_a_launch_that_gives_up_is_solved_by_launches(entry, dev):
         assert closed[1:] == (0, 2)
         s.solve(entry, coef, b)
         assert s.counts() == closed
+
+
+def test_give_ups_of_all_entries_count_together(dev):
+    coef, b = system(100, 71, 9, 0.5)
+    with Solver(dev) as s:
+        s.ctx.call("km_one_launch_give_up", 2)
+        s.solve("km_bicgstab_noalloc", coef, b)
+        s.solve("smooth", coef, b)
+        for entry in ENTRIES:
+            s.solve(entry, coef, b)
+        assert s.counts() == (0, 0, 2)
