@@ -163,9 +163,10 @@ int km_bicgstab(km_ctx* ctx, int NX, int NY, const double* coef, const double* b
  * and a launch that got no memory for its exchange words or could not get all
  * its workgroups resident within two seconds, are solved by launches.  The results do not depend on what else runs.
  * Launches of this kind wait for one another on a device. */
-/* How many solves of this context ran in one launch, how many such launches
- * refused their system (a boundary row that is not empty), and how many gave
- * up waiting; any pointer may be null. */
+/* How many solves of this context ran in one launch, how many were refused by
+ * theirs (a boundary row that is not empty: the context's next 31 solves of
+ * that kind and size go to the launches directly), and how many such launches
+ * gave up waiting; any pointer may be null. */
 int km_one_launch_counts(const km_ctx* ctx, int64_t* run, int64_t* refused, int64_t* gave_up);
 /* For tests of the way back: the next n such launches of this context find
  * that a wait has run into its limit, leave at their first exchange and are

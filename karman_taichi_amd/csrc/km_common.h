@@ -159,6 +159,7 @@ struct km_ctx {
     void* scratch = nullptr;       // device address of this device's no-allocation scratch array
     km_persist* persist = nullptr; // exchange buffers of the one-launch solves
     int64_t one_count[3] = {};     // one-launch solves: run, refused, given up (km_one_launch_counts; two close the path)
+    std::map<std::tuple<int, int, int>, int> one_rest;   // (family, NX, NY) refused -> solves until it is tried again
     int one_raise = 0;             // km_one_launch_give_up: launches still to find the abort word raised
     km_mg* mg = nullptr;           // V-cycle hierarchy (KM_FLAG_MG)
 };

@@ -1288,8 +1288,32 @@ PSys<T> system(km_ctx* ctx, int slot, int shape, int NX, int NY, const void* c, 
     return s;
 }
 
+// A refused system costs its launch, the tail behind it and a wait before its
+// solve by launches begins (24 to 41 us on solves of 190 to 370 us, 34 x 34 to
+// 515 x 130 cells), and a program that writes identity rows on the rim of its
+// systems does so every time.  So a size that was refused rests: its next kRest
+// solves of that family go straight to the launches (100 x 71 cells 336 us
+// with plain BiCGSTAB against 362, 236 with the coarse level against 266), then one
+// is tried again (a program may have several kinds of systems of one size).
+// Only the path is chosen by it: the kernel checks every system it is given.
+enum Family { kPlainFamily, kTwoLevelFamily, kSmoothFamily };
+constexpr int kRest = 31;
+
+void refused(km_ctx* ctx, Family f, int NX, int NY) {
+    if (ctx->one_rest.size() >= 64) ctx->one_rest.clear();
+    ctx->one_rest[std::make_tuple((int)f, NX, NY)] = kRest;
+}
+
+bool rests(km_ctx* ctx, Family f, int NX, int NY) {
+    const auto it = ctx->one_rest.find(std::make_tuple((int)f, NX, NY));
+    if (it == ctx->one_rest.end()) return false;
+    if (it->second-- > 0) return true;
+    ctx->one_rest.erase(it);
+    return false;
+}
+
 // Launch, the tail, and the final states; *ran = false if it gave up.
-int finish(km_ctx* ctx, int nsys, const std::function<void()>& launch, KState* out, const std::function<int()>* tail,
+int finish(km_ctx* ctx, Family fam, int nsys, const int* NX, const int* NY, const std::function<void()>& launch, KState* out, const std::function<int()>* tail,
            bool* ran, km_persist* K, int rounds) {
     volatile int* hf = ctx->h_flag;
     for (int q = 0; q < nsys; ++q)
@@ -1314,6 +1338,7 @@ int finish(km_ctx* ctx, int nsys, const std::function<void()>& launch, KState* o
         aborted = aborted || w[3];
         if (!f.done) return km_fail(ctx, KM_EHIP, "solver stopped without reporting completion");
         if (f.status >= kUnsupported) *ran = false;
+        if (f.status == kUnsupported) refused(ctx, fam, NX[q], NY[q]);
     }
     if (aborted) {
         *ran = false;
@@ -1348,7 +1373,7 @@ constexpr int kMaxSide = 1300;
 bool closed(const km_ctx* ctx) { return ctx->one_count[2] >= 2; }
 
 bool fits_twolevel(km_ctx* ctx, const km_coarse* C, int NX, int NY, int* shape) {
-    if (!C || C->m > kMaxM || closed(ctx)) return false;
+    if (!C || C->m > kMaxM || closed(ctx) || rests(ctx, kTwoLevelFamily, NX, NY)) return false;
     const int cus = std::min(kMaxWg, compute_units(ctx));
     const int nx = NX - 2, ny = NY - 2;
     if (nx > kMaxSide || ny > kMaxSide) return false;
@@ -1371,8 +1396,8 @@ bool fits_twolevel(km_ctx* ctx, const km_coarse* C, int NX, int NY, int* shape) 
 // looks at one system only: a pair's results are those of two solves.
 constexpr int kHalfShapes = 4;
 
-bool fits_smooth(km_ctx* ctx, int NX, int NY, int* shape) {
-    if (closed(ctx) || std::max(NX, NY) - 2 > kMaxSide + 1) return false;
+bool smooth_shape(km_ctx* ctx, int NX, int NY, int* shape) {
+    if (std::max(NX, NY) - 2 > kMaxSide + 1) return false;
     const int cus = std::min(kMaxWg, compute_units(ctx));
     for (int half = 1; half >= 0; --half)
         for (int k = 0; k < (half ? kHalfShapes : kNumShapes); ++k) {
@@ -1382,6 +1407,10 @@ bool fits_smooth(km_ctx* ctx, int NX, int NY, int* shape) {
             return true;
         }
     return false;
+}
+
+bool fits_smooth(km_ctx* ctx, int NX, int NY, int* shape) {
+    return !closed(ctx) && !rests(ctx, kSmoothFamily, NX, NY) && smooth_shape(ctx, NX, NY, shape);
 }
 
 #define KM_SHAPES(X) X(0) X(1) X(2) X(3) X(4) X(5) X(6)
@@ -1425,7 +1454,7 @@ int twolevel(km_ctx* ctx, int shape, int NX, int NY, const double* coef, const T
 #undef KM_CASE
         }
     };
-    return finish(ctx, 1, launch, out, tail, ran, K, 2);
+    return finish(ctx, kTwoLevelFamily, 1, &NX, &NY, launch, out, tail, ran, K, 2);
 }
 
 template <typename T>
@@ -1439,7 +1468,7 @@ int smooth(km_ctx* ctx, int nsys, const int* NX, const int* NY, const T* const* 
     PSys<T> s[2] = {};
     int shape[2] = {0, 0};
     for (int q = 0; q < nsys; ++q) {
-        KM_REQUIRE(ctx, fits_smooth(ctx, NX[q], NY[q], &shape[q]), "system %d does not fit one launch", q);
+        KM_REQUIRE(ctx, smooth_shape(ctx, NX[q], NY[q], &shape[q]), "system %d does not fit one launch", q);
         s[q] = system<T>(ctx, q, shape[q], NX[q], NY[q], coef[q], rhs[q], xd[q], ws[q], eps, max_iter[q], 1.0);
     }
     const bool together = nsys == 2 && shape[0] == shape[1] && s[0].G + s[1].G <= std::min(kMaxWg, compute_units(ctx));
@@ -1466,7 +1495,7 @@ int smooth(km_ctx* ctx, int nsys, const int* NX, const int* NY, const T* const* 
             for (int q = 0; q < nsys; ++q) one(shape[q], s[q], none);
         }
     };
-    return finish(ctx, nsys, launch, out, tail, ran, ctx->persist, 2);
+    return finish(ctx, kSmoothFamily, nsys, NX, NY, launch, out, tail, ran, ctx->persist, 2);
 }
 
 int gate(int device) {
@@ -1481,8 +1510,8 @@ int gate(int device) {
 // against 16 by launches), else the smallest tiles that number at most one per
 // compute unit.  A tile chosen by km_set_tile asks for the launches.
 bool fits_plain(km_ctx* ctx, int NX, int NY, int* shape) {
-    if (closed(ctx) || NX < 3 || NY < 3 ||
-        ctx->tile_override.count(std::make_tuple(NX, NY, KM_F64)))
+    if (closed(ctx) || NX < 3 || NY < 3 || ctx->tile_override.count(std::make_tuple(NX, NY, KM_F64)) ||
+        rests(ctx, kPlainFamily, NX, NY))
         return false;
     const int cus = std::min(kMaxWg, compute_units(ctx));
     for (int one = 1; one >= 0; --one)
@@ -1549,7 +1578,7 @@ int plain(km_ctx* ctx, int shape, bool cg, int NX, int NY, const double* coef, c
 #undef KM_CASE
         }
     };
-    return finish(ctx, 1, launch, out, tail, ran, K, 3);
+    return finish(ctx, kPlainFamily, 1, &NX, &NY, launch, out, tail, ran, K, 3);
 }
 
 template int twolevel<double>(km_ctx*, int, int, int, const double*, const double*, double*, double*, double, int,

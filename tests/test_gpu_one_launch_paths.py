@@ -116,8 +116,8 @@ def test_plain_shapes_take_one_launch(NX, NY, run, entry, dev):
         assert (counts[0] > 0) == bool(run)
 
 
-ENTRIES = ["km_bicgstab", "km_cg", "km_bicgstab_noalloc", "from_x", "coarse", "coarse_mixed", "smooth", "smooth_mixed", "pair",
-           "group"]
+ENTRIES = ["km_bicgstab", "km_cg", "km_bicgstab_noalloc", "from_x", "coarse", "coarse_mixed", "smooth",
+           "smooth_mixed", "pair", "group"]
 
 
 @pytest.mark.parametrize("entry", ENTRIES)
@@ -151,3 +151,31 @@ def test_give_ups_of_all_entries_count_together(dev):
         for entry in ENTRIES:
             s.solve(entry, coef, b)
         assert s.counts() == (0, 0, 2)
+
+
+def with_rim(coef, b):
+    """The same system with a coupled identity row on the rim."""
+    coef, b = coef.copy(), b.copy()
+    coef[0, 0, 5], b[0, 5] = 2.0, 1.0
+    return coef, b
+
+
+@pytest.mark.parametrize("entry", ENTRIES)
+def test_a_refused_size_rests(entry, dev):
+    """A program whose systems have identity rows on the rim pays for one
+    refusal in 32 solves, and every system is solved whichever path it takes."""
+    coef, b = system(100, 71, 9, 0.5)
+    with Solver(dev) as s:
+        s.solve(entry, *with_rim(coef, b))
+        first = s.counts()
+        assert first[0] == first[2] == 0 and first[1] in (1, 2)
+        for _ in range(3):
+            s.solve(entry, *with_rim(coef, b))
+            s.solve(entry, coef, b)
+        assert s.counts() == first
+        s.solve(entry, *system(90, 71, 9, 0.5))          # another size does not rest
+        assert s.counts()[0] > 0 and s.counts()[1] == first[1]
+        run = s.counts()[0]
+        for _ in range(40):
+            s.solve(entry, coef, b)
+        assert s.counts()[0] > run and s.counts()[1] == first[1]
