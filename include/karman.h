@@ -159,10 +159,14 @@ int km_bicgstab(km_ctx* ctx, int NX, int NY, const double* coef, const double* b
 /* One launch: km_bicgstab, km_cg and km_fbicgstab (with KM_FLAG_COARSE or
  * KM_FLAG_SMOOTH and no network) run a whole solve as one launch of at most one
  * workgroup per compute unit where the system's tiles fit the GPU, its boundary
- * rows and columns are empty and no tile was set by the caller; other systems,
- * and a launch that got no memory for its exchange words or could not get all
- * its workgroups resident within two seconds, are solved by launches.  The results do not depend on what else runs.
- * Launches of this kind wait for one another on a device. */
+ * rows and columns are empty and no tile was set by the caller.  Other systems
+ * are solved by launches, and so are those whose launch got no memory for its
+ * exchange words or gave up because not all its workgroups were resident
+ * within two seconds (another process holds compute units); after two that
+ * gave up the context solves by launches only.  Solves by launches add their
+ * sums in another order: they stop at the same tolerance, with other rounding.
+ * Launches of this kind wait for one another on a device, whichever context or
+ * stream of the process they come from. */
 /* How many solves of this context ran in one launch, how many were refused by
  * theirs (a boundary row that is not empty: the context's next 31 solves of
  * that kind and size go to the launches directly), and how many such launches
