@@ -35,7 +35,8 @@ struct km_net {
     bf16 *wf = nullptr, *wt = nullptr;
     bf16 *X0, *e0, *p1, *e1, *p2, *e2, *p3, *e3, *d2, *d1, *d0;
     bf16 *dy_d0, *dy_d1, *dy_d2, *dy_e3, *dy_e2, *dy_e1, *dy_e0;
-    float *z, *q, *ae, *dX0, *dX1, *dX2, *wpart;
+    float *z, *q, *ae, *dX0, *dX1, *dX2;
+    float* wpart = nullptr;     // partial sums of the weight gradients (from the first training pass on)
     int cus = 1;                // compute units
     float *c32, *r32;           // FP32 staging of one system (km_unet_apply)
     double *P, *stats, *loss;
@@ -1101,7 +1102,6 @@ int alloc(km_ctx* ctx, km_net* N, int B, int NX, int NY) {
         {(void**)&M.dy_e0, B * hw0 * 16 * bb},
         {(void**)&M.z, B * n * fb},          {(void**)&M.q, B * n * fb},          {(void**)&M.ae, B * n * fb},
         {(void**)&M.dX0, B * hw0 * 16 * fb}, {(void**)&M.dX1, B * hw1 * 32 * fb}, {(void**)&M.dX2, B * hw2 * 64 * fb},
-        {(void**)&M.wpart, kWpartMax * fb},
         {(void**)&M.c32, 5 * n * fb},        {(void**)&M.r32, n * fb},
         {(void**)&M.P, kPartials * sizeof(double)}, {(void**)&M.stats, kMaxBatch * 8 * sizeof(double)},
         {(void**)&M.loss, kMaxBatch * sizeof(double)},
@@ -1144,6 +1144,21 @@ int alloc(km_ctx* ctx, km_net* N, int B, int NX, int NY) {
     N->Gs = (int)(gs > 1024 ? 1024 : gs);
     KM_HIP_SYNC(ctx, hipMemcpy(N->dL, N->lay.L, sizeof(LayerOff) * NL, hipMemcpyHostToDevice));
     KM_HIP_SYNC(ctx, hipMemset(N->stats, 0, kMaxBatch * 8 * sizeof(double)));
+    return KM_OK;
+}
+
+// The partial sums' 128 MB: for contexts that train, of whatever sizes.
+int alloc_wpart(km_ctx* ctx, km_net* N) {
+    if (N->wpart) return KM_OK;
+    const size_t bytes = kWpartMax * sizeof(float);
+    void* p = nullptr;
+    hipError_t e;
+    {
+        KmHostLock lk(km_host_mutex());
+        e = hipMalloc(&p, bytes);
+    }
+    if (e != hipSuccess) return km_fail(ctx, KM_ENOMEM, "network hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
+    N->wpart = static_cast<float*>(p);
     return KM_OK;
 }
 
@@ -1330,6 +1345,7 @@ void km_net_free(km_ctx* ctx) {
     if (!ctx || !ctx->net) return;
     KmHostLock lk(km_host_mutex());
     if (ctx->net->arena) (void)hipFree(ctx->net->arena);
+    if (ctx->net->wpart) (void)hipFree(ctx->net->wpart);
     delete ctx->net;
     ctx->net = nullptr;
 }
@@ -1367,6 +1383,7 @@ int km_unet_loss_grad(km_ctx* ctx, const float* params, int B, int NX, int NY, c
     KM_REQUIRE(ctx, params && coef && r && grad, "null pointer");
     if (int rc = kmnet::prepare(ctx, B, NX, NY, params)) return rc;
     km_net* N = ctx->net;
+    if (int rc = alloc_wpart(ctx, N)) return rc;
     const int64_t n = (int64_t)NX * NY;
     const int H = N->H, W = N->W, Gs = N->Gs;
     hipStream_t s = ctx->stream;
