@@ -1086,6 +1086,9 @@ int alloc(km_ctx* ctx, km_net* N, int B, int NX, int NY) {
     KM_REQUIRE(ctx, NX >= 4 && NY >= 4, "system %d x %d too small for the network", NX, NY);
     if (N->arena && NX == N->NX && NY == N->NY && B < N->B) B = N->B;
     const int H = (NX - 2 + 7) / 8 * 8, W = (NY - 2 + 7) / 8 * 8;
+    // k_wgrad counts pixels, up to a row and a chunk past the last, in 32 bits
+    // (2^31 of them would take 800 GB of activations)
+    KM_REQUIRE(ctx, ((int64_t)B * H + 1) * W + 2 * kWgPx <= INT32_MAX, "%d images of %d x %d pixels: too many", B, H, W);
     const int64_t hw0 = (int64_t)H * W, hw1 = hw0 / 4, hw2 = hw0 / 16, hw3 = hw0 / 64;
     const int64_t n = (int64_t)NX * NY;
     const size_t bb = sizeof(bf16), fb = sizeof(float);

@@ -58,3 +58,15 @@ def test_inference_holds_no_training_memory(dev):
     finally:
         for ctx in ctxs:
             ctx.close()
+
+
+def test_more_pixels_than_the_kernels_count_are_refused(dev):
+    """64 images of 8192 x 8192 pixels are 2^32: refused by the size, before
+    anything is allocated or read."""
+    params = torch.tensor(unet.init_params(3), device=dev)
+    ctx = _lib.Context(torch.cuda.current_device(), torch.cuda.current_stream(dev).cuda_stream)
+    try:
+        with pytest.raises(_lib.KarmanError, match="too many"):
+            ctx.call("km_unet_loss_grad", ptr(params), 64, 8194, 8194, ptr(params), ptr(params), None, ptr(params), None)
+    finally:
+        ctx.close()
