@@ -13,6 +13,7 @@
 // concatenation); 2x2 average pools are small bandwidth-bound kernels.
 #include "km_unet.h"
 
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 
@@ -490,6 +491,7 @@ k_wgrad(int H, int W, int B, const bf16* __restrict__ src0, const bf16* __restri
         __syncthreads();
 #pragma unroll
         for (int ch = 0; ch < PX / 32; ++ch) {
+            if (base + ch * 32 >= hi) break;    // a share may be half a chunk longer than whole ones
             const int p0 = ch * 32 + g * 8;     // this lane's first pixel of the chunk
             // bit e of the bytes: pixel e has a neighbour above, below, left, right
             unsigned has;
@@ -1035,14 +1037,21 @@ void wgrad(km_net* N, int l, int H, int W, int B, const bf16* s0, const bf16* s1
     constexpr int most_ct = 32 / (COUT / 16), CT = (NCT + 3) / 4 < most_ct ? (NCT + 3) / 4 : most_ct;
     const int ncg = (NCT + 4 * CT - 1) / (4 * CT);
     const int64_t npx = (int64_t)B * H * W;
-    // The longest FP32 sums: those of 4096 workgroups, or of half the buffer.
-    int64_t nsplit = (4096 + ncg - 1) / ncg;
+    // The longest FP32 sum of a weight (the parts' sums are FP64): the shorter of
+    // 1 / (4 quarters) of the pixels, which is the shorter one at the coarse
+    // encoder levels and in small passes (e2 and e3 at 4 x 1280 x 256 pixels 96
+    // against 128, most layers at 4 x 320 x 64 32 against 64), and 1 / most of
+    // them, the shorter one for the decoder (d0 576 against 1280).  Errors
+    // against 64-bit sums over the same activations, e2 of 4 x 1280 x 256, 4 x 320
+    // x 64 and 1 x 96 x 20: 2.58, 2.53 and 2.78e-8 of the gradient's norm, by the
+    // second alone 2.70, 2.69 and 3.01e-8 (rounding exact sums to FP32 leaves
+    // 2.2e-8).  The first costs 22 us of 1250 at 4 x 1280 x 256: more parts.
     const int64_t cap = kWpartMax / (COUT * KP);
-    if (nsplit > cap / 2) nsplit = cap / 2;
-    const int64_t most = (npx + kWgPx - 1) / kWgPx;
-    if (nsplit > most) nsplit = most;
-    int64_t pps = (npx + nsplit - 1) / nsplit;
-    pps = (pps + kWgPx - 1) / kWgPx * kWgPx;
+    constexpr int groups = COUT >= 128 ? (NCT + 3) / 4 : (NCT + 7) / 8;
+    const int64_t quarters = std::min<int64_t>((1024 + groups - 1) / groups, cap / 8);
+    const int64_t most = std::min<int64_t>((4096 + ncg - 1) / ncg, cap / 2);
+    const int64_t longest = std::min(((npx + quarters - 1) / quarters + 127) / 128 * 32,
+                                     ((npx + most - 1) / most + kWgPx - 1) / kWgPx * kWgPx);
     // From there down, the pixels per workgroup whose rounds of resident
     // workgroups take the fewest pixel steps (plus one chunk's for the partial
     // sums of each round): with 576 the two wide decoder layers at
@@ -1055,8 +1064,8 @@ void wgrad(km_net* N, int l, int H, int W, int B, const bf16* s0, const bf16* s1
         return e == hipSuccess && n > 0 ? n : 2;
     }();
     const int64_t places = (int64_t)per_cu * N->cus;
-    int64_t least = INT64_MAX;
-    for (int64_t k = pps; k >= kWgPx; k -= kWgPx) {
+    int64_t least = INT64_MAX, pps = longest;
+    for (int64_t k = longest; k >= 32; k -= k % kWgPx ? 32 : kWgPx) {
         const int64_t parts = (npx + k - 1) / k;
         if (parts > cap) break;
         const int64_t steps = (parts * ncg + places - 1) / places * (k + kWgPx);
@@ -1065,7 +1074,7 @@ void wgrad(km_net* N, int l, int H, int W, int B, const bf16* s0, const bf16* s1
             pps = k;
         }
     }
-    nsplit = (npx + pps - 1) / pps;
+    const int64_t nsplit = (npx + pps - 1) / pps;
     hipLaunchKernelGGL((k_wgrad<MODE, C0, C1, COUT, CT>), dim3((unsigned)nsplit, (unsigned)ncg), dim3(KM_BLOCK), 0, st,
                        H, W, B, s0, s1, dY, (int)pps, N->wpart);
     const LayerOff& L = N->lay.L[l];

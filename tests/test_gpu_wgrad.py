@@ -34,3 +34,29 @@ def test_gradients_at_chunk_edges(nx, ny, B, dev):
         err = np.linalg.norm(a - b) / np.linalg.norm(b)
         print(f"{nx}x{ny} x {B} {name}: {err:.1e}")
         assert err < 3e-2, name
+
+
+@pytest.mark.parametrize("nx,ny", [(1280, 192), (328, 72), (96, 24)])
+def test_gradients_of_copies_equal_those_of_one(nx, ny, dev):
+    """Four copies of a system have the gradient of one (the loss is a mean, its
+    factor 1/4 exact) with the pixels shared out differently among the
+    workgroups: 32 to 576 each, and at 1280 x 192 shares of 96 pixels, a chunk
+    and a half.  An FP32 sum of 576 terms is off by at most 576 x 2^-24 = 3.4e-5
+    of the sum of their magnitudes; the bound on the difference, 1e-4 of the
+    layer's largest weight gradient, is that with room for terms that cancel
+    threefold."""
+    coef, r = small_system(7, nx=nx, ny=ny)
+    params = unet.init_params(11)
+    net = learned.UNetPreconditioner(params=params, device=dev)
+    grads = []
+    for B in (1, 4):
+        c = torch.tensor(np.stack([coef] * B).astype(np.float32), device=dev)
+        rt = torch.tensor(np.stack([r] * B).astype(np.float32), device=dev)
+        _, g = net.loss_grad(c, rt)
+        grads.append(g.cpu().numpy().astype(np.float64).copy())
+    for name, (o, shape) in unet.param_slices()[0].items():
+        m = int(np.prod(shape))
+        a, b = grads[0][o:o + m], grads[1][o:o + m]
+        err = np.abs(a - b).max() / np.abs(a).max()
+        print(f"{nx}x{ny} {name}: {err:.1e}")
+        assert err < 1e-4, name
