@@ -1359,13 +1359,20 @@ int finish(km_ctx* ctx, Family fam, int nsys, const int* NX, const int* NY, cons
 
 namespace kmpersist {
 
-// Longer systems stay by launches.  A p' solve takes 31 iterations at 1280 x 256,
-// 39 at 1500 x 300 and 50 to 62 at 1999 x 401; from about 40 on BiCGSTAB amplifies
-// the rounding of another summation order, in p' itself or in the momentum
-// solves before it, to the size of the tolerance, and the step's result, though
-// as accurate, is another one (eps = 1e-8: p' changes by 1e-12, 4e-10 and 1e-9 of
-// its norm at those sizes).  The gain would be 1.4x at 1500 x 300 (p' 50 us per
-// iteration against 72), 1.2x at 1999 x 401, and 2.5x for the momentum solves.
+// Preconditioned systems with a longer side stay with the launches, so that
+// their results stay what they were: the kernel itself takes any system whose
+// tiles fit, and is faster there too.  The two paths add their sums in another
+// order, a solve may stop an iteration earlier or later, and a step's fields
+// differ by about the tolerance, at every size.  Measured over three outer steps
+// at eps 1e-8: v by 1.0e-8 of its norm at 1280 x 256, 1.3e-8 at 1400 x 280, 8e-9
+// at 640 x 640, 8e-10 at 1999 x 401 (at eps 1e-10 by 1.6e-10); p' by 1e-12 to 1e-10
+// where it takes up to 60 iterations, by up to 1.6e-9 where it takes 134 (900 x
+// 900).  That is taken below the line, where a step of a 5 : 1 channel is twice
+// as fast (2.0x at 1024 x 205, 2.1x at 1280 x 256), and not above it, where the
+// gain falls (1.6x at 1400 x 280, 1.5x at 1500 x 300, 1.4x at 1999 x 401: tiles of
+// more than 48 x 32 cells).  The line looks at the longer side only: 1400 x 60
+// (1.9x) lies outside it, 900 x 900 (1.2x) inside.  Plain solves, two to four
+// times as fast at any size, have no such line.
 constexpr int kMaxSide = 1300;
 
 // Two launches that waited out their limit, of any entry: something holds the
