@@ -9,9 +9,15 @@ corrections and the continuity residual.  Every ``n_outer`` steps the time
 level advances (u0 <- u), as in a time-accurate run.
 
 Prints ONE JSON line (rank 0).  Extra keys:
-  roofline      achieved HBM GB/s of the dominant solver kernel vs 8 TB/s,
-                algorithmic bytes / kernel time from HIP events on the
-                solver's stream; traffic from rocprofv3 counters (profiles/)
+  one_launch    solves per step that ran in one launch, from the context's
+                counts over the timed steps
+  roofline      what bounds the timed step's p' solve.  By launches: achieved
+                HBM GB/s of the dominant solver kernel vs 8 TB/s, algorithmic
+                bytes / kernel time from HIP events on the solver's stream;
+                traffic from rocprofv3 counters (profiles/).  In one launch:
+                the solve's compulsory bytes over its time, which the exchange
+                between workgroups bounds; the kernels of the launches, which
+                the timed step then does not run, stand under launch_path
   cpu_baseline  the C/OpenMP FP64 restatement with the reference's kernel
                 decomposition (oracle/cpu_simple.c) on this host's cores,
                 timed on a bounded sample of the same workload
@@ -44,6 +50,10 @@ BYTES_PER_CELL = {"bicg_p": 11 * 8, "bicg_s": 9 * 8, "bicg_r": 7 * 8,
                   # the same for a symmetric p' system (KM_FLAG_SYMMETRIC, as the
                   # step's p' solve runs them): aP, aE, aN planes only
                   "tl_pv+sym": 7 * 8 + 1, "tl_st+sym": 9 * 8 + 1}
+# a p' solve in one launch reads five coefficient planes, b and the mask once and writes x once
+SOLVE_BYTES_PER_CELL = 7 * 8 + 1
+# preconditioned systems with a longer side solve by launches (kMaxSide, csrc/km_persist.hip)
+ONE_LAUNCH_SIDE = 1300
 # the coarse rows of tl_cv / tl_ct read A_c^-1 (m x m) and a few m-vectors
 COARSE_VECTORS = {"tl_cv": 4, "tl_ct": 6}
 
@@ -190,9 +200,11 @@ def main():
         t0 = time.perf_counter()
         iu, iv = s.solve_momentum_eqn(1)
         s.correct_conserv()
+        n0 = s.ctx.one_launch_counts()[0]
         t1 = time.perf_counter()
         ip = s.solve_pcorrection_eqn()      # synchronous: returns after the solve
         t2 = time.perf_counter()
+        p_one = s.ctx.one_launch_counts()[0] > n0
         s._correct()
         s.compute_mdiv()
         step_count[0] += 1
@@ -200,7 +212,8 @@ def main():
             s.time_forward()
         if rec is not None:
             rec.append({"mom_ms": (t1 - t0) * 1e3, "p_ms": (t2 - t1) * 1e3, "p_it": ip.iterations,
-                        "u_it": iu.iterations, "v_it": iv.iterations, "p_true": ip.rel_resid_true, "p_status": ip.status})
+                        "u_it": iu.iterations, "v_it": iv.iterations, "p_true": ip.rel_resid_true, "p_status": ip.status,
+                        "p_one": p_one})
 
     log(f"bench: case {case.name} mode {args.mode}, spin-up {args.spinup_time_steps} time steps, "
         f"warmup {args.warmup}, steps {args.steps}")
@@ -220,11 +233,13 @@ def main():
         s.ctx.call("km_set_coarse_chunks", *[int(v) for v in args.chunks.split(",")])
     torch.cuda.synchronize()
     rec = []
+    one0 = s.ctx.one_launch_counts()
     t0 = time.perf_counter()
     for k in range(args.steps):
         one_step(rec)
     torch.cuda.synchronize()
     wall = time.perf_counter() - t0
+    one = [b - a for a, b in zip(one0, s.ctx.one_launch_counts())]
     ms_per_step = wall * 1e3 / args.steps
     steps_per_s = args.steps / wall
     p_it = [r["p_it"] for r in rec]
@@ -298,6 +313,29 @@ def main():
     except (OSError, ValueError):
         pass
     log(f"bench: kernel us {kern} (dispatch events {kern_ev}), dominant {dom}: {achieved:.0f} GB/s")
+    # by launches: these kernels are the timed step's; in one launch (as the
+    # stage-by-stage steps' counts say) they are only those of larger systems
+    launch_path = {"smoothing_tile": tile,
+                   "kernel_us_back_to_back": {k: round(v, 3) for k, v in kern.items()},
+                   "kernel_us_dispatch_events": {k: round(v, 3) for k, v in kern_ev.items()},
+                   "roofline": {"bound": "hbm", "kernel": dom, "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
+                                "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
+                                "alg_bytes_per_launch": launch_bytes,
+                                **({"coefficient_planes": 3 if symk else 5} if twolevel and not learned else {}),
+                                "note": mall_note(cells_p, coarse["unknowns"] if coarse else 0)}}
+    p_one = one[0] > 0 and bool(srec) and all(r["p_one"] for r in srec)
+    if p_one:
+        solve_us = statistics.median(p_ms) * 1e3
+        got = SOLVE_BYTES_PER_CELL * cells_p / solve_us / 1e3
+        path = {"roofline": {"bound": "latency", "kernel": "k_solve" if twolevel and not learned else "k_plain",
+                             "achieved": round(got, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                             "frac": round(got / HBM_PEAK_GBS, 4), "alg_bytes_per_launch": SOLVE_BYTES_PER_CELL * cells_p,
+                             "us_per_iteration": round(sum(p_ms) / sum(p_ms_it) * 1e3, 3),
+                             "note": "a whole solve per launch, its vectors on chip: rounds of exchange between the "
+                                     "workgroups and the loads after them bound it, not memory"},
+                "launch_path": launch_path}
+    else:
+        path = {k: v for k, v in launch_path.items() if k != "smoothing_tile"}
 
     if args.calib_copy_mb:
         # a plain copy of known size: its FETCH_SIZE / WRITE_SIZE readings
@@ -335,7 +373,7 @@ def main():
                                f"{case.obstacle_cells}x{case.obstacle_cells} cylinder, "
                                f"{n_outer} outer steps per time step, inner eps 1e-8",
                    "mode": args.mode, "p_solver": p_solver, "p_twolevel": twolevel, "p_network": learned,
-                   "p_vectors": "f32" if fp32 else "f64", "smoothing_tile": tile, "coarse": coarse,
+                   "p_vectors": "f32" if fp32 else "f64", "smoothing_tile": None if p_one else tile, "coarse": coarse,
                    "momentum": "fbicgstab+rbgs" if momentum == "rbgs" else "bicgstab",
                    "step": "km_simple_step" if native else "stage by stage"},
         "p_solve_ms_median": round(statistics.median(p_ms), 3) if p_ms else None,
@@ -352,13 +390,9 @@ def main():
         "learned_compare": lcompare,
         "p_cells_iters_per_s": round(cells_p * total_p_it / total_p_s, 1) if p_ms else None,
         "us_per_p_iter": round(total_p_s / total_p_it * 1e6, 3) if p_ms else None,
-        "kernel_us_back_to_back": {k: round(v, 3) for k, v in kern.items()},
-        "kernel_us_dispatch_events": {k: round(v, 3) for k, v in kern_ev.items()},
-        "roofline": {"bound": "hbm", "kernel": dom, "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
-                     "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
-                     "alg_bytes_per_launch": launch_bytes,
-                     **({"coefficient_planes": 3 if symk else 5} if twolevel and not learned else {}),
-                     "note": mall_note(cells_p, coarse["unknowns"] if coarse else 0)},
+        "one_launch": {"solves_per_step": round(one[0] / args.steps, 2), "refused": one[1], "gave_up": one[2],
+                       "p_solve": p_one},
+        **path,
         "cpu_baseline": cpu,
     }
     print(json.dumps(out), flush=True)
@@ -481,15 +515,18 @@ def bench_batch(args):
     for _ in range(args.warmup):
         batch_step()
     torch.cuda.synchronize()
+    ctxs = [c for _, c in b._workers] if workers else [b.ctx]
+    one0 = sum(c.one_launch_counts()[0] for c in ctxs)
     t0 = time.perf_counter()
     recs = [batch_step() for _ in range(args.steps)]
     torch.cuda.synchronize()
     wall = time.perf_counter() - t0
+    one = sum(c.one_launch_counts()[0] for c in ctxs) - one0
     p_it = [inf[2].iterations for rec in recs for inf in rec]
     n_fp32 = sum(bool(c.mixed) for c in case_list) if workers else 0
     cell_its = sum(c.shape_p[0] * c.shape_p[1] * inf[2].iterations for rec in recs for c, inf in zip(case_list, rec))
-    # algorithmic bytes of the p' iterations alone (the two-level path's
-    # K_PV, K_CV, K_ST, K_CT: per cell 57 + 73 + 80 B with FP64 vectors, 41 +
+    # algorithmic bytes of the p' iterations by launches alone (of the cases
+    # too long for one launch: K_PV, K_CV, K_ST, K_CT: per cell 57 + 73 + 80 B with FP64 vectors, 41 +
     # 49 + 40 B with FP32 vectors and FP64 coefficient planes, plus two reads
     # of the m x m FP64 coarse inverse and the coarse vectors); the momentum
     # solves, stages and refinement residuals are not counted
@@ -497,6 +534,8 @@ def bench_batch(args):
     if coarse:
         for rec in recs:
             for c, inf in zip(case_list, rec):
+                if max(c.nx, c.ny) <= ONE_LAUNCH_SIDE:
+                    continue
                 m = coarse_unknowns(c.nx, c.ny)
                 per_cell = (41 + 49 + 40) if (workers and c.mixed) else (57 + 73 + 80)
                 cells = c.shape_p[0] * c.shape_p[1]
@@ -516,6 +555,8 @@ def bench_batch(args):
                       "fp32_vector_cases": n_fp32},
            "p_iters_min_median_max": [min(p_it), sorted(p_it)[len(p_it) // 2], max(p_it)],
            "p_cells_iters_per_s": round(cell_its / wall, 1),
+           "one_launch_solves_per_step": round(one / args.steps, 1),
+           "cases_by_launches": sum(max(c.nx, c.ny) > ONE_LAUNCH_SIDE for c in case_list) if coarse else b.n,
            "p_iter_bytes_per_s": round(p_bytes / wall, 1) if coarse else None,
            "p_iter_hbm_fraction": round(p_bytes / wall / (HBM_PEAK_GBS * 1e9), 4) if coarse else None,
            "case_steps_per_s": round(args.steps * b.n / wall, 3)}

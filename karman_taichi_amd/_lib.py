@@ -183,6 +183,12 @@ class Context:
     def synchronize(self):
         self.call("km_synchronize")
 
+    def one_launch_counts(self):
+        """(run, refused, gave up): the context's one-launch solves so far."""
+        n = [ctypes.c_int64() for _ in range(3)]
+        self.call("km_one_launch_counts", *[ctypes.byref(v) for v in n])
+        return tuple(v.value for v in n)
+
     def close(self):
         if getattr(self, "h", None):
             self._lib.km_destroy(self.h)

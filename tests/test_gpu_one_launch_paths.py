@@ -36,9 +36,7 @@ class Solver:
         self.ctx.close()
 
     def counts(self):
-        n = [ctypes.c_int64() for _ in range(3)]
-        self.ctx.call("km_one_launch_counts", *[ctypes.byref(v) for v in n])
-        return tuple(v.value for v in n)
+        return self.ctx.one_launch_counts()
 
     def solve(self, entry, coef, b):
         NX, NY = b.shape
