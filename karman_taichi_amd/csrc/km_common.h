@@ -93,6 +93,23 @@ static inline bool tile_ok(int TI, int TJ) {
     return (TI + 2) * (TJ + 2) <= (cpt + 2) * KM_BLOCK;
 }
 
+// The tile of a system whose tiles have not been timed: each row in the fewest
+// near-equal segments of at most 256 columns, and rows stacked until a tile
+// covers about 256 cells, as far as that is valid.  Where no number of rows is
+// (segments of 255 and 256 columns have no room for their halo), one segment
+// more.
+static inline void default_tile(int NX, int NY, int* TI, int* TJ) {
+    for (int segs = (NY + 255) / 256;; ++segs) {
+        const int tj = (NY + segs - 1) / segs;
+        int ti = (256 + tj - 1) / tj;
+        if (ti > NX) ti = NX;
+        while (ti > 1 && !tile_ok(ti, tj)) --ti;
+        *TI = ti;
+        *TJ = tj;
+        if (tile_ok(ti, tj)) return;
+    }
+}
+
 // A flat (pointwise) launch over n elements: G workgroups, each owning a
 // contiguous chunk (a multiple of the workgroup size) of the index range.
 struct Flat {

@@ -1173,22 +1173,15 @@ int km_set_plain_totals(km_ctx* ctx, int mode) {
     return KM_OK;
 }
 
-// Tile choice: an explicit override, else the cached choice, else a default
-// that splits each row into near-equal segments of at most 256 columns and
-// stacks rows until a tile covers about 256 cells.
+// Tile choice: an explicit override, else the cached choice, else the default.
 int km_choose_tile(km_ctx* ctx, int NX, int NY, int prec, int* TI, int* TJ) {
     auto key = std::make_tuple(NX, NY, prec);
     auto ov = ctx->tile_override.find(key);
     if (ov != ctx->tile_override.end()) { *TI = ov->second.first; *TJ = ov->second.second; return KM_OK; }
     auto it = ctx->tiles.find(key);
     if (it != ctx->tiles.end()) { *TI = it->second.first; *TJ = it->second.second; return KM_OK; }
-    const int segs = (NY + 255) / 256;
-    int tj = (NY + segs - 1) / segs;
-    int ti = (256 + tj - 1) / tj;
-    if (ti > NX) ti = NX;
-    ctx->tiles[key] = {ti, tj};
-    *TI = ti;
-    *TJ = tj;
+    default_tile(NX, NY, TI, TJ);
+    ctx->tiles[key] = {*TI, *TJ};
     return KM_OK;
 }
 
@@ -1483,7 +1476,7 @@ int64_t scratch_max_cells() { return (int64_t)((KM_NOALLOC_SCRATCH_BYTES - kScra
 
 // The tile of an n-cell system without timing candidates or caching a choice
 // (the autotuner's timing needs workspace): an override, else the cached
-// choice, else the default split of km_choose_tile.
+// choice, else the default.
 int peek_tile(km_ctx* ctx, int NX, int NY, Tile* out) {
     auto key = std::make_tuple(NX, NY, (int)KM_F64);
     int TI, TJ;
@@ -1496,10 +1489,7 @@ int peek_tile(km_ctx* ctx, int NX, int NY, Tile* out) {
         TI = it->second.first;
         TJ = it->second.second;
     } else {
-        const int segs = (NY + 255) / 256;
-        TJ = (NY + segs - 1) / segs;
-        TI = (256 + TJ - 1) / TJ;
-        if (TI > NX) TI = NX;
+        default_tile(NX, NY, &TI, &TJ);
     }
     KM_REQUIRE(ctx, tile_ok(TI, TJ), "tile %dx%d is not valid for the iteration kernels", TI, TJ);
     *out = make_tile(NX, NY, TI, TJ);
