@@ -1368,7 +1368,7 @@ struct PlainMem {
 // tune (may be null) times the tiles before the first solve by launches.
 int bicgstab_plain(km_ctx* ctx, const PlainMem& m, Tile tl, const double* coef, const double* b, double* x,
                    double eps, int max_iter, int flags, bool use_graph, km_solve_info* info,
-                   const std::function<int(Tile*)>& tune = nullptr) {
+                   const std::function<int(Tile*, bool)>& tune = nullptr) {
     const int64_t n = (int64_t)tl.NX * tl.NY;
     const bool from_r = (flags & KM_FLAG_X0) != 0;
     const bool check_true = (flags & KM_FLAG_TRUE) != 0;
@@ -1380,26 +1380,28 @@ int bicgstab_plain(km_ctx* ctx, const PlainMem& m, Tile tl, const double* coef, 
         if (int rc = residual_norm2(ctx, tl, coef, b, x, m.ws /* r */, false, nullptr, m.P, m.dres)) return rc;
     }
     // One solve, in one launch where the system fits (r, for a start from x, in
-    // m.ws), else, or if that launch gives up, by launches on tuned tiles
+    // m.ws), else, or if that launch gives up, by launches on tuned tiles.
     // The one-launch solve is followed by the true residual (its square in the
-    // first of the host's result words) before the host waits: tailed.
+    // first of the host's result words) before the host waits: tailed.  Where the
+    // true residual is checked after each solve it is formed there.
     bool tailed = false;
+    const bool want_tail = info && !check_true;
     const std::function<int()> tail = [&]() { return residual_mapped(ctx, tl, coef, b, x, m.P); };
     auto solve = [&](bool from_x, int cap, double ref, double tol, KState* out) -> int {
         int shape = 0;
         if (kmpersist::fits_plain(ctx, tl.NX, tl.NY, &shape)) {
             bool ran = false;
             if (int rc = kmpersist::plain(ctx, shape, false, tl.NX, tl.NY, coef, from_x ? m.ws : b, x, from_x, m.ws + n,
-                                          m.words, tol, cap, ref, out, info ? &tail : nullptr, &ran))
+                                          m.words, tol, cap, ref, out, want_tail ? &tail : nullptr, &ran))
                 return rc;
-            tailed = ran && info;
+            tailed = ran && want_tail;
             if (ran) return KM_OK;
             // x may have been written in part: r again
             if (from_x)
                 if (int rc = residual_norm2(ctx, tl, coef, b, x, m.ws, false, nullptr, m.P, m.dres)) return rc;
         }
         if (tune)
-            if (int rc = tune(&tl)) return rc;
+            if (int rc = tune(&tl, from_x)) return rc;
         return bicgstab_typed<double>(ctx, tl, coef, b, x, m.ws, from_x, tol, cap, use_graph, m.st, out, ref, m.P);
     };
     KState s;
@@ -1438,7 +1440,7 @@ int bicgstab_plain(km_ctx* ctx, const PlainMem& m, Tile tl, const double* coef, 
             double rr = 0.0;
             if (tailed) {
                 rr = km_mapped_res(ctx, 0);
-                if (!from_r && !check_true) bb = s.r0;   // <b,b>, the solve's first <r,r>
+                if (!from_r) bb = s.r0;   // <b,b>, the solve's first <r,r>
             } else {
                 if (!from_r && !check_true)
                     if (int rc = dot_sync(ctx, n, KM_F64, b, b, &bb, m.P, m.dres)) return rc;
@@ -1526,16 +1528,12 @@ int km_bicgstab(km_ctx* ctx, int NX, int NY, const double* coef, const double* b
     Tile tl;
     if (int rc = get_tile(ctx, NX, NY, KM_F64, &tl)) return rc;
     const PlainMem m{&ctx->st[0], ctx->partials, ctx->dres, ws, nullptr};
-    // timing the tiles overwrites the workspace: r, which a start from x has
-    // put there, is formed again
-    const bool from_x = (flags & KM_FLAG_X0) != 0;
-    auto tune = [&](Tile* t) -> int {
-        if (ctx->tuned.count(std::make_tuple(NX, NY, (int)KM_F64))) return get_tile(ctx, NX, NY, KM_F64, t);
+    auto tune = [&](Tile* t, bool from_x) -> int {
+        const size_t timed = ctx->tuned.size();
         if (int rc = ensure_tuned<double>(ctx, NX, NY, KM_F64, coef, b, ws)) return rc;
         if (int rc = get_tile(ctx, NX, NY, KM_F64, t)) return rc;
-        return from_x || (flags & KM_FLAG_TRUE)
-                   ? residual_norm2(ctx, *t, coef, b, x, ws, false, nullptr)
-                   : (int)KM_OK;
+        // timing overwrites the workspace: r, which a start from x has put there, is formed again
+        return from_x && ctx->tuned.size() != timed ? residual_norm2(ctx, *t, coef, b, x, ws, false, nullptr) : (int)KM_OK;
     };
     return bicgstab_plain(ctx, m, tl, coef, b, x, eps, max_iter, flags, !(flags & KM_FLAG_NO_GRAPH), info, tune);
 }
