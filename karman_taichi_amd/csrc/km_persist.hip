@@ -296,8 +296,10 @@ __device__ __forceinline__ void solve_body(const PSys<T>& s, int L) {
     const int ti0 = 1 + ta * TI, tj0 = 1 + tb * TJ;
     unsigned round = s.round;
     // raised before this launch (by the one before it, say): leave at the first
-    // round instead of waiting too
-    if (t == 0) bad = (int)get(s.abort);
+    // round instead of waiting too.  In flight while the frame is loaded (waited
+    // for here it was 1 us per solve).
+    unsigned raised = 0;
+    if (t == 0) raised = get(s.abort);
 
     // boundary cells of the system next to this tile: x = 0, and their rows
     // must be empty (checked: otherwise the launch gives up)
@@ -648,6 +650,7 @@ __device__ __forceinline__ void solve_body(const PSys<T>& s, int L) {
 
     double rho = 0.0, alpha = 0.0, omega = 1.0, r0 = 0.0, best = 1e300;
     int it = 0, best_it = 0, status = -1;
+    if (t == 0) bad = (int)raised;
     __syncthreads();
     if (COARSE) {
         // Y(r) = Y(p) = A_c^-1 P^T rhs
@@ -926,8 +929,8 @@ __global__ void __launch_bounds__(NT) k_plain(PPlain s) {
     const int64_t n = (int64_t)NX * NY;
     const int ta = L / s.tiles_j, tb = L - ta * s.tiles_j;
     const int ti0 = 1 + ta * TI, tj0 = 1 + tb * TJ;
-    unsigned round = s.round;
-    if (t == 0) bad = (int)get(s.abort);
+    unsigned round = s.round, raised = 0;
+    if (t == 0) raised = get(s.abort);   // as in solve_body
     for (int k = t; k < (TI + 2) * W; k += NT) z[k] = 0.0;
     // boundary rows must be empty (see solve_body)
     const int j0 = tb == 0 ? 0 : tj0, j1 = tj0 + TJ > ny ? NY : tj0 + TJ;
@@ -1036,6 +1039,7 @@ __global__ void __launch_bounds__(NT) k_plain(PPlain s) {
     };
     int it = 0, status = -1;
     double r0 = 0.0, rho = 0.0, rho0 = 1.0, alpha = 0.0, omega = 0.0, rTr = 0.0;
+    if (t == 0) bad = (int)raised;   // before the sum's barrier
     // <r,r> (and <r,r~>, the same at the start); the count of odd boundary cells first
     bool ok = sum(odd, 0.0, s.part[1]);
     if (ok) total(s.part[1], nullptr, nullptr);
